@@ -41,7 +41,8 @@ extern "C" {
                               16: per-batch-row document metadata (layout m_sb),
                                   dropout with document masks;
                               17: rmx_linear_scan_status;
-                              18: right-bounded windows (problem window_right) */
+                              18: right-bounded windows (problem window_right), and since,
+                                  as additions: rmx_mamba2_dt_cumsum_state_bwd */
 
 /* error codes */
 #define RMX_OK 0
@@ -406,6 +407,20 @@ int32_t rmx_mamba2_dt_cumsum_bwd(const void* dt, int32_t dt_is_f32, const float*
                                  int32_t T, int32_t nheads, void* stream);
 
 /*
+ * The gradient of rmx_mamba2_dt_cumsum behind rmx_mamba2_chunk_state: as
+ * rmx_mamba2_dt_cumsum_bwd without a decay gradient, with g_cum_A and g_e as
+ * rmx_mamba2_chunk_state_bwd leaves them. g_cum_A[r, T-1, h] is not read: it stands for
+ * -sum_{t<T-1} g_cum_A[r, t, h] (every weight depends on cum_A at T-1), so the suffix sums
+ * are minus the prefix sums of the other entries and are taken that way (no cancellation
+ * for the early tokens, whose weights have decayed).
+ */
+int32_t rmx_mamba2_dt_cumsum_state_bwd(const void* dt, int32_t dt_is_f32, const float* dt_bias,
+                                       const float* A, int32_t dt_softplus, const float* g_cum_A,
+                                       const float* g_e, float* g_dt, float* g_A,
+                                       float* g_dt_bias, int32_t rows, int32_t T, int32_t nheads,
+                                       void* stream);
+
+/*
  * Mamba2 shard final state from x, B and dt: the final_states of mamba-ssm's
  * mamba_chunk_scan_combined(..., return_final_states=True) from a zero state,
  * which the reference's CP scan wrapper gathers across ranks (mamba.py:113-141,
@@ -429,8 +444,8 @@ int32_t rmx_mamba2_chunk_state(const uint16_t* x, const uint16_t* B, const float
  * Gradient of rmx_mamba2_chunk_state given g_state = dL/dstate (fp32, like
  * state): writes g_x (bf16, like x), g_B (bf16, like B), g_e and g_cum_A (fp32
  * [rows, T, H]). g_cum_A[r, T-1, h] is left as -g_w w of that token; the full
- * entry is sum_{t<T-1} g_w w = -sum_{t<T-1} g_cum_A[r, t, h], which the caller
- * writes (every weight depends on cum_A at T-1). workspace (nullable) of at least
+ * entry is sum_{t<T-1} g_w w = -sum_{t<T-1} g_cum_A[r, t, h] (every weight depends on
+ * cum_A at T-1), which rmx_mamba2_dt_cumsum_state_bwd takes it for. workspace (nullable) of at least
  * rmx_mamba2_chunk_state_bwd_workspace(...) bytes, 16-byte aligned: with it (and a
  * nonzero size: head_dim 64), g_state is first converted to bf16 there and the kernel moves two
  * heads per step, reading G by LDS DMA; without it the one-head form runs. Both give

@@ -114,6 +114,8 @@ SIGNATURES = {
                                     _vp]),
     "rmx_mamba2_dt_cumsum_bwd": (_i32, [_vp, _i32, _vp, _vp, _i32] + [_vp] * 7
                                  + [_i32, _i32, _i32, _vp]),
+    "rmx_mamba2_dt_cumsum_state_bwd": (_i32, [_vp, _i32, _vp, _vp, _i32] + [_vp] * 5
+                                       + [_i32, _i32, _i32, _vp]),
     "rmx_mamba2_chunk_state": (_i32, [_vp] * 6 + [_i32] * 6 + [_vp]),
     "rmx_mamba2_chunk_state_bwd_workspace": (ctypes.c_size_t, [_i32] * 4),
     "rmx_mamba2_chunk_state_bwd": (_i32, [_vp] * 10 + [_i32] * 6 + [_vp, ctypes.c_size_t, _vp]),

@@ -541,20 +541,42 @@ int32_t rmx_mamba2_dt_cumsum(const void* dt, int32_t dt_is_f32, const float* dt_
                     "rmx_mamba2_dt_cumsum launch");
 }
 
-int32_t rmx_mamba2_dt_cumsum_bwd(const void* dt, int32_t dt_is_f32, const float* dt_bias,
-                                 const float* A, int32_t dt_softplus, const float* g_cum_A,
-                                 const float* g_e, const float* g_decay, const float* decay,
-                                 float* g_dt, float* g_A, float* g_dt_bias, int32_t rows,
-                                 int32_t T, int32_t nheads, void* stream) {
+static int dt_cumsum_bwd(const void* dt, int32_t dt_is_f32, const float* dt_bias, const float* A,
+                         int32_t dt_softplus, const float* g_cum_A, const float* g_e,
+                         const float* g_decay, const float* decay, float* g_dt, float* g_A,
+                         float* g_dt_bias, int32_t rows, int32_t T, int32_t nheads, int closed,
+                         void* stream, const char* what) {
   int rc = check_dt(dt, dt_is_f32, A, dt_softplus, rows, T, nheads);
   if (rc) return rc;
   if ((int64_t)rows * T * nheads == 0) return RMX_OK;
   if (!g_dt || !g_A || (g_decay && !decay)) return fail(RMX_EINVAL, "NULL tensor pointer");
   return dev_status(rmx::launch_mamba2_dt_cumsum_bwd(dt, dt_is_f32, dt_bias, A, dt_softplus,
                                                      g_cum_A, g_e, g_decay, decay, g_dt, g_A,
-                                                     g_dt_bias, rows, T, nheads,
+                                                     g_dt_bias, rows, T, nheads, closed,
                                                      (hipStream_t)stream),
-                    "rmx_mamba2_dt_cumsum_bwd launch");
+                    what);
+}
+
+int32_t rmx_mamba2_dt_cumsum_bwd(const void* dt, int32_t dt_is_f32, const float* dt_bias,
+                                 const float* A, int32_t dt_softplus, const float* g_cum_A,
+                                 const float* g_e, const float* g_decay, const float* decay,
+                                 float* g_dt, float* g_A, float* g_dt_bias, int32_t rows,
+                                 int32_t T, int32_t nheads, void* stream) {
+  return dt_cumsum_bwd(dt, dt_is_f32, dt_bias, A, dt_softplus, g_cum_A, g_e, g_decay, decay, g_dt,
+                       g_A, g_dt_bias, rows, T, nheads, 0, stream,
+                       "rmx_mamba2_dt_cumsum_bwd launch");
+}
+
+int32_t rmx_mamba2_dt_cumsum_state_bwd(const void* dt, int32_t dt_is_f32, const float* dt_bias,
+                                       const float* A, int32_t dt_softplus, const float* g_cum_A,
+                                       const float* g_e, float* g_dt, float* g_A,
+                                       float* g_dt_bias, int32_t rows, int32_t T, int32_t nheads,
+                                       void* stream) {
+  if ((int64_t)rows * T * nheads > 0 && (!g_cum_A || !g_e))
+    return fail(RMX_EINVAL, "NULL tensor pointer");
+  return dt_cumsum_bwd(dt, dt_is_f32, dt_bias, A, dt_softplus, g_cum_A, g_e, nullptr, nullptr, g_dt,
+                       g_A, g_dt_bias, rows, T, nheads, 1, stream,
+                       "rmx_mamba2_dt_cumsum_state_bwd launch");
 }
 
 static int check_state(const uint16_t* x, const uint16_t* B, const float* e, const float* cum_A,

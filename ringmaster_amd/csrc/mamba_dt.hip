@@ -3,10 +3,23 @@
 //   e_t = softplus(dt_t + dt_bias) when dt_softplus, else dt_t
 //   cum_A_t = sum_{s<=t} A e_s,   decay = exp(cum_A_{T-1})
 // and the gradient of that map. softplus follows torch (beta 1, threshold 20:
-// x > 20 -> x). A workgroup = 4 waves over one row and 64 consecutive heads
-// (lane = head, so each step of a wave reads 64 consecutive dt values); the
-// waves take consecutive quarters of the tokens and exchange their quarter sums
-// through LDS between a summing pass and a writing pass.
+// x > 20 -> x).
+//
+// Both directions are a prefix (suffix) sum along T. The rows of a call are few (8 for 8
+// ranks), so a workgroup per row leaves the chip idle: walking T = 8192 tokens of 64 heads
+// that way took 1958 us forward and 1806 us backward, the softplus on 8 of 256 CUs. The
+// tokens are cut into chunks, one workgroup each: 512 threads, HT = 8..64 heads (the least
+// that covers H) by 512 / HT runs of 16 tokens, a thread holding its run in registers (16
+// loads in flight, softplus computed once). The chunks meet through the output itself, so no
+// workspace is needed and no workgroup waits for another:
+//   forward: chunk scans (each from zero) / the scan of the chunks' last tokens, in place /
+//     every other token plus the last token of the chunk before;
+//   backward: chunk sums of g_cum into g_dt at each chunk's first token / those turned into
+//     what enters each chunk / the chunks, each reading its own first token before the
+//     barrier that precedes its stores.
+// A sequence of one chunk is one launch. At 8 rows x 8192 x 64 the three launches take 28 + 5 + 9
+// us forward and 5 + 5 + 35 us backward; the first and the last of these are bound by the VALU
+// work of softplus (25 MB and 42 MB moved).
 #include "rmx_kernels.h"
 
 namespace rmx {
@@ -27,6 +40,7 @@ struct DtArgs {
   float* g_A;            // bwd += [H]
   float* g_bias;         // bwd += [H] (softplus only) or null
   int rows, T, H;
+  int nchunk;
 };
 
 __device__ __forceinline__ float dt_at(const DtArgs& a, int64_t i) {
@@ -34,133 +48,291 @@ __device__ __forceinline__ float dt_at(const DtArgs& a, int64_t i) {
                   : bf2f(reinterpret_cast<const uint16_t*>(a.dt)[i]);
 }
 __device__ __forceinline__ float softplus_t(float x) { return x > 20.f ? x : log1pf(expf(x)); }
-__device__ __forceinline__ float softplus_grad(float x) {  // d softplus / dx
-  if (x > 20.f) return 1.f;
-  const float z = expf(x);
-  return z / (z + 1.f);
-}
 
-// tokens of wave w: [T w / 4, T (w + 1) / 4)
-__device__ __forceinline__ void quarter(int T, int w, int& lo, int& hi) {
-  lo = (int)((int64_t)T * w / 4);
-  hi = (int)((int64_t)T * (w + 1) / 4);
-}
+constexpr int kDtThreads = 512;
+constexpr int kDtRun = 16;  // tokens per thread
+template <int HT>
+struct DtCfg {
+  static constexpr int NS = kDtThreads / HT;     // runs per workgroup
+  static constexpr int CT = NS * kDtRun;         // tokens per chunk
+};
 
-__global__ __launch_bounds__(256) void mamba2_dt_cumsum_kernel(const DtArgs a) {
-  __shared__ float part[4][64];
-  const int hb = (a.H + 63) / 64;
-  const int r = blockIdx.x / hb;
-  const int h = (blockIdx.x % hb) * 64 + (threadIdx.x & 63);
-  const int w = threadIdx.x >> 6;
-  const bool hv = h < a.H;
-  const float Ah = hv ? a.A[h] : 0.f;
-  const float bh = (hv && a.bias) ? a.bias[h] : 0.f;
-  int lo, hi;
-  quarter(a.T, w, lo, hi);
-  const int64_t base = (int64_t)r * a.T * a.H + h;
-  auto e_of = [&](int t) -> float {
-    const float x = dt_at(a, base + (int64_t)t * a.H);
-    return a.softplus ? softplus_t(x + bh) : x;
-  };
-  float s = 0.f;
-  if (hv) {
-#pragma unroll 8
-    for (int t = lo; t < hi; ++t) s += Ah * e_of(t);
+// A workgroup's chunk and a thread's run: [t0, t0 + n) of head h, run s of the chunk.
+template <int HT>
+struct DtPos {
+  int row, h, s, c, n;
+  bool hv;
+  int64_t t0, base;  // element of (row, t0, h)
+  __device__ __forceinline__ explicit DtPos(const DtArgs& a) {
+    const int hb = (a.H + HT - 1) / HT;
+    c = blockIdx.x % a.nchunk;
+    const int rb = blockIdx.x / a.nchunk;
+    row = rb / hb;
+    h = (rb % hb) * HT + (int)(threadIdx.x % HT);
+    s = threadIdx.x / HT;
+    hv = h < a.H;
+    t0 = (int64_t)c * DtCfg<HT>::CT + s * kDtRun;
+    n = !hv || t0 >= a.T ? 0 : (a.T - t0 < kDtRun ? (int)(a.T - t0) : kDtRun);
+    base = ((int64_t)row * a.T + t0) * a.H + h;
   }
-  part[w][threadIdx.x & 63] = s;
-  __syncthreads();
+};
+
+// sum of the values of the runs before s (or after s) at this thread's head
+template <int HT, bool AFTER>
+__device__ __forceinline__ float dt_other_runs(const float (*part)[HT], int s) {
+  float v = 0.f;
+  const int col = threadIdx.x % HT;
+  if (AFTER) {
+    for (int r = DtCfg<HT>::NS - 1; r > s; --r) v += part[r][col];
+  } else {
+    for (int r = 0; r < s; ++r) v += part[r][col];
+  }
+  return v;
+}
+
+// ---------------------------------------------------------------- forward
+// cum_A within the chunk (from zero), e; with one chunk also the decay
+template <int HT>
+__global__ __launch_bounds__(kDtThreads) void mamba2_dt_scan_kernel(const DtArgs a) {
+  __shared__ float part[DtCfg<HT>::NS][HT];
+  const DtPos<HT> p(a);
+  const float Ah = p.hv ? a.A[p.h] : 0.f;
+  const float bh = (p.hv && a.bias) ? a.bias[p.h] : 0.f;
+  float c[kDtRun];
+#pragma unroll
+  for (int i = 0; i < kDtRun; ++i) c[i] = i < p.n ? dt_at(a, p.base + (int64_t)i * a.H) : 0.f;
   float run = 0.f;
-  for (int v = 0; v < w; ++v) run += part[v][threadIdx.x & 63];
-  if (hv) {
-#pragma unroll 8
-    for (int t = lo; t < hi; ++t) {
-      const float e = e_of(t);
-      run += Ah * e;
-      a.cum_A[base + (int64_t)t * a.H] = run;
-      if (a.e_out) a.e_out[base + (int64_t)t * a.H] = e;
-    }
-    if (w == 3) a.decay[(int64_t)r * a.H + h] = expf(run);
+#pragma unroll
+  for (int i = 0; i < kDtRun; ++i) {
+    const float e = a.softplus ? softplus_t(c[i] + bh) : c[i];
+    if (a.e_out && i < p.n) a.e_out[p.base + (int64_t)i * a.H] = e;
+    run += i < p.n ? Ah * e : 0.f;
+    c[i] = run;
   }
+  part[p.s][threadIdx.x % HT] = run;
+  __syncthreads();
+  const float before = dt_other_runs<HT, false>(part, p.s);
+#pragma unroll
+  for (int i = 0; i < kDtRun; ++i)
+    if (i < p.n) a.cum_A[p.base + (int64_t)i * a.H] = before + c[i];
+  if (a.nchunk == 1 && p.n > 0 && p.t0 + p.n == a.T)
+    a.decay[(int64_t)p.row * a.H + p.h] = expf(before + run);
 }
 
-// G_t = g_cum_t (+ g_decay decay at t = T-1);  R_s = sum_{t>=s} G_t;
-// g_e_s = A R_s (+ the direct g_e_s);  g_A += sum_s R_s e_s;  g_dt_s = g_e_s softplus'(dt_s + bias)
-// (or g_e_s);  g_bias += sum_s g_dt_s (softplus only).
-__global__ __launch_bounds__(256) void mamba2_dt_cumsum_bwd_kernel(const DtArgs a) {
-  __shared__ float part[4][64];
-  __shared__ float red[2][4][64];
+// What the chunks hand on, in place, one value per chunk and head: INCL: x[c] := sum_{c'<=c}
+// x[c'] (and the decay of the whole row); else x[c] := first + sum_{c'>c} x[c'] (SUFFIX), or
+// -sum_{c'<c} x[c']. 16 waves x 64 heads; wave w folds a sixteenth of the chunks.
+enum { kDtInclusive, kDtSuffix, kDtNegPrefix };
+template <int KIND>
+__global__ __launch_bounds__(1024) void mamba2_dt_chunks_kernel(const DtArgs a, float* x, int CT,
+                                                                int at_end) {
+  __shared__ float part[16][64];
   const int hb = (a.H + 63) / 64;
-  const int r = blockIdx.x / hb;
-  const int lane = threadIdx.x & 63;
+  const int row = blockIdx.x / hb, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int h = (blockIdx.x % hb) * 64 + lane;
-  const int w = threadIdx.x >> 6;
   const bool hv = h < a.H;
-  const float Ah = hv ? a.A[h] : 0.f;
-  const float bh = (hv && a.bias) ? a.bias[h] : 0.f;
-  int lo, hi;
-  quarter(a.T, w, lo, hi);
-  const int64_t base = (int64_t)r * a.T * a.H + h;
-  const float gd = (hv && a.g_decay) ? a.g_decay[(int64_t)r * a.H + h] * a.decay[(int64_t)r * a.H + h]
-                                     : 0.f;
-  auto G_of = [&](int t) -> float {
-    float g = a.g_cum ? a.g_cum[base + (int64_t)t * a.H] : 0.f;
-    return t == a.T - 1 ? g + gd : g;
+  const int n = a.nchunk;
+  const int lo = (int)((int64_t)n * w / 16), hi = (int)((int64_t)n * (w + 1) / 16);
+  auto at = [&](int c) -> int64_t {  // the chunk's last (at_end) or first token
+    const int64_t first = (int64_t)c * CT, end = first + CT < a.T ? first + CT : a.T;
+    return ((int64_t)row * a.T + (at_end ? end - 1 : first)) * a.H + h;
   };
   float s = 0.f;
   if (hv) {
 #pragma unroll 8
-    for (int t = lo; t < hi; ++t) s += G_of(t);
+    for (int c = lo; c < hi; ++c) s += x[at(c)];
   }
   part[w][lane] = s;
   __syncthreads();
-  float run = 0.f;  // suffix sum of the later quarters
-  for (int v = w + 1; v < 4; ++v) run += part[v][lane];
-  float pa = 0.f, pb = 0.f;
-  if (hv) {
+  if (!hv) return;
+  float run = 0.f;
+  if (KIND == kDtSuffix) {
+    if (a.g_decay) run = a.g_decay[(int64_t)row * a.H + h] * a.decay[(int64_t)row * a.H + h];
+    for (int v = 15; v > w; --v) run += part[v][lane];
 #pragma unroll 8
-    for (int t = hi - 1; t >= lo; --t) {
-      run += G_of(t);
-      const float x = dt_at(a, base + (int64_t)t * a.H);
-      const float e = a.softplus ? softplus_t(x + bh) : x;
-      pa += run * e;
-      const float ge = Ah * run + (a.g_e ? a.g_e[base + (int64_t)t * a.H] : 0.f);
-      const float gdt = a.softplus ? ge * softplus_grad(x + bh) : ge;
-      pb += gdt;
-      a.g_dt[base + (int64_t)t * a.H] = gdt;
+    for (int c = hi - 1; c >= lo; --c) {
+      const float v = x[at(c)];
+      x[at(c)] = run;
+      run += v;
+    }
+  } else {
+    for (int v = 0; v < w; ++v) run += part[v][lane];
+#pragma unroll 8
+    for (int c = lo; c < hi; ++c) {
+      const float v = x[at(c)];
+      if (KIND == kDtNegPrefix) x[at(c)] = -run;
+      run += v;
+      if (KIND == kDtInclusive) x[at(c)] = run;
+    }
+    if (KIND == kDtInclusive && w == 15) a.decay[(int64_t)row * a.H + h] = expf(run);
+  }
+}
+
+// chunk c > 0: every token but the last (already final) plus the last token of chunk c - 1
+template <int HT>
+__global__ __launch_bounds__(kDtThreads) void mamba2_dt_carry_kernel(const DtArgs a) {
+  const DtPos<HT> p(a);
+  if (p.c == 0 || p.n <= 0) return;
+  const int64_t first = (int64_t)p.c * DtCfg<HT>::CT;
+  const int64_t end = first + DtCfg<HT>::CT < a.T ? first + DtCfg<HT>::CT : a.T;
+  const float in = a.cum_A[((int64_t)p.row * a.T + first - 1) * a.H + p.h];
+  const int n = p.t0 + p.n == end ? p.n - 1 : p.n;
+  float c[kDtRun];
+#pragma unroll
+  for (int i = 0; i < kDtRun; ++i) c[i] = i < n ? a.cum_A[p.base + (int64_t)i * a.H] : 0.f;
+#pragma unroll
+  for (int i = 0; i < kDtRun; ++i)
+    if (i < n) a.cum_A[p.base + (int64_t)i * a.H] = in + c[i];
+}
+
+// ---------------------------------------------------------------- backward
+// g_dt at the chunk's first token := sum of the chunk's g_cum
+template <int HT>
+__global__ __launch_bounds__(kDtThreads) void mamba2_dt_sums_kernel(const DtArgs a) {
+  __shared__ float part[DtCfg<HT>::NS][HT];
+  const DtPos<HT> p(a);
+  float g[kDtRun];
+#pragma unroll
+  for (int i = 0; i < kDtRun; ++i) g[i] = i < p.n ? a.g_cum[p.base + (int64_t)i * a.H] : 0.f;
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < kDtRun; ++i) s += g[i];
+  part[p.s][threadIdx.x % HT] = s;
+  __syncthreads();
+  if (p.s == 0 && p.hv) a.g_dt[p.base] = s + dt_other_runs<HT, true>(part, 0);
+}
+
+// G_t = g_cum_t (+ g_decay decay at t = T-1);  R_s = sum_{t>=s} G_t, or (CLOSED: g_cum_{T-1}
+// stands for minus the sum of the others) R_s = -sum_{t<s} G_t, summed from the front so that
+// the small R of early tokens keep their precision;
+// g_e_s = A R_s (+ the direct g_e_s);  g_A += sum_s R_s e_s;  g_dt_s = g_e_s softplus'(dt_s + bias)
+// (or g_e_s);  g_bias += sum_s g_dt_s (softplus only).
+template <int HT, bool CLOSED>
+__global__ __launch_bounds__(kDtThreads) void mamba2_dt_bwd_kernel(const DtArgs a) {
+  __shared__ float part[DtCfg<HT>::NS][HT];
+  __shared__ float red[2][DtCfg<HT>::NS][HT];
+  const DtPos<HT> p(a);
+  const int col = threadIdx.x % HT;
+  const float Ah = p.hv ? a.A[p.h] : 0.f;
+  const float bh = (p.hv && a.bias) ? a.bias[p.h] : 0.f;
+  float in = 0.f;  // what enters the chunk
+  if (p.hv) {
+    if (a.nchunk > 1 && a.g_cum)
+      in = a.g_dt[((int64_t)p.row * a.T + (int64_t)p.c * DtCfg<HT>::CT) * a.H + p.h];
+    else if (!CLOSED && a.g_decay)
+      in = a.g_decay[(int64_t)p.row * a.H + p.h] * a.decay[(int64_t)p.row * a.H + p.h];
+  }
+  float g[kDtRun], x[kDtRun], d[kDtRun];
+#pragma unroll
+  for (int i = 0; i < kDtRun; ++i) {
+    const int64_t at = p.base + (int64_t)i * a.H;
+    g[i] = i < p.n && a.g_cum ? a.g_cum[at] : 0.f;
+    x[i] = i < p.n ? dt_at(a, at) : 0.f;
+    d[i] = i < p.n && a.g_e ? a.g_e[at] : 0.f;
+  }
+  float run = 0.f;
+  if (CLOSED) {
+#pragma unroll
+    for (int i = 0; i < kDtRun; ++i) {
+      const float v = g[i];
+      g[i] = run;
+      run -= v;
+    }
+  } else {
+#pragma unroll
+    for (int i = kDtRun - 1; i >= 0; --i) {
+      run += g[i];
+      g[i] = run;
     }
   }
-  red[0][w][lane] = pa;
-  red[1][w][lane] = pb;
-  __syncthreads();
-  if (w == 0 && hv) {
-    const float sa = red[0][0][lane] + red[0][1][lane] + red[0][2][lane] + red[0][3][lane];
-    const float sb = red[1][0][lane] + red[1][1][lane] + red[1][2][lane] + red[1][3][lane];
-    atomicAdd(a.g_A + h, sa);
-    if (a.softplus && a.g_bias) atomicAdd(a.g_bias + h, sb);
+  part[p.s][col] = run;
+  __syncthreads();  // (also: every thread has read the chunk's first g_dt)
+  in += dt_other_runs<HT, !CLOSED>(part, p.s);
+  float pa = 0.f, pb = 0.f;
+#pragma unroll
+  for (int i = 0; i < kDtRun; ++i) {
+    const float R = in + g[i], y = x[i] + bh;
+    const float ge = Ah * R + d[i];
+    float e = x[i], gdt = ge;
+    if (a.softplus) {
+      const float z = expf(y);
+      e = y > 20.f ? y : log1pf(z);
+      gdt = y > 20.f ? ge : ge * (z / (z + 1.f));
+    }
+    if (i < p.n) {
+      pa += R * e;
+      pb += gdt;
+      a.g_dt[p.base + (int64_t)i * a.H] = gdt;
+    }
   }
+  red[0][p.s][col] = pa;
+  red[1][p.s][col] = pb;
+  __syncthreads();
+  if (p.s == 0 && p.hv) {
+    atomicAdd(a.g_A + p.h, pa + dt_other_runs<HT, true>(red[0], 0));
+    if (a.softplus && a.g_bias) atomicAdd(a.g_bias + p.h, pb + dt_other_runs<HT, true>(red[1], 0));
+  }
+}
+
+// ---------------------------------------------------------------- launchers
+template <int HT>
+static int dt_grid(DtArgs& a) {
+  a.nchunk = (int)(((int64_t)a.T + DtCfg<HT>::CT - 1) / DtCfg<HT>::CT);
+  return (int)((int64_t)a.rows * ((a.H + HT - 1) / HT) * a.nchunk);
+}
+
+template <int HT>
+static void launch_dt_fwd(DtArgs a, hipStream_t stream) {
+  const unsigned grid = (unsigned)dt_grid<HT>(a), rows = (unsigned)(a.rows * ((a.H + 63) / 64));
+  hipLaunchKernelGGL((mamba2_dt_scan_kernel<HT>), dim3(grid), dim3(kDtThreads), 0, stream, a);
+  if (a.nchunk == 1) return;
+  hipLaunchKernelGGL((mamba2_dt_chunks_kernel<kDtInclusive>), dim3(rows), dim3(1024), 0, stream, a,
+                     a.cum_A, DtCfg<HT>::CT, 1);
+  hipLaunchKernelGGL((mamba2_dt_carry_kernel<HT>), dim3(grid), dim3(kDtThreads), 0, stream, a);
+}
+
+template <int HT, bool CLOSED>
+static void launch_dt_bwd(DtArgs a, hipStream_t stream) {
+  const unsigned grid = (unsigned)dt_grid<HT>(a), rows = (unsigned)(a.rows * ((a.H + 63) / 64));
+  if (a.nchunk > 1 && a.g_cum) {
+    hipLaunchKernelGGL((mamba2_dt_sums_kernel<HT>), dim3(grid), dim3(kDtThreads), 0, stream, a);
+    hipLaunchKernelGGL((mamba2_dt_chunks_kernel<CLOSED ? kDtNegPrefix : kDtSuffix>), dim3(rows),
+                       dim3(1024), 0, stream, a, a.g_dt, DtCfg<HT>::CT, 0);
+  }
+  hipLaunchKernelGGL((mamba2_dt_bwd_kernel<HT, CLOSED>), dim3(grid), dim3(kDtThreads), 0, stream, a);
 }
 
 hipError_t launch_mamba2_dt_cumsum(const void* dt, int dt_f32, const float* bias, const float* A,
                                    int softplus, float* cum_A, float* e, float* decay, int rows,
                                    int T, int H, hipStream_t stream) {
-  DtArgs a{dt, dt_f32, bias, A, softplus, cum_A, e, nullptr, decay, nullptr, nullptr, nullptr,
-           nullptr, nullptr, rows, T, H};
-  const int64_t grid = (int64_t)rows * ((H + 63) / 64);
-  if (grid == 0) return hipSuccess;
-  hipLaunchKernelGGL(mamba2_dt_cumsum_kernel, dim3((unsigned)grid), dim3(256), 0, stream, a);
+  const DtArgs a{dt, dt_f32, bias, A, softplus, cum_A, e, nullptr, decay, nullptr, nullptr, nullptr,
+                 nullptr, nullptr, rows, T, H, 0};
+  if ((int64_t)rows * T * H == 0) return hipSuccess;
+  if (H <= 8) launch_dt_fwd<8>(a, stream);
+  else if (H <= 16) launch_dt_fwd<16>(a, stream);
+  else if (H <= 32) launch_dt_fwd<32>(a, stream);
+  else launch_dt_fwd<64>(a, stream);
   return hipGetLastError();
+}
+
+template <bool CLOSED>
+static void launch_dt_bwd_h(const DtArgs& a, hipStream_t stream) {
+  if (a.H <= 8) launch_dt_bwd<8, CLOSED>(a, stream);
+  else if (a.H <= 16) launch_dt_bwd<16, CLOSED>(a, stream);
+  else if (a.H <= 32) launch_dt_bwd<32, CLOSED>(a, stream);
+  else launch_dt_bwd<64, CLOSED>(a, stream);
 }
 
 hipError_t launch_mamba2_dt_cumsum_bwd(const void* dt, int dt_f32, const float* bias,
                                        const float* A, int softplus, const float* g_cum,
                                        const float* g_e, const float* g_decay, const float* decay,
                                        float* g_dt, float* g_A, float* g_bias, int rows, int T,
-                                       int H, hipStream_t stream) {
-  DtArgs a{dt, dt_f32, bias, A, softplus, nullptr, nullptr, g_e, const_cast<float*>(decay),
-           g_cum, g_decay, g_dt, g_A, g_bias, rows, T, H};
-  const int64_t grid = (int64_t)rows * ((H + 63) / 64);
-  if (grid == 0) return hipSuccess;
-  hipLaunchKernelGGL(mamba2_dt_cumsum_bwd_kernel, dim3((unsigned)grid), dim3(256), 0, stream, a);
+                                       int H, int closed, hipStream_t stream) {
+  const DtArgs a{dt, dt_f32, bias, A, softplus, nullptr, nullptr, g_e, const_cast<float*>(decay),
+                 g_cum, g_decay, g_dt, g_A, g_bias, rows, T, H, 0};
+  if ((int64_t)rows * T * H == 0) return hipSuccess;
+  if (closed) launch_dt_bwd_h<true>(a, stream);
+  else launch_dt_bwd_h<false>(a, stream);
   return hipGetLastError();
 }
 

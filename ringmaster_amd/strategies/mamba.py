@@ -129,41 +129,46 @@ def cp_state_prefix(ssm_state: torch.Tensor, chunk_decay: torch.Tensor, group=No
     return cp_state_prefix_gathered(ssm_state[None], chunk_decay[None], 0, single_hop=single_hop)
 
 
+def _dt_forward(dt, A, dt_bias, softplus, want_e):
+    """(cum_A, decay, e) from dt ``[rows, T, H]``; e (the effective dt) None unless ``want_e``."""
+    rows, T, H = dt.shape
+    cum = torch.empty((rows, T, H), dtype=torch.float32, device=dt.device)
+    decay = torch.empty((rows, H), dtype=torch.float32, device=dt.device)
+    e = torch.empty_like(cum) if want_e else None
+    abi.check(abi.lib().rmx_mamba2_dt_cumsum(
+        dt.data_ptr(), int(dt.dtype == torch.float32), abi.ptr(dt_bias), A.data_ptr(),
+        int(softplus), cum.data_ptr(), abi.ptr(e), decay.data_ptr(), rows, T, H,
+        abi.stream_of(dt)))
+    return cum, decay, e
+
+
 class _DtCumsum(torch.autograd.Function):
-    """(cum_A, decay, e) from dt; e (the effective dt) only when ``want_e``."""
+    """(cum_A, decay) from dt."""
 
     @staticmethod
-    def forward(ctx, dt, A, dt_bias, softplus, want_e):
-        rows, T, H = dt.shape
-        cum = torch.empty((rows, T, H), dtype=torch.float32, device=dt.device)
-        decay = torch.empty((rows, H), dtype=torch.float32, device=dt.device)
-        e = torch.empty((rows, T, H) if want_e else (0,), dtype=torch.float32, device=dt.device)
-        abi.check(abi.lib().rmx_mamba2_dt_cumsum(
-            dt.data_ptr(), int(dt.dtype == torch.float32), abi.ptr(dt_bias), A.data_ptr(),
-            int(softplus), cum.data_ptr(), e.data_ptr() if want_e else None, decay.data_ptr(),
-            rows, T, H, abi.stream_of(dt)))
+    def forward(ctx, dt, A, dt_bias, softplus):
+        cum, decay, _ = _dt_forward(dt, A, dt_bias, softplus, False)
         ctx.save_for_backward(dt, A, dt_bias, decay)
         ctx.softplus = softplus
         ctx.set_materialize_grads(False)
-        return cum, decay, e
+        return cum, decay
 
     @staticmethod
-    def backward(ctx, g_cum, g_decay, g_e):
+    def backward(ctx, g_cum, g_decay):
         dt, A, dt_bias, decay = ctx.saved_tensors
         rows, T, H = dt.shape
-        if g_cum is None and g_decay is None and g_e is None:
-            return None, None, None, None, None
+        if g_cum is None and g_decay is None:
+            return None, None, None, None
         g_cum = None if g_cum is None else g_cum.contiguous().float()
         g_decay = None if g_decay is None else g_decay.contiguous().float()
-        g_e = None if g_e is None or g_e.numel() == 0 else g_e.contiguous().float()
         g_dt = torch.empty((rows, T, H), dtype=torch.float32, device=dt.device)
         g_A = torch.zeros(H, dtype=torch.float32, device=dt.device)
         g_b = torch.zeros(H, dtype=torch.float32, device=dt.device) if dt_bias is not None else None
         abi.check(abi.lib().rmx_mamba2_dt_cumsum_bwd(
             dt.data_ptr(), int(dt.dtype == torch.float32), abi.ptr(dt_bias), A.data_ptr(),
-            int(ctx.softplus), abi.ptr(g_cum), abi.ptr(g_e), abi.ptr(g_decay), decay.data_ptr(),
+            int(ctx.softplus), abi.ptr(g_cum), None, abi.ptr(g_decay), decay.data_ptr(),
             g_dt.data_ptr(), g_A.data_ptr(), abi.ptr(g_b), rows, T, H, abi.stream_of(dt)))
-        return g_dt.to(dt.dtype), g_A, g_b, None, None
+        return g_dt.to(dt.dtype), g_A, g_b, None
 
 
 def mamba2_chunk_decay(dt: torch.Tensor, A: torch.Tensor, dt_bias: torch.Tensor | None = None,
@@ -186,25 +191,31 @@ def mamba2_chunk_decay(dt: torch.Tensor, A: torch.Tensor, dt_bias: torch.Tensor 
     b32 = None
     if dt_softplus and dt_bias is not None:
         b32 = dt_bias.float().contiguous()
-    cum, decay, _ = _DtCumsum.apply(d3, A32, b32, bool(dt_softplus), False)
+    cum, decay = _DtCumsum.apply(d3, A32, b32, bool(dt_softplus))
     return cum.reshape(*lead, T, H), decay.reshape(*lead, H)
 
 
 class _ChunkState(torch.autograd.Function):
+    """The shard state from x, B and the step (dt through ``softplus`` and the bias), whose
+    cumsum and effective values stay inside: their gradients go from the state's backward
+    kernel straight into the cumsum's."""
+
     @staticmethod
-    def forward(ctx, x, B, e, cum_A, t0):
+    def forward(ctx, x, B, dt, A, dt_bias, softplus, t0):
         rows, T, H, D = x.shape
         G, N = B.shape[2], B.shape[3]
+        cum_A, _, e = _dt_forward(dt, A, dt_bias, softplus, True)
         state = torch.empty((rows, H, D, N), dtype=torch.float32, device=x.device)
         abi.check(abi.lib().rmx_mamba2_chunk_state(
             x.data_ptr(), B.data_ptr(), e.data_ptr(), cum_A.data_ptr(), abi.ptr(t0),
             state.data_ptr(), rows, T, H, D, G, N, abi.stream_of(x)))
-        ctx.save_for_backward(x, B, e, cum_A, t0)
+        ctx.save_for_backward(x, B, dt, A, dt_bias, e, cum_A, t0)
+        ctx.softplus = softplus
         return state
 
     @staticmethod
     def backward(ctx, g):
-        x, B, e, cum_A, t0 = ctx.saved_tensors
+        x, B, dt, A, dt_bias, e, cum_A, t0 = ctx.saved_tensors
         rows, T, H, D = x.shape
         G, N = B.shape[2], B.shape[3]
         g = g.contiguous().float()
@@ -218,10 +229,15 @@ class _ChunkState(torch.autograd.Function):
             x.data_ptr(), B.data_ptr(), e.data_ptr(), cum_A.data_ptr(), abi.ptr(t0),
             g.data_ptr(), g_x.data_ptr(), g_B.data_ptr(), g_e.data_ptr(), g_cum.data_ptr(),
             rows, T, H, D, G, N, abi.ptr(ws), ws_bytes, abi.stream_of(x)))
-        if T:
-            # every weight exp(cum_A[T-1] - cum_A[t]) also depends on cum_A[T-1]
-            g_cum[:, T - 1] = -g_cum[:, :T - 1].sum(1)
-        return g_x, g_B, g_e, g_cum, None
+        g_dt = torch.empty_like(g_e)
+        g_A = torch.zeros(H, dtype=torch.float32, device=x.device)
+        g_b = torch.zeros(H, dtype=torch.float32, device=x.device) if dt_bias is not None else None
+        # (g_cum at T-1, on which every weight depends, is minus the sum of the others there)
+        abi.check(lib.rmx_mamba2_dt_cumsum_state_bwd(
+            dt.data_ptr(), int(dt.dtype == torch.float32), abi.ptr(dt_bias), A.data_ptr(),
+            int(ctx.softplus), g_cum.data_ptr(), g_e.data_ptr(), g_dt.data_ptr(), g_A.data_ptr(),
+            abi.ptr(g_b), rows, T, H, abi.stream_of(x)))
+        return g_x, g_B, g_dt.to(dt.dtype), g_A, g_b, None, None
 
 
 def last_document_start(seq_idx: torch.Tensor) -> torch.Tensor:
@@ -268,21 +284,20 @@ def mamba2_chunk_state(x: torch.Tensor, dt: torch.Tensor, A: torch.Tensor, B: to
     if dt_softplus and lo <= 0.0 and hi == float("inf"):
         # softplus >= 0, so the clamp is the identity: the dt kernel computes the step
         b32 = dt_bias.float().contiguous() if dt_bias is not None else None
-        cum, _, e = _DtCumsum.apply(d3, A.float().contiguous(), b32, True, True)
+        step, soft = d3, True
     else:
         # a bias without softplus, or a clamp that bites: the step in fp32 elementwise
         # ops first (mamba.py:143-148), then the kernel's cumsum over it
         step = d3.float() if dt_bias is None else d3.float() + dt_bias.float()
         if dt_softplus:
             step = torch.nn.functional.softplus(step)
-        step = step.clamp(lo, hi).contiguous()
-        cum, _, e = _DtCumsum.apply(step, A.float().contiguous(), None, False, True)
+        step, b32, soft = step.clamp(lo, hi).contiguous(), None, False
     t0 = None
     if seq_idx is not None:
         if tuple(seq_idx.shape) != (*lead, T):
             raise ValueError("seq_idx must be [..., T]")
         t0 = last_document_start(seq_idx.reshape(-1, T))
-    state = _ChunkState.apply(x3, B3, e, cum, t0)
+    state = _ChunkState.apply(x3, B3, step, A.float().contiguous(), b32, soft, t0)
     return state.reshape(*lead, H, D, N)
 
 

@@ -1,0 +1,81 @@
+"""The chunked dt cumsum (rmx_mamba2_dt_cumsum and its two backwards) at the edges of its
+chunks: 512 / HT runs of 16 tokens, HT = 8, 16, 32 or 64 heads per workgroup."""
+import pytest
+import torch
+
+from tests.gpu_util import seeded
+
+pytestmark = pytest.mark.gpu
+
+# chunk tokens: H <= 8: 1024, <= 16: 512, <= 32: 256, else 128
+CASES = [(1, 1, 1), (2, 1024, 8), (1, 1025, 3), (2, 513, 16), (1, 255, 24), (2, 769, 32),
+         (1, 128, 64), (2, 129, 64), (3, 2000, 65), (1, 17, 130)]
+
+
+@pytest.mark.parametrize("softplus,f32", [(True, False), (True, True), (False, True)])
+@pytest.mark.parametrize("rows,T,H", CASES)
+def test_dt_cumsum_chunks(rows, T, H, softplus, f32):
+    """Values within 8 fp32 roundings of the largest prefix (chunk, run and token sums of one
+    sign), gradients within the same of their absolute sums, against fp64."""
+    from ringmaster_amd import abi
+
+    print(f"case dt rows={rows} T={T} H={H} softplus={softplus} f32={f32}", flush=True)
+    raw = seeded((rows, T, H), 1)
+    # without softplus the step itself is given, and steps are positive
+    dt = (raw if softplus else 0.1 * raw.abs()).to(torch.float32 if f32 else torch.bfloat16)
+    bias = seeded((H,), 2) - 2.0 if softplus else None
+    A = -torch.exp(seeded((H,), 3))
+    g_cum, g_e, g_dec = seeded((rows, T, H), 4), seeded((rows, T, H), 5), seeded((rows, H), 6)
+
+    def ref(closed):
+        d, a = dt.double().requires_grad_(True), A.double().requires_grad_(True)
+        b = bias.double().requires_grad_(True) if softplus else None
+        e = torch.nn.functional.softplus(d + b) if softplus else d * 1.0
+        cum = torch.cumsum(e * a, 1)
+        g = g_cum.double()
+        loss = (e * g_e.double()).sum()
+        if closed:
+            loss = loss + ((cum - cum[:, -1:]) * g)[:, :-1].sum()
+        else:
+            loss = loss + (cum * g).sum() + (torch.exp(cum[:, -1]) * g_dec.double()).sum()
+        leaves = [d, a] + ([b] if softplus else [])
+        return e, cum, torch.autograd.grad(loss, leaves)
+
+    dev = lambda x: None if x is None else x.cuda()  # noqa: E731
+    dd, bd, Ad, gc, ge, gd = (dev(x) for x in (dt, bias, A, g_cum, g_e, g_dec))
+    cum, e, decay = (torch.empty(s, device="cuda") for s in ((rows, T, H), (rows, T, H), (rows, H)))
+    lib, s = abi.lib(), abi.stream_of(dd)
+    abi.check(lib.rmx_mamba2_dt_cumsum(dd.data_ptr(), int(f32), abi.ptr(bd), Ad.data_ptr(),
+                                       int(softplus), cum.data_ptr(), e.data_ptr(),
+                                       decay.data_ptr(), rows, T, H, s))
+    e_r, cum_r, _ = ref(False)
+    eps = 2.0 ** -23
+    scale = (e_r * A.double()).abs().sum(1, keepdim=True).detach()
+    assert ((cum.cpu() - cum_r).abs() <= 8 * eps * scale + 1e-30).all()
+    assert ((e.cpu() - e_r).abs() <= 8 * eps * e_r.abs() + 1e-30).all()
+    # exp turns the absolute error of cum_A into a relative one
+    dec_r = torch.exp(cum_r[:, -1]).detach()
+    dec_err = (16 * eps * (1 + scale[:, 0])) * dec_r + 1e-37
+    assert ((decay.cpu() - dec_r).abs() <= dec_err).all()
+
+    for closed in (False, True):
+        g_dt = torch.empty_like(cum)
+        g_A, g_b = torch.zeros(H, device="cuda"), torch.zeros(H, device="cuda")
+        head = (dd.data_ptr(), int(f32), abi.ptr(bd), Ad.data_ptr(), int(softplus))
+        tail = (g_dt.data_ptr(), g_A.data_ptr(), g_b.data_ptr() if softplus else None, rows, T, H, s)
+        if closed:
+            abi.check(lib.rmx_mamba2_dt_cumsum_state_bwd(*head, gc.data_ptr(), ge.data_ptr(), *tail))
+        else:
+            abi.check(lib.rmx_mamba2_dt_cumsum_bwd(*head, gc.data_ptr(), ge.data_ptr(),
+                                                   gd.data_ptr(), decay.data_ptr(), *tail))
+        _, _, grads = ref(closed)
+        # the summands a suffix sum can hold (the decay's own error with them), times |A|, plus
+        # the direct gradient
+        g_abs = g_cum.double().abs().sum(1, keepdim=True) + (
+            (dec_r + dec_err / eps) * g_dec.double()).abs()[:, None]
+        bar = 32 * eps * (A.double().abs() * g_abs + g_e.double().abs())
+        assert ((g_dt.cpu() - grads[0]).abs() <= bar).all()
+        bar_A = 32 * eps * (g_abs * e_r.detach().abs()).sum((0, 1))
+        assert ((g_A.cpu() - grads[1]).abs() <= bar_A).all()
+        if softplus:
+            assert ((g_b.cpu() - grads[2]).abs() <= bar.sum((0, 1))).all()
