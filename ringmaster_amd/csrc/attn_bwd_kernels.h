@@ -1148,53 +1148,149 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_kernel(const BwdParams p
   wait_all_loads();  // zero-length loads issued past the end
 
   // ---- epilogue: lane (hl, l32) holds column d = 32 db + l32 of keys kw0 + c_row(hl, r).
-  // The accumulating modes read all of the lane's prior dV and dK values before the first
-  // store: element by element, each read would wait for the store before it (the compiler
-  // cannot tell that they touch different elements), one memory round trip per element.
-  const int mode = P.dkv_mode;
+  // Stored from there, every element is a 2- or 4-byte store with its own 64-bit address and
+  // mode test: 128 of them per lane and about 50 KB of code, 20 us per workgroup (a launch of
+  // one 64-query tile took 28 us). The gradients go through the dead tile buffers instead
+  // (each wave's 32 keys as fp32 rows, dV in the Q tiles, dK in the dO tiles, the halves of
+  // 64-column groups swapped in every second group of four rows so that the two lane halves
+  // write different banks) and come back as 16-byte chunks of whole rows, one mode test per
+  // chunk; the accumulating modes read all of a lane's prior chunks before its first store
+  // (one wait, not one memory round trip per row). A launch of one tile: 28.4 -> 12.8 us at
+  // head dim 128, 19.4 -> 8.7 at 64.
+  // Caller pointers below vector alignment take the element-wise form, straight from the
+  // accumulators; the document and dropout kernels a compact loop over the staged rows. The
+  // choice is the register allocator's: with the compact loop the FULL and causal main loops
+  // move 47 values per tile between VGPRs and AGPRs instead of 14 and run 1% slower, with the
+  // element-wise form the document loop takes 20 more VALU instructions per tile and the
+  // dropout kernels spill 192 registers (the compact form: none).
+  constexpr int CPR = HD / 4;    // 16-byte chunks per fp32 row
+  constexpr int RPI = 64 / CPR;  // rows per instruction of a wave
+  constexpr int NI = 32 / RPI;   // instructions per wave and gradient
+  static_assert(C::BKV * HD * 4 <= NB * C::QT, "gradient staging");
+  int pe = wc.p;  // read the problem anew: its pointers are not kept in SGPRs across the loop
+  asm volatile("" : "+s"(pe));
+  const rmx_bwd_problem& E = prm.P[pe];
+  const int mode = E.dkv_mode;
   const bool rd = mode == RMX_GRAD_ACC_F32 || mode == RMX_GRAD_ACC_FINAL;
-  float prev[2][NDB][16];
-  if (rd) {
+  const bool w32 = mode == RMX_GRAD_WRITE_F32 || mode == RMX_GRAD_ACC_F32;
+  const bool vec = (!(rd || w32) || (((uintptr_t)E.dv_acc | (uintptr_t)E.dk_acc) & 15) == 0) &&
+                   (w32 || (((uintptr_t)E.dv | (uintptr_t)E.dk) & 7) == 0);
+  constexpr bool ELEMS = !DROP && MASK != RMX_MASK_DOC;
+  if (ELEMS && !vec) {
+    float prev[2][NDB][16];
+    if (rd) {
 #pragma unroll
-    for (int g = 0; g < 2; ++g) {
-      const float* gacc = g == 0 ? P.dv_acc : P.dk_acc;
+      for (int g = 0; g < 2; ++g) {
+        const float* gacc = g == 0 ? E.dv_acc : E.dk_acc;
 #pragma unroll
-      for (int db = 0; db < NDB; ++db) {
-        const int d = 32 * db + l32;
+        for (int db = 0; db < NDB; ++db) {
+          const int d = 32 * db + l32;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int kk = kw0 + c_row(hl, r);
-          const int64_t ao = bb * L.ka_sb + (int64_t)kk * L.ka_ss + kvh * L.ka_sh + d;
-          prev[g][db][r] = d < D && kk < sk ? gacc[ao] : 0.f;
+          for (int r = 0; r < 16; ++r) {
+            const int kk = kw0 + c_row(hl, r);
+            const int64_t ao = bb * L.ka_sb + (int64_t)kk * L.ka_ss + kvh * L.ka_sh + d;
+            prev[g][db][r] = d < D && kk < sk ? gacc[ao] : 0.f;
+          }
         }
       }
     }
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      const float sc = g == 0 ? 1.f : -L.scale;
+      float* gacc = g == 0 ? E.dv_acc : E.dk_acc;
+      uint16_t* gbf = g == 0 ? E.dv : E.dk;
+#pragma unroll
+      for (int db = 0; db < NDB; ++db) {
+        const int d = 32 * db + l32;
+        if (d >= D) continue;  // columns past the head dim are not stored
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int kk = kw0 + c_row(hl, r);
+          if (kk >= sk) continue;
+          const float gv = (g == 0 ? dv[db][r] : dk[db][r]) * sc;
+          const int64_t ao = bb * L.ka_sb + (int64_t)kk * L.ka_ss + kvh * L.ka_sh + d;
+          const int64_t bo = bb * L.dk_sb + (int64_t)kk * L.dk_ss + kvh * L.dk_sh + d;
+          if (mode == RMX_GRAD_WRITE_F32) {
+            gacc[ao] = gv;
+          } else if (mode == RMX_GRAD_ACC_F32) {
+            gacc[ao] = prev[g][db][r] + gv;
+          } else if (mode == RMX_GRAD_ACC_FINAL) {
+            gbf[bo] = f2e<DT>(prev[g][db][r] + gv);
+          } else {
+            gbf[bo] = f2e<DT>(gv);
+          }
+        }
+      }
+    }
+    return;
   }
+  __syncthreads();  // every wave is past its reads of the last tiles and its loads have landed
+  const int el = lane_again();
+  {
+    const int eh = el >> 5, e32 = el & 31;
+    float* const sv = reinterpret_cast<float*>(&sQ[0][0]) + 32 * wave * HD;
+    float* const sd = reinterpret_cast<float*>(&sO[0][0]) + 32 * wave * HD;
 #pragma unroll
-  for (int g = 0; g < 2; ++g) {
-    const float sc = g == 0 ? 1.f : -L.scale;
-    float* gacc = g == 0 ? P.dv_acc : P.dk_acc;
-    uint16_t* gbf = g == 0 ? P.dv : P.dk;
-#pragma unroll
-    for (int db = 0; db < NDB; ++db) {
-      const int d = 32 * db + l32;
-      if (d >= D) continue;  // columns past the head dim are not stored
+    for (int db = 0; db < NDB; ++db)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int kk = kw0 + c_row(hl, r);
-        if (kk >= sk) continue;
-        const float gv = (g == 0 ? dv[db][r] : dk[db][r]) * sc;
-        const int64_t ao = bb * L.ka_sb + (int64_t)kk * L.ka_ss + kvh * L.ka_sh + d;
-        const int64_t bo = bb * L.dk_sb + (int64_t)kk * L.dk_ss + kvh * L.dk_sh + d;
-        if (mode == RMX_GRAD_WRITE_F32) {
-          gacc[ao] = gv;
-        } else if (mode == RMX_GRAD_ACC_F32) {
-          gacc[ao] = prev[g][db][r] + gv;
-        } else if (mode == RMX_GRAD_ACC_FINAL) {
-          gbf[bo] = f2e<DT>(prev[g][db][r] + gv);
-        } else {
-          gbf[bo] = f2e<DT>(gv);
+        const int o = c_row(eh, r) * HD + ((32 * db + e32) ^ (32 * eh));  // (row >> 2) & 1 == eh
+        sv[o] = dv[db][r];
+        sd[o] = -L.scale * dk[db][r];
+      }
+  }
+  __syncthreads();
+  const int ch = el % CPR, rr = el / CPR;
+  if (4 * ch >= L.head_dim) return;  // columns past the head dim are not stored
+#pragma unroll 1
+  for (int g = 0; g < 2; ++g) {
+    const float* const stg = reinterpret_cast<const float*>(g == 0 ? &sQ[0][0] : &sO[0][0]) + 32 * wave * HD;
+    float* const gacc = (g == 0 ? E.dv_acc : E.dk_acc) + bb * L.ka_sb + kvh * L.ka_sh + 4 * ch;
+    uint16_t* const gbf = (g == 0 ? E.dv : E.dk) + bb * L.dk_sb + kvh * L.dk_sh + 4 * ch;
+    if (!ELEMS && !vec) {
+#pragma unroll 1
+      for (int row = rr; row < 32 && kw0 + row < sk; row += RPI) {
+        const int64_t kk = kw0 + row;
+        const float* const src = stg + row * HD + 4 * (ch ^ (8 * ((row >> 2) & 1)));
+#pragma unroll 1
+        for (int e = 0; e < 4; ++e) {
+          float* const x = gacc + kk * L.ka_ss + e;
+          const float gv = rd ? *x + src[e] : src[e];
+          if (w32)
+            *x = gv;
+          else
+            gbf[kk * L.dk_ss + e] = f2e<DT>(gv);
         }
+      }
+      continue;
+    }
+    f32x4 v[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int row = RPI * i + rr;
+      v[i] = *reinterpret_cast<const f32x4*>(stg + row * HD + 4 * (ch ^ (8 * ((row >> 2) & 1))));
+    }
+    if (rd) {
+      f32x4 prev[NI];
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int kk = kw0 + RPI * i + rr;
+        prev[i] = kk < sk ? *reinterpret_cast<const f32x4*>(gacc + (int64_t)kk * L.ka_ss) : f32x4{};
+      }
+#pragma unroll
+      for (int i = 0; i < NI; ++i) v[i] += prev[i];
+    }
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int kk = kw0 + RPI * i + rr;
+      if (kk >= sk) continue;
+      if (w32) {
+        *reinterpret_cast<f32x4*>(gacc + (int64_t)kk * L.ka_ss) = v[i];
+      } else {
+        u32x2 w;
+        w[0] = cvt_pk<DT>(v[i][0], v[i][1]);
+        w[1] = cvt_pk<DT>(v[i][2], v[i][3]);
+        *reinterpret_cast<u32x2*>(gbf + (int64_t)kk * L.dk_ss) = w;
       }
     }
   }

@@ -103,6 +103,14 @@ __device__ __forceinline__ void st16(void* p, const u32x4& v) { *reinterpret_cas
 // instead of if-converting it into per-element selects on every tile.
 __device__ __forceinline__ void keep_branch() { asm volatile(""); }
 
+// The lane index, computed anew: an epilogue that takes it from here keeps no per-lane value
+// alive across a main loop whose registers are all in use.
+__device__ __forceinline__ int lane_again() {
+  int l = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+  asm volatile("" : "+v"(l));
+  return l;
+}
+
 // Wait for every outstanding memory operation of the wave. Issued once before a
 // main loop whose body reads registers filled by loads issued before it: the
 // waitcnt pass cannot tell those loads from the loop's own prefetches, and
