@@ -1918,21 +1918,19 @@ hipError_t launch_bwd_t(const rmx_attn_layout& L, const rmx_bwd_problem* probs, 
       ik[nk++] = i;
     }
   }
-  int oq[RMX_MAX_BATCHED], ok[RMX_MAX_BATCHED], groups[RMX_MAX_BATCHED], ntile[RMX_MAX_BATCHED];
+  int oq[RMX_MAX_BATCHED], ok[RMX_MAX_BATCHED], ntile[RMX_MAX_BATCHED];
   order_by_cost(nq, cq, oq);
   order_by_cost(nk, ck, ok);
   for (int i = 0; i < nq; ++i) {
     pq.P[i] = probs[iq[oq[i]]];
-    groups[i] = L.batch * L.hq;
     ntile[i] = (pq.P[i].sq + BQ_DQ - 1) / BQ_DQ;
   }
-  const int tq = plan_workgroups(pq.map, nq, groups, ntile);
+  const int tq = plan_workgroups(pq.map, nq, L.batch * L.hq, G, ntile, L.mask == RMX_MASK_CAUSAL);
   for (int i = 0; i < nk; ++i) {
     pk.P[i] = probs[ik[ok[i]]];
-    groups[i] = L.batch * L.hkv;
     ntile[i] = (pk.P[i].sk + BKV - 1) / BKV;
   }
-  const int tk = plan_workgroups(pk.map, nk, groups, ntile);
+  const int tk = plan_workgroups(pk.map, nk, L.batch * L.hkv, 1, ntile, L.mask == RMX_MASK_CAUSAL);
   if constexpr (HD == 256) {
     if (tk > 0) {
       const dim3 grid(tk);

@@ -659,15 +659,15 @@ static hipError_t launch_fwd_t(const rmx_attn_layout& L, const rmx_fwd_problem* 
   drop_params(L.dropout_p, &prm.drop_thr, &prm.drop_scale);
   // longest workgroups (most key tiles) first
   long long cost[RMX_MAX_BATCHED];
-  int order[RMX_MAX_BATCHED], groups[RMX_MAX_BATCHED], ntile[RMX_MAX_BATCHED];
+  int order[RMX_MAX_BATCHED], ntile[RMX_MAX_BATCHED];
   for (int i = 0; i < n; ++i) cost[i] = probs[i].sk;
   order_by_cost(n, cost, order);
   for (int i = 0; i < n; ++i) {
     prm.P[i] = probs[order[i]];
-    groups[i] = L.batch * L.hq;
     ntile[i] = (prm.P[i].sq + BQ - 1) / BQ;
   }
-  const int grid = plan_workgroups(prm.map, n, groups, ntile);
+  const int grid = plan_workgroups(prm.map, n, L.batch * L.hq, L.hq / L.hkv, ntile,
+                                   L.mask == RMX_MASK_CAUSAL);
   if (grid == 0) return hipSuccess;
   if (L.mask == RMX_MASK_CAUSAL)
     hipLaunchKernelGGL((attn_fwd_kernel<HD, RMX_MASK_CAUSAL, DT, DROP>), dim3(grid),
