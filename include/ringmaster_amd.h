@@ -42,7 +42,8 @@ extern "C" {
                                   dropout with document masks;
                               17: rmx_linear_scan_status;
                               18: right-bounded windows (problem window_right), and since,
-                                  as additions: rmx_mamba2_dt_cumsum_state_bwd */
+                                  as additions: rmx_mamba2_dt_cumsum_state_bwd,
+                                  rmx_attn_bwd_ws */
 
 /* error codes */
 #define RMX_OK 0
@@ -219,6 +220,20 @@ int32_t rmx_attn_bwd_delta(const rmx_attn_layout* layout, const void* out, int32
  */
 int32_t rmx_attn_bwd(const rmx_attn_layout* layout, const rmx_bwd_problem* problems,
                      int32_t nproblems, void* stream);
+
+/*
+ * The same with device memory for partial dK/dV sums: a call with few key blocks (or causal
+ * ones of very different lengths) then gives each several workgroups, whose fp32 partial
+ * gradients are summed in a fixed order before the mode is applied. rmx_attn_bwd_workspace
+ * returns the bytes the call can use (0: it runs as rmx_attn_bwd does, also for arguments
+ * rmx_attn_bwd refuses); the workspace (nullable, 16-byte aligned) is scratch of this call,
+ * its contents on entry do not matter, and one smaller than that is not used. No counterpart
+ * in the reference.
+ */
+size_t rmx_attn_bwd_workspace(const rmx_attn_layout* layout, const rmx_bwd_problem* problems,
+                              int32_t nproblems);
+int32_t rmx_attn_bwd_ws(const rmx_attn_layout* layout, const rmx_bwd_problem* problems,
+                        int32_t nproblems, void* workspace, size_t workspace_bytes, void* stream);
 
 /*
  * Standalone online-softmax merge, `update_out_and_lse` (ring/merge.py:20-31):

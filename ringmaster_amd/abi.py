@@ -96,6 +96,10 @@ SIGNATURES = {
     "rmx_attn_bwd_delta": (_i32, [ctypes.POINTER(AttnLayout), _vp, _i32, _vp, _vp, _vp, _vp, _i32,
                                   _vp]),
     "rmx_attn_bwd": (_i32, [ctypes.POINTER(AttnLayout), ctypes.POINTER(BwdProblem), _i32, _vp]),
+    "rmx_attn_bwd_workspace": (ctypes.c_size_t, [ctypes.POINTER(AttnLayout),
+                                                 ctypes.POINTER(BwdProblem), _i32]),
+    "rmx_attn_bwd_ws": (_i32, [ctypes.POINTER(AttnLayout), ctypes.POINTER(BwdProblem), _i32, _vp,
+                               ctypes.c_size_t, _vp]),
     "rmx_lse_merge": (_i32, [_vp, _vp, _vp, _i32, _vp, _i32, _i32, _i32, _i32,
                              ctypes.POINTER(_i64), ctypes.POINTER(_i64), ctypes.POINTER(_i64),
                              ctypes.POINTER(_i64), _i32, _vp]),

@@ -175,8 +175,8 @@ int32_t rmx_attn_bwd_delta(const rmx_attn_layout* layout, const void* out, int32
                     "rmx_attn_bwd_delta launch");
 }
 
-int32_t rmx_attn_bwd(const rmx_attn_layout* layout, const rmx_bwd_problem* problems,
-                     int32_t nproblems, void* stream) {
+static int check_attn_bwd(const rmx_attn_layout* layout, const rmx_bwd_problem* problems,
+                          int32_t nproblems) {
   int rc = check_layout(layout);
   if (rc) return rc;
   if (nproblems < 0 || (nproblems > 0 && !problems))
@@ -217,13 +217,42 @@ int32_t rmx_attn_bwd(const rmx_attn_layout* layout, const rmx_bwd_problem* probl
       }
     }
   }
+  return RMX_OK;
+}
+
+size_t rmx_attn_bwd_workspace(const rmx_attn_layout* layout, const rmx_bwd_problem* problems,
+                              int32_t nproblems) {
+  if (check_attn_bwd(layout, problems, nproblems)) return 0;
+  size_t bytes = 0;
   for (int i = 0; i < nproblems; i += RMX_MAX_BATCHED) {
-    const int n = nproblems - i < RMX_MAX_BATCHED ? nproblems - i : RMX_MAX_BATCHED;
-    rc = dev_status(rmx::launch_attn_bwd(*layout, problems + i, n, (hipStream_t)stream),
+    const int n = std::min(nproblems - i, RMX_MAX_BATCHED);
+    bytes = std::max(bytes, rmx::dkdv_split(*layout, problems + i, n).bytes());
+  }
+  return bytes;
+}
+
+int32_t rmx_attn_bwd_ws(const rmx_attn_layout* layout, const rmx_bwd_problem* problems,
+                        int32_t nproblems, void* workspace, size_t workspace_bytes, void* stream) {
+  int rc = check_attn_bwd(layout, problems, nproblems);
+  if (rc) return rc;
+  if (workspace && !aligned(workspace, 16))
+    return fail(RMX_EINVAL, "workspace must be 16-byte aligned");
+  for (int i = 0; i < nproblems; i += RMX_MAX_BATCHED) {
+    const int n = std::min(nproblems - i, RMX_MAX_BATCHED);
+    rmx::DkdvSplit split{1, 0, 0};
+    if (workspace) split = rmx::dkdv_split(*layout, problems + i, n);
+    if (split.bytes() > workspace_bytes) split = rmx::DkdvSplit{1, 0, 0};
+    rc = dev_status(rmx::launch_attn_bwd(*layout, problems + i, n, split, workspace,
+                                         (hipStream_t)stream),
                     "rmx_attn_bwd launch");
     if (rc) return rc;
   }
   return RMX_OK;
+}
+
+int32_t rmx_attn_bwd(const rmx_attn_layout* layout, const rmx_bwd_problem* problems,
+                     int32_t nproblems, void* stream) {
+  return rmx_attn_bwd_ws(layout, problems, nproblems, nullptr, 0, stream);
 }
 
 int32_t rmx_lse_merge(float* out, float* lse, const void* blk_out, int32_t blk_type,

@@ -121,40 +121,197 @@ hipError_t launch_attn_bwd_delta(const rmx_attn_layout& L, const void* out, int 
   return hipGetLastError();
 }
 
+// ---------------------------------------------------------------- dK/dV splits
+// Workgroups per key block of a dK/dV launch. The launch's time is estimated for every
+// number of splits from the tile counts of its key blocks (the masks' own ranges; documents
+// count as causal): a tile and a workgroup cost what the kernels measure on a lone CU,
+// workgroups run in rounds over the CUs, and a split launch adds the fold kernel and the
+// partial gradients' traffic. Launches of many rounds stay whole. Whole -> split, us a launch:
+// 4096^2 causal 32/8 heads of 128 403 -> 314 (2), 2048^2 189 -> 101 (3), 512^2 58 -> 34 (4);
+// 4096^2 causal 16/4 heads of 256 821 -> 343 (4), of 64 253 -> 102 (4); the same 4096^2 with
+// 32 KV heads fills the chip and would go from 321 to 419 in two.
+DkdvSplit dkdv_split(const rmx_attn_layout& L, const rmx_bwd_problem* probs, int n) {
+  constexpr int kCu = 256, kBkv = 128, kMaxSplit = 16;
+  DkdvSplit out{1, 0, 0};
+  const int hd = L.head_dim > 128 ? 256 : L.head_dim > 64 ? 128 : 64;
+  const int bq = hd == 256 ? 32 : 64, G = L.hq / L.hkv;
+  // us: per tile, per workgroup, of the fold launch
+  const double tile = hd == 256 ? 1.6 : hd == 128 ? 1.4 : 1.1, wg = hd == 256 ? 12. : hd == 128 ? 6. : 4.,
+               fold = 5.;
+  const int64_t per = (int64_t)L.batch * L.hkv;
+  int64_t blocks = 0, keys = 0;
+  int skmax = 0, np = 0;
+  for (int i = 0; i < n; ++i) {
+    const rmx_bwd_problem& p = probs[i];
+    if (p.sq == 0 || p.sk == 0 || p.dkv_mode == RMX_GRAD_NONE) continue;
+    blocks += per * ((p.sk + kBkv - 1) / kBkv);
+    keys += per * p.sk;
+    skmax = p.sk > skmax ? p.sk : skmax;
+    ++np;
+  }
+  if (blocks == 0 || blocks >= 4 * kCu) return out;
+  int64_t tiles = 0;  // of all blocks
+  int longest = 0;
+  for (int i = 0; i < n; ++i) {
+    const rmx_bwd_problem& p = probs[i];
+    if (p.sq == 0 || p.sk == 0 || p.dkv_mode == RMX_GRAD_NONE) continue;
+    const int64_t nqt = (p.sq + bq - 1) / bq, off = (int64_t)p.sk - p.sq + p.window_right;
+    for (int64_t k0 = 0; k0 < p.sk; k0 += kBkv) {
+      int64_t lo = 0, hi = nqt;
+      if (L.mask != RMX_MASK_FULL) {
+        lo = k0 - off <= 0 ? 0 : (k0 - off) / bq;
+        if (lo > nqt) lo = nqt;
+      }
+      if (p.has_window) {
+        const int64_t qmax = k0 + kBkv - 1 + (int64_t)p.window_left - ((int64_t)p.sk - p.sq);
+        hi = qmax < 0 ? 0 : (qmax / bq + 1 < nqt ? qmax / bq + 1 : nqt);
+      }
+      const int t = hi > lo ? (int)(hi - lo) * G : 0;
+      tiles += per * t;
+      longest = t > longest ? t : longest;
+    }
+  }
+  double best = 0;
+  for (int s = 1; s <= kMaxSplit && (s == 1 || s <= longest); ++s) {
+    const double one = wg + tile * ((longest + s - 1) / s);
+    const double share = (wg * blocks * s + tile * tiles) / kCu;  // an even share of the work
+    // even blocks run in whole rounds; uneven ones fill the CUs behind the longest
+    const bool even = tiles == blocks * (int64_t)longest;
+    double t = even ? one * ((blocks * s + kCu - 1) / kCu) : (share > one ? share : one) + 0.5 * tile;
+    if (s > 1) t += fold + 1e6 * (double)s * keys * L.head_dim * 8 * 2 / 4e12;
+    if (s == 1 || t < best) {
+      best = t;
+      out.n = s;
+    }
+  }
+  if (out.n > 1) {
+    out.prob = per * skmax * (int64_t)L.head_dim;
+    out.grad = out.prob * np;
+  }
+  return out;
+}
+
+struct FoldParams {
+  rmx_attn_layout L;
+  rmx_bwd_problem P[RMX_MAX_BATCHED];
+  const float* ws;
+  int nsplit, skmax;
+  int64_t prob, grad;
+};
+
+// Sum of the splits' partial dV (blockIdx.y even) and dK (odd) rows of one problem, stored in
+// its mode. Bound by its traffic (nsplit fp32 reads per element); a thread owns 4 columns of a
+// row, HD / 4 threads a row, the splits' loads four at a time in flight.
+template <int HD, int DT>
+__global__ __launch_bounds__(256) void dkdv_fold_kernel(const FoldParams prm) {
+  constexpr int CPR = HD / 4, RPB = 256 / CPR;
+  const rmx_attn_layout& L = prm.L;
+  const rmx_bwd_problem& P = prm.P[blockIdx.y >> 1];
+  const int g = blockIdx.y & 1, D = L.head_dim;
+  const int col = 4 * (threadIdx.x % CPR);
+  const int64_t row = (int64_t)blockIdx.x * RPB + threadIdx.x / CPR;  // (batch, kv head, key)
+  if (col >= D || row >= (int64_t)L.batch * L.hkv * P.sk) return;
+  const int bh = (int)(row / P.sk), key = (int)(row - (int64_t)bh * P.sk);
+  const int bb = bh / L.hkv, h = bh % L.hkv;
+  const float* src = prm.ws + (blockIdx.y >> 1) * prm.prob + g * prm.grad +
+                     ((int64_t)bh * prm.skmax + key) * D + col;
+  f32x4 v = *reinterpret_cast<const f32x4*>(src);
+#pragma unroll 4
+  for (int s = 1; s < prm.nsplit; ++s)
+    v += *reinterpret_cast<const f32x4*>(src + s * 2 * prm.grad);
+  const int mode = P.dkv_mode;
+  const bool rd = mode == RMX_GRAD_ACC_F32 || mode == RMX_GRAD_ACC_FINAL;
+  const bool w32 = mode == RMX_GRAD_WRITE_F32 || mode == RMX_GRAD_ACC_F32;
+  float* const acc = (g ? P.dk_acc : P.dv_acc) + bb * L.ka_sb + (int64_t)key * L.ka_ss + h * L.ka_sh + col;
+  uint16_t* const bf = (g ? P.dk : P.dv) + bb * L.dk_sb + (int64_t)key * L.dk_ss + h * L.dk_sh + col;
+  const bool vec = (!(rd || w32) || ((uintptr_t)acc & 15) == 0) && (w32 || ((uintptr_t)bf & 7) == 0);
+  if (vec) {
+    if (rd) v += *reinterpret_cast<const f32x4*>(acc);
+    if (w32) {
+      *reinterpret_cast<f32x4*>(acc) = v;
+    } else {
+      u32x2 w;
+      w[0] = cvt_pk<DT>(v[0], v[1]);
+      w[1] = cvt_pk<DT>(v[2], v[3]);
+      *reinterpret_cast<u32x2*>(bf) = w;
+    }
+    return;
+  }
+  for (int e = 0; e < 4; ++e) {  // a caller pointer below vector alignment
+    const float x = rd ? acc[e] + v[e] : v[e];
+    if (w32)
+      acc[e] = x;
+    else
+      bf[e] = f2e<DT>(x);
+  }
+}
+
+template <int HD>
+static void launch_fold_t(const FoldParams& prm, int n, int64_t rows, bool f16, hipStream_t stream) {
+  constexpr int RPB = 256 / (HD / 4);
+  const dim3 grid((unsigned)((rows + RPB - 1) / RPB), 2 * n);
+  if (f16)
+    hipLaunchKernelGGL((dkdv_fold_kernel<HD, RMX_DTYPE_F16>), grid, dim3(256), 0, stream, prm);
+  else
+    hipLaunchKernelGGL((dkdv_fold_kernel<HD, RMX_DTYPE_BF16>), grid, dim3(256), 0, stream, prm);
+}
+
+hipError_t launch_dkdv_fold(const rmx_attn_layout& L, const rmx_bwd_problem* probs, int n,
+                            const DkdvSplit& split, const void* ws, hipStream_t stream) {
+  FoldParams prm;
+  prm.L = L;
+  for (int i = 0; i < n; ++i) prm.P[i] = probs[i];
+  prm.ws = static_cast<const float*>(ws);
+  prm.nsplit = split.n;
+  const int64_t per = (int64_t)L.batch * L.hkv;
+  prm.skmax = (int)(split.prob / (per * L.head_dim));
+  prm.prob = split.prob;
+  prm.grad = split.grad;
+  const int64_t rows = per * prm.skmax;
+  const bool f16 = L.dtype == RMX_DTYPE_F16;
+  if (L.head_dim > 128)
+    launch_fold_t<256>(prm, n, rows, f16, stream);
+  else if (L.head_dim > 64)
+    launch_fold_t<128>(prm, n, rows, f16, stream);
+  else
+    launch_fold_t<64>(prm, n, rows, f16, stream);
+  return hipGetLastError();
+}
+
 // the head-dim-64 and -128 launches are instantiated in attn_bwd_vf.hip
 extern template hipError_t launch_bwd_t<64, RMX_DTYPE_BF16, false>(const rmx_attn_layout&,
-    const rmx_bwd_problem*, int, hipStream_t);
+    const rmx_bwd_problem*, int, const DkdvSplit&, void*, hipStream_t);
 extern template hipError_t launch_bwd_t<64, RMX_DTYPE_BF16, true>(const rmx_attn_layout&,
-    const rmx_bwd_problem*, int, hipStream_t);
+    const rmx_bwd_problem*, int, const DkdvSplit&, void*, hipStream_t);
 extern template hipError_t launch_bwd_t<64, RMX_DTYPE_F16, false>(const rmx_attn_layout&,
-    const rmx_bwd_problem*, int, hipStream_t);
+    const rmx_bwd_problem*, int, const DkdvSplit&, void*, hipStream_t);
 extern template hipError_t launch_bwd_t<64, RMX_DTYPE_F16, true>(const rmx_attn_layout&,
-    const rmx_bwd_problem*, int, hipStream_t);
+    const rmx_bwd_problem*, int, const DkdvSplit&, void*, hipStream_t);
 extern template hipError_t launch_bwd_t<128, RMX_DTYPE_BF16, false>(const rmx_attn_layout&,
-    const rmx_bwd_problem*, int, hipStream_t);
+    const rmx_bwd_problem*, int, const DkdvSplit&, void*, hipStream_t);
 extern template hipError_t launch_bwd_t<128, RMX_DTYPE_BF16, true>(const rmx_attn_layout&,
-    const rmx_bwd_problem*, int, hipStream_t);
+    const rmx_bwd_problem*, int, const DkdvSplit&, void*, hipStream_t);
 extern template hipError_t launch_bwd_t<128, RMX_DTYPE_F16, false>(const rmx_attn_layout&,
-    const rmx_bwd_problem*, int, hipStream_t);
+    const rmx_bwd_problem*, int, const DkdvSplit&, void*, hipStream_t);
 extern template hipError_t launch_bwd_t<128, RMX_DTYPE_F16, true>(const rmx_attn_layout&,
-    const rmx_bwd_problem*, int, hipStream_t);
+    const rmx_bwd_problem*, int, const DkdvSplit&, void*, hipStream_t);
 
 template <int DT, bool DROP>
 static hipError_t launch_bwd_hd(const rmx_attn_layout& L, const rmx_bwd_problem* probs, int n,
-                                hipStream_t stream) {
-  if (L.head_dim > 128) return launch_bwd_t<256, DT, DROP>(L, probs, n, stream);
-  if (L.head_dim > 64) return launch_bwd_t<128, DT, DROP>(L, probs, n, stream);
-  return launch_bwd_t<64, DT, DROP>(L, probs, n, stream);
+                                const DkdvSplit& split, void* ws, hipStream_t stream) {
+  if (L.head_dim > 128) return launch_bwd_t<256, DT, DROP>(L, probs, n, split, ws, stream);
+  if (L.head_dim > 64) return launch_bwd_t<128, DT, DROP>(L, probs, n, split, ws, stream);
+  return launch_bwd_t<64, DT, DROP>(L, probs, n, split, ws, stream);
 }
 
 hipError_t launch_attn_bwd(const rmx_attn_layout& L, const rmx_bwd_problem* probs, int n,
-                           hipStream_t stream) {
+                           const DkdvSplit& split, void* ws, hipStream_t stream) {
   const bool f16 = L.dtype == RMX_DTYPE_F16, drop = L.dropout_p > 0.f;
   if (drop)
-    return f16 ? launch_bwd_hd<RMX_DTYPE_F16, true>(L, probs, n, stream)
-               : launch_bwd_hd<RMX_DTYPE_BF16, true>(L, probs, n, stream);
-  return f16 ? launch_bwd_hd<RMX_DTYPE_F16, false>(L, probs, n, stream)
-             : launch_bwd_hd<RMX_DTYPE_BF16, false>(L, probs, n, stream);
+    return f16 ? launch_bwd_hd<RMX_DTYPE_F16, true>(L, probs, n, split, ws, stream)
+               : launch_bwd_hd<RMX_DTYPE_BF16, true>(L, probs, n, split, ws, stream);
+  return f16 ? launch_bwd_hd<RMX_DTYPE_F16, false>(L, probs, n, split, ws, stream)
+             : launch_bwd_hd<RMX_DTYPE_BF16, false>(L, probs, n, split, ws, stream);
 }
 
 }  // namespace rmx

@@ -36,6 +36,10 @@ struct BwdParams {
   float scale_log2;
   uint32_t drop_thr;  // dropout: keep when the element's hash >= drop_thr
   float drop_scale;   // 1 / (1 - p)
+  // dK/dV: workgroups per key block (see the split notes at the dK/dV kernel) and the elements
+  // between the partial gradients of two splits
+  int nsplit;
+  int64_t split_stride;
 };
 
 // ---------------------------------------------------------------- shared helpers
@@ -53,6 +57,11 @@ __device__ __forceinline__ void grad_store4(int mode, float* acc, uint16_t* bf, 
     w[1] = cvt_pk<DT>(v[2], v[3]);
     *reinterpret_cast<u32x2*>(bf) = w;
   }
+}
+
+// first of n items of share i of s
+__device__ __forceinline__ int split_lo(int n, int i, int s) {
+  return s == 1 ? (i ? n : 0) : (int)((int64_t)n * i / s);
 }
 
 // ---------------------------------------------------------------- tiles
@@ -558,6 +567,12 @@ __global__ __launch_bounds__(DqCfg<HD>::NT, 1) void attn_bwd_dq_kernel(const Bwd
 // get S := -inf on their masked pairs before their exponentials, with nl clamped
 // to a finite value so that a row with lse = -inf (it attends nothing) gives 0,
 // not NaN.
+// A key block's tiles are the queries of every q head of its group: with few key blocks,
+// or causal ones (the first block walks every query, the last one tile), that leaves CUs
+// idle behind long workgroups. The launcher then gives each block nsplit workgroups with
+// equal shares of its tiles. They write fp32 partial gradients to the caller's workspace,
+// which dkdv_fold_kernel adds in split order (deterministic) and stores in the call's mode
+// (the rule and its measurements: dkdv_split in attn_bwd.hip).
 // Q/dO tiles (with lse, delta) arrive by LDS DMA into four buffers; a tile is
 // issued three barriers before it is read. Tiles past the end are issued as
 // zero-length loads (they write zeros to a free buffer and touch no memory),
@@ -610,7 +625,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_kernel(const BwdParams p
   const int G = L.hq / L.hkv;
   const int sq = P.sq, sk = P.sk;
   constexpr int mask = MASK;
-  const int k0 = wc.tile * C::BKV;
+  const int split = wc.tile % prm.nsplit, k0 = wc.tile / prm.nsplit * C::BKV;
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (SGPR)
@@ -663,7 +678,10 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_kernel(const BwdParams p
     qt_end = sRange[1] + 1;
     if (qt_end < qt_begin) qt_end = qt_begin;
   }
-  const int ntile = (qt_end - qt_begin) * G;  // (q head, query tile) pairs, q head major
+  // (q head, query tile) pairs, q head major: this split's share [t_lo, t_lo + ntile)
+  const int nqr = qt_end - qt_begin;
+  const int t_lo = split_lo(nqr * G, split, prm.nsplit);
+  const int ntile = split_lo(nqr * G, split + 1, prm.nsplit) - t_lo;
   // no query tile: accumulated dK and dV keep their values
   if (ntile == 0 && P.dkv_mode == RMX_GRAD_ACC_F32) return;
   const int wave_klast = (kw0 + 31 < sk ? kw0 + 31 : sk - 1);
@@ -912,7 +930,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_kernel(const BwdParams p
   };
 
   // ---- prologue: tiles 0, 1 and 2 issued, documents of tile 0 in LDS
-  Cursor cur = {qt_begin, 0};
+  Cursor cur = {qt_begin + (nqr > 0 ? t_lo % nqr : 0), nqr > 0 ? t_lo / nqr : 0};
   Cursor nx1 = advance(cur), nx2 = advance(nx1), nx3 = advance(nx2);
   dma_tile(0, cur, ntile > 0);
   dma_tile(1, nx1, ntile > 1);
@@ -1245,7 +1263,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_kernel(const BwdParams p
 #pragma unroll 1
   for (int g = 0; g < 2; ++g) {
     const float* const stg = reinterpret_cast<const float*>(g == 0 ? &sQ[0][0] : &sO[0][0]) + 32 * wave * HD;
-    float* const gacc = (g == 0 ? E.dv_acc : E.dk_acc) + bb * L.ka_sb + kvh * L.ka_sh + 4 * ch;
+    float* const gacc = (g == 0 ? E.dv_acc : E.dk_acc) + split * prm.split_stride + bb * L.ka_sb + kvh * L.ka_sh + 4 * ch;
     uint16_t* const gbf = (g == 0 ? E.dv : E.dk) + bb * L.dk_sb + kvh * L.dk_sh + 4 * ch;
     if (!ELEMS && !vec) {
 #pragma unroll 1
@@ -1353,7 +1371,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_d256_kernel(const BwdPar
   const int G = L.hq / L.hkv;
   const int sq = P.sq, sk = P.sk;
   constexpr int mask = MASK;
-  const int k0 = wc.tile * BKV;
+  const int split = wc.tile % prm.nsplit, k0 = wc.tile / prm.nsplit * BKV;
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (SGPR)
@@ -1406,7 +1424,10 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_d256_kernel(const BwdPar
     qt_end = sRange[1] + 1;
     if (qt_end < qt_begin) qt_end = qt_begin;
   }
-  const int ntile = (qt_end - qt_begin) * G;  // (q head, query tile) pairs, q head major
+  // (q head, query tile) pairs, q head major: this split's share [t_lo, t_lo + ntile)
+  const int nqr = qt_end - qt_begin;
+  const int t_lo = split_lo(nqr * G, split, prm.nsplit);
+  const int ntile = split_lo(nqr * G, split + 1, prm.nsplit) - t_lo;
   // no query tile: accumulated dK and dV keep their values
   if (ntile == 0 && P.dkv_mode == RMX_GRAD_ACC_F32) return;
   const int wave_klast = (kw0 + 31 < sk ? kw0 + 31 : sk - 1);
@@ -1645,7 +1666,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_d256_kernel(const BwdPar
   };
 
   // ---- prologue: the K block, tiles 0 and 1 issued; tile 0's documents in LDS
-  Cursor cur = {qt_begin, 0};
+  Cursor cur = {qt_begin + (nqr > 0 ? t_lo % nqr : 0), nqr > 0 ? t_lo / nqr : 0};
   Cursor nx1 = advance(cur), nx2 = advance(nx1);
   if (ntile > 0) dma_tile(0, 0, cur);
   if (ntile > 1) dma_tile(1, 1, nx1);
@@ -1887,13 +1908,14 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_d256_kernel(const BwdPar
       }
     }
   };
-  store(dv, 1.f, P.dv_acc, P.dv);
-  store(dk, -L.scale, P.dk_acc, P.dk);
+  const int64_t so = split * prm.split_stride;
+  store(dv, 1.f, P.dv_acc ? P.dv_acc + so : nullptr, P.dv);
+  store(dk, -L.scale, P.dk_acc ? P.dk_acc + so : nullptr, P.dk);
 }
 
 template <int HD, int DT, bool DROP>
 hipError_t launch_bwd_t(const rmx_attn_layout& L, const rmx_bwd_problem* probs, int n,
-                        hipStream_t stream) {
+                        const DkdvSplit& split, void* ws, hipStream_t stream) {
   constexpr int BQ_DQ = DqCfg<HD>::BQ, BKV = HD == 256 ? 128 : DkdvCfg<HD>::BKV;
   BwdParams pq, pk;
   pq.L = L;
@@ -1926,9 +1948,26 @@ hipError_t launch_bwd_t(const rmx_attn_layout& L, const rmx_bwd_problem* probs, 
     ntile[i] = (pq.P[i].sq + BQ_DQ - 1) / BQ_DQ;
   }
   const int tq = plan_workgroups(pq.map, nq, L.batch * L.hq, G, ntile, L.mask == RMX_MASK_CAUSAL);
+  pq.nsplit = 1;
+  pq.split_stride = 0;
+  pk.nsplit = split.n;
+  pk.split_stride = split.n > 1 ? 2 * split.grad : 0;
   for (int i = 0; i < nk; ++i) {
     pk.P[i] = probs[ik[ok[i]]];
-    ntile[i] = (pk.P[i].sk + BKV - 1) / BKV;
+    ntile[i] = (pk.P[i].sk + BKV - 1) / BKV * split.n;
+  }
+  rmx_bwd_problem fold[RMX_MAX_BATCHED];
+  if (split.n > 1) {  // the kernels write partial gradients, the fold kernel the call's outputs
+    for (int i = 0; i < nk; ++i) {
+      fold[i] = pk.P[i];
+      pk.P[i].dkv_mode = RMX_GRAD_WRITE_F32;
+      pk.P[i].dv_acc = static_cast<float*>(ws) + i * split.prob;
+      pk.P[i].dk_acc = pk.P[i].dv_acc + split.grad;
+      pk.P[i].dv = pk.P[i].dk = nullptr;
+    }
+    pk.L.ka_ss = L.head_dim;
+    pk.L.ka_sh = split.prob / ((int64_t)L.batch * L.hkv);
+    pk.L.ka_sb = pk.L.ka_sh * L.hkv;
   }
   const int tk = plan_workgroups(pk.map, nk, L.batch * L.hkv, 1, ntile, L.mask == RMX_MASK_CAUSAL);
   if constexpr (HD == 256) {
@@ -1955,6 +1994,10 @@ hipError_t launch_bwd_t(const rmx_attn_layout& L, const rmx_bwd_problem* probs, 
       hipError_t e = hipGetLastError();
       if (e != hipSuccess) return e;
     }
+  }
+  if (tk > 0 && split.n > 1) {
+    const hipError_t e = launch_dkdv_fold(L, fold, nk, split, ws, stream);
+    if (e != hipSuccess) return e;
   }
   if (tq > 0) {
     const dim3 grid(tq);

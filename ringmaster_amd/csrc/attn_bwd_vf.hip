@@ -7,20 +7,20 @@
 namespace rmx {
 
 template hipError_t launch_bwd_t<64, RMX_DTYPE_BF16, false>(const rmx_attn_layout&,
-    const rmx_bwd_problem*, int, hipStream_t);
+    const rmx_bwd_problem*, int, const DkdvSplit&, void*, hipStream_t);
 template hipError_t launch_bwd_t<64, RMX_DTYPE_BF16, true>(const rmx_attn_layout&,
-    const rmx_bwd_problem*, int, hipStream_t);
+    const rmx_bwd_problem*, int, const DkdvSplit&, void*, hipStream_t);
 template hipError_t launch_bwd_t<64, RMX_DTYPE_F16, false>(const rmx_attn_layout&,
-    const rmx_bwd_problem*, int, hipStream_t);
+    const rmx_bwd_problem*, int, const DkdvSplit&, void*, hipStream_t);
 template hipError_t launch_bwd_t<64, RMX_DTYPE_F16, true>(const rmx_attn_layout&,
-    const rmx_bwd_problem*, int, hipStream_t);
+    const rmx_bwd_problem*, int, const DkdvSplit&, void*, hipStream_t);
 template hipError_t launch_bwd_t<128, RMX_DTYPE_BF16, false>(const rmx_attn_layout&,
-    const rmx_bwd_problem*, int, hipStream_t);
+    const rmx_bwd_problem*, int, const DkdvSplit&, void*, hipStream_t);
 template hipError_t launch_bwd_t<128, RMX_DTYPE_BF16, true>(const rmx_attn_layout&,
-    const rmx_bwd_problem*, int, hipStream_t);
+    const rmx_bwd_problem*, int, const DkdvSplit&, void*, hipStream_t);
 template hipError_t launch_bwd_t<128, RMX_DTYPE_F16, false>(const rmx_attn_layout&,
-    const rmx_bwd_problem*, int, hipStream_t);
+    const rmx_bwd_problem*, int, const DkdvSplit&, void*, hipStream_t);
 template hipError_t launch_bwd_t<128, RMX_DTYPE_F16, true>(const rmx_attn_layout&,
-    const rmx_bwd_problem*, int, hipStream_t);
+    const rmx_bwd_problem*, int, const DkdvSplit&, void*, hipStream_t);
 
 }  // namespace rmx

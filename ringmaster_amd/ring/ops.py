@@ -272,4 +272,9 @@ def attn_bwd(jobs: list[BwdJob], *, scale: float, mask: int, dropout=None) -> No
         p.sq, p.sk = j.q.shape[1], j.k.shape[1]
         p.dq_mode, p.dkv_mode = j.dq_mode, j.dkv_mode
         _set_problem_extras(p, j)
-    abi.check(abi.lib().rmx_attn_bwd(ctypes.byref(lay), arr, len(jobs), abi.stream_of(q0)))
+    lib = abi.lib()
+    # partial dK/dV sums of calls with few or uneven key blocks (0 bytes: none)
+    nbytes = lib.rmx_attn_bwd_workspace(ctypes.byref(lay), arr, len(jobs))
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=q0.device) if nbytes else None
+    abi.check(lib.rmx_attn_bwd_ws(ctypes.byref(lay), arr, len(jobs), abi.ptr(ws), nbytes,
+                                  abi.stream_of(q0)))

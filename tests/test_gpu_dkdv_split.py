@@ -1,0 +1,107 @@
+"""dK/dV with split key blocks (rmx_attn_bwd_ws) against the whole ones (rmx_attn_bwd)."""
+import ctypes
+
+import pytest
+import torch
+
+from tests.gpu_util import bf16_pair, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+# b, sq, sk, hq, hkv, d, mask, extras; each is a shape the rule splits
+CASES = [
+    (1, 512, 512, 8, 2, 128, "causal", {}),
+    (2, 200, 333, 8, 1, 64, "full", {}),
+    (1, 700, 300, 4, 1, 96, "full", {}),                       # sq > sk, padded head dim
+    (1, 300, 700, 8, 2, 128, "causal", dict(window=90)),
+    (1, 257, 257, 8, 2, 256, "causal", {}),
+    (2, 320, 129, 8, 2, 200, "full", dict(drop=(0.3, 5))),
+    (1, 640, 640, 8, 1, 64, "doc", {}),
+    (1, 600, 600, 16, 1, 128, "causal", dict(drop=(0.1, 9), f16=True)),
+]
+
+
+@pytest.mark.parametrize("b,sq,sk,hq,hkv,d,kind,x", CASES)
+@pytest.mark.parametrize("off", [0, 1])
+def test_split_equals_whole(b, sq, sk, hq, hkv, d, kind, x, off):
+    """Two problems of one call (the second with half the keys), every mode; ``off`` = 1 puts
+    the outputs one element past vector alignment. The splits only change the order of fp32
+    sums (rel-L2 a few 2^-24, held to 1e-6); 16-bit results may differ by one rounding of it."""
+    from ringmaster_amd import abi
+    from ringmaster_amd.ring import ops
+    from ringmaster_amd.ring.kernels import block_forward
+
+    print(f"case split b={b} {sq}x{sk} h={hq}/{hkv} d={d} {kind} {x} off={off}", flush=True)
+    h16 = torch.float16 if x.get("f16") else torch.bfloat16
+    q, k, v, do = (bf16_pair((b, n, h, d), s)[1].to(h16)
+                   for n, h, s in ((sq, hq, 1), (sk, hkv, 2), (sk, hkv, 3), (sq, hq, 4)))
+    sc, drop = d ** -0.5, x.get("drop")
+    mask = {"causal": abi.MASK_CAUSAL, "doc": abi.MASK_DOC}.get(kind, abi.MASK_FULL)
+    _, lse, out32 = block_forward(q, k, v, sc, kind == "causal", keep_f32=True, dropout=drop,
+                                  window=x.get("window"))
+    delta = torch.empty((b, hq, sq), device="cuda")
+    nlse = torch.empty_like(delta)
+    ops.attn_bwd_delta(out32, do, delta, hkv, lse=lse, nlse=nlse)
+    meta = [{}, {}]
+    sk2 = sk // 2
+    if kind == "doc":
+        ar = torch.arange(sq, dtype=torch.int32, device="cuda")
+        meta = [dict(q_gidx=ar, k_gidx=ar[:n], q_doc=ar // 250, k_doc=ar[:n] // 250)
+                for n in (sk, sk2)]
+
+    lib = abi.lib()
+
+    def run(mode, split):
+        acc = [torch.empty(b * sk * hkv * d + 8, device="cuda") for _ in range(4)]
+        half = [torch.zeros(b * sk * hkv * d + 8, dtype=h16, device="cuda") for _ in range(4)]
+        for i, t in enumerate(acc):
+            t[:] = torch.linspace(-1, 1 + i, t.numel(), device="cuda")
+        jobs, outs = [], []
+        for i, n in enumerate((sk, sk2)):
+            view = lambda t: t[off:off + b * sk * hkv * d].view(b, sk, hkv, d)[:, :n]  # noqa: E731
+            g = dict(dk_acc=view(acc[2 * i]), dv_acc=view(acc[2 * i + 1]),
+                     dk=view(half[2 * i]), dv=view(half[2 * i + 1]))
+            jobs.append(ops.BwdJob(q=q, k=k[:, :n], v=v[:, :n], dout=do, lse=lse, delta=delta,
+                                   nlse=nlse, dq_mode=abi.GRAD_NONE, dkv_mode=mode,
+                                   window=x.get("window"), **g, **meta[i]))
+            outs += [g["dk"], g["dv"]] if mode in (abi.GRAD_WRITE_BF16, abi.GRAD_ACC_FINAL) \
+                else [g["dk_acc"], g["dv_acc"]]
+        seen = []
+        real = lib.rmx_attn_bwd_workspace
+
+        class Spy:
+            def __getattr__(self, name):
+                if name == "rmx_attn_bwd_workspace":
+                    def size(*a):
+                        n = real(*a)
+                        seen.append(n)
+                        return n if split else 0
+                    return size
+                return getattr(lib, name)
+
+        keep, abi.lib = abi.lib, lambda: Spy()
+        try:
+            ops.attn_bwd(jobs, scale=sc, mask=mask, dropout=drop)
+        finally:
+            abi.lib = keep
+        torch.cuda.synchronize()
+        assert seen[0] > 0, "the rule does not split this shape"
+        return [o.float().clone() for o in outs]
+
+    for mode in (abi.GRAD_WRITE_F32, abi.GRAD_ACC_F32, abi.GRAD_WRITE_BF16, abi.GRAD_ACC_FINAL):
+        whole, split = run(mode, False), run(mode, True)
+        bar = 1e-6 if mode in (abi.GRAD_WRITE_F32, abi.GRAD_ACC_F32) else 1e-3
+        for a, c in zip(whole, split):
+            assert a.abs().sum() > 0 and rel_l2(c.cpu(), a.cpu()) < bar
+
+
+def test_refused_arguments_and_small_workspaces():
+    """The workspace query of a refused call is 0 and the call itself still refuses."""
+    from ringmaster_amd import abi
+
+    lib = abi.lib()
+    lay = abi.AttnLayout()
+    lay.batch, lay.hq, lay.hkv, lay.head_dim, lay.scale = 1, 3, 2, 64, 1.0
+    arr = (abi.BwdProblem * 1)()
+    assert lib.rmx_attn_bwd_workspace(ctypes.byref(lay), arr, 1) == 0
+    assert lib.rmx_attn_bwd_ws(ctypes.byref(lay), arr, 1, None, 0, None) == abi.RMX_EINVAL
