@@ -140,6 +140,13 @@ def _mask_of(causal: bool, right):
     return abi.MASK_CAUSAL, min(int(right), 1 << 28)  # sk < 2^27: past that, unbounded
 
 
+def _drop_of(dropout):
+    """(p, 64-bit seed) of a block's dropout argument (None: no dropout)."""
+    if dropout is None or not dropout[0]:
+        return 0.0, 0
+    return float(dropout[0]), int(dropout[1]) & _M64
+
+
 def block_forward(q, k, v, scale: float, causal: bool, keep_f32: bool = False, window=None,
                   dropout=None, right=None):
     """(out [b, sq, hq, d] in q's dtype, lse fp32 [b, hq, sq]) of one block; with ``keep_f32`` also
@@ -151,9 +158,13 @@ def block_forward(q, k, v, scale: float, causal: bool, keep_f32: bool = False, w
     lse = torch.empty((b, hq, sq), dtype=torch.float32, device=q.device)
     out32 = torch.empty((b, sq, hq, d), dtype=torch.float32, device=q.device) if keep_f32 else None
     mask, shift = _mask_of(causal, right)
-    ops.attn_fwd([ops.FwdJob(q=q, k=k, v=v, mode=abi.FWD_WRITE, out=out, lse=lse,
-                             acc_out=out32, window=window, right=shift)],
-                 scale=scale, mask=mask, dropout=dropout)
+    p, seed = _drop_of(dropout)
+    bases = dict(q=q, k=k, v=v, out=out, lse=lse, acc_out=out32)
+    plan = ops.plan(
+        ("block_fwd", mask, shift, window, scale, p, keep_f32, ops.signature(q, k, v)),
+        lambda: ops.LaunchPlan([([ops.FwdJob(mode=abi.FWD_WRITE, window=window, right=shift,
+                                             **bases)], scale, mask)], bases, p))
+    plan.run_fwd(bases, seed, q, ops.NO_SPAN)
     return (out, lse, out32) if keep_f32 else (out, lse)
 
 
@@ -177,10 +188,15 @@ def block_backward(dout, q, k, v, out, lse, scale: float, causal: bool, dq=None,
         k.shape, dtype=k.dtype, device=k.device)
     dv_t = dv if (dv is not None and dv.stride() == dk_t.stride()) else torch.empty_like(dk_t)
     mask, shift = _mask_of(causal, right)
-    ops.attn_bwd([ops.BwdJob(q=q, k=k, v=v, dout=dout, lse=lse, delta=delta, nlse=nlse,
-                             dq_mode=abi.GRAD_WRITE_BF16, dkv_mode=abi.GRAD_WRITE_BF16,
-                             dq=dq_t, dk=dk_t, dv=dv_t, window=window, right=shift)],
-                 scale=scale, mask=mask, dropout=dropout)
+    p, seed = _drop_of(dropout)
+    bases = dict(q=q, k=k, v=v, dout=dout, lse=lse, delta=delta, nlse=nlse, dq=dq_t, dk=dk_t, dv=dv_t)
+    plan = ops.plan(
+        ("block_bwd", mask, shift, window, scale, p,
+         ops.signature(q, k, v, dout, lse, dq_t, dk_t, dv_t)),
+        lambda: ops.LaunchPlan([([ops.BwdJob(dq_mode=abi.GRAD_WRITE_BF16,
+                                             dkv_mode=abi.GRAD_WRITE_BF16, window=window,
+                                             right=shift, **bases)], scale, mask)], bases, p))
+    plan.run_bwd(bases, seed, q)
     for dst, src in ((dq, dq_t), (dk, dk_t), (dv, dv_t)):
         if dst is not None and dst is not src:
             dst.copy_(src)

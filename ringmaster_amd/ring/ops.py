@@ -10,9 +10,12 @@ and are launched together (up to 16 per kernel launch).
 
 from __future__ import annotations
 
+import collections
 import ctypes
 import dataclasses
+import threading
 
+import numpy as np
 import torch
 
 from ringmaster_amd import abi
@@ -195,11 +198,8 @@ def _set_meta_stride(lay, jobs, batch):
     lay.m_sb = int(strides.pop()) if strides else 0
 
 
-def attn_fwd(jobs: list[FwdJob], *, scale: float, mask: int, dropout=None) -> None:
-    """Launch the batched block forward (rmx_attn_fwd) for ``jobs``; ``dropout`` is None or
-    (p, seed)."""
-    if not jobs:
-        return
+def _pack_fwd(jobs, scale, mask, dropout):
+    """The (layout, problem array) of one rmx_attn_fwd call."""
     q0, k0 = jobs[0].q, jobs[0].k
     batch, hq, d, hkv = q0.shape[0], q0.shape[2], q0.shape[3], k0.shape[2]
     for j in jobs:
@@ -217,7 +217,16 @@ def attn_fwd(jobs: list[FwdJob], *, scale: float, mask: int, dropout=None) -> No
         p.q_doc, p.k_doc = _int32(j.q_doc), _int32(j.k_doc)
         p.sq, p.sk, p.mode = j.q.shape[1], j.k.shape[1], j.mode
         _set_problem_extras(p, j)
-    abi.check(abi.lib().rmx_attn_fwd(ctypes.byref(lay), arr, len(jobs), abi.stream_of(q0)))
+    return lay, arr
+
+
+def attn_fwd(jobs: list[FwdJob], *, scale: float, mask: int, dropout=None) -> None:
+    """Launch the batched block forward (rmx_attn_fwd) for ``jobs``; ``dropout`` is None or
+    (p, seed)."""
+    if not jobs:
+        return
+    lay, arr = _pack_fwd(jobs, scale, mask, dropout)
+    abi.check(abi.lib().rmx_attn_fwd(ctypes.byref(lay), arr, len(jobs), abi.stream_of(jobs[0].q)))
 
 
 def attn_bwd_delta(out: torch.Tensor, dout: torch.Tensor, delta: torch.Tensor, hkv: int,
@@ -234,24 +243,25 @@ def attn_bwd_delta(out: torch.Tensor, dout: torch.Tensor, delta: torch.Tensor, h
         raise ValueError("a 16-bit out must share dout's type and strides")
     if (nlse is None) != (lse is None):
         raise ValueError("lse and nlse go together")
-    job = FwdJob(q=dout, k=dout[:, :0, :hkv], v=dout[:, :0, :hkv], out=dout, lse=delta,
-                 acc_out=out if f32 else None)
-    jobs = [job]
-    if nlse is not None:
-        if lse.shape != delta.shape or nlse.shape != delta.shape:
-            raise ValueError("lse, delta and nlse must share their shape")
-        jobs += [FwdJob(q=dout, k=job.k, v=job.v, lse=lse), FwdJob(q=dout, k=job.k, v=job.v, lse=nlse)]
-    lay = _fill_layout(jobs, batch, hq, hkv, d, 1.0, abi.MASK_FULL)
+    if nlse is not None and (lse.shape != delta.shape or nlse.shape != delta.shape):
+        raise ValueError("lse, delta and nlse must share their shape")
+
+    def layout():
+        job = FwdJob(q=dout, k=dout[:, :0, :hkv], v=dout[:, :0, :hkv], out=dout, lse=delta,
+                     acc_out=out if f32 else None)
+        jobs = [job]
+        if nlse is not None:
+            jobs += [FwdJob(q=dout, k=job.k, v=job.v, lse=lse), FwdJob(q=dout, k=job.k, v=job.v, lse=nlse)]
+        return _fill_layout(jobs, batch, hq, hkv, d, 1.0, abi.MASK_FULL)
+
+    lay = plan(("delta", hkv, signature(out, dout, delta, lse, nlse)), layout)
     abi.check(abi.lib().rmx_attn_bwd_delta(ctypes.byref(lay), out.data_ptr(), int(f32),
                                            dout.data_ptr(), delta.data_ptr(), abi.ptr(lse),
                                            abi.ptr(nlse), sq, abi.stream_of(dout)))
 
 
-def attn_bwd(jobs: list[BwdJob], *, scale: float, mask: int, dropout=None) -> None:
-    """Launch the batched block backward (rmx_attn_bwd) for ``jobs``; ``dropout`` must be the
-    forward's (p, seed) and each job the forward's dropout offsets."""
-    if not jobs:
-        return
+def _pack_bwd(jobs, scale, mask, dropout):
+    """The (layout, problem array) of one rmx_attn_bwd call."""
     q0, k0 = jobs[0].q, jobs[0].k
     batch, hq, d, hkv = q0.shape[0], q0.shape[2], q0.shape[3], k0.shape[2]
     for j in jobs:
@@ -272,9 +282,157 @@ def attn_bwd(jobs: list[BwdJob], *, scale: float, mask: int, dropout=None) -> No
         p.sq, p.sk = j.q.shape[1], j.k.shape[1]
         p.dq_mode, p.dkv_mode = j.dq_mode, j.dkv_mode
         _set_problem_extras(p, j)
+    return lay, arr
+
+
+def attn_bwd(jobs: list[BwdJob], *, scale: float, mask: int, dropout=None) -> None:
+    """Launch the batched block backward (rmx_attn_bwd) for ``jobs``; ``dropout`` must be the
+    forward's (p, seed) and each job the forward's dropout offsets."""
+    if not jobs:
+        return
+    lay, arr = _pack_bwd(jobs, scale, mask, dropout)
     lib = abi.lib()
     # partial dK/dV sums of calls with few or uneven key blocks (0 bytes: none)
     nbytes = lib.rmx_attn_bwd_workspace(ctypes.byref(lay), arr, len(jobs))
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=q0.device) if nbytes else None
-    abi.check(lib.rmx_attn_bwd_ws(ctypes.byref(lay), arr, len(jobs), abi.ptr(ws), nbytes,
-                                  abi.stream_of(q0)))
+    _launch_bwd(lib, lay, arr, len(jobs), nbytes, jobs[0].q)
+
+
+def _launch_bwd(lib, lay, problems, n, nbytes, like):
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=like.device) if nbytes else None
+    abi.check(lib.rmx_attn_bwd_ws(ctypes.byref(lay), problems, n, abi.ptr(ws), nbytes,
+                                  abi.stream_of(like)))
+
+
+# ---------------------------------------------------------------- launch plans
+# Building a call's jobs (views, checks, strides) takes 20-40 us of host time per job, more
+# than a small ring step's kernels. A plan keeps what those jobs come to for one signature of
+# shapes, strides, types and options: the layouts, and the problem tables with every pointer as
+# an offset from its base tensor. A later call of the same signature adds its own base
+# addresses to a copy of the table. Plans hold no addresses and no tensors, are immutable and
+# at most PLANS_MAX of them are kept.
+PLANS_MAX = 256
+_plans: collections.OrderedDict = collections.OrderedDict()
+_plans_lock = threading.Lock()
+
+
+def signature(*tensors):
+    """What a plan depends on of its base tensors."""
+    return tuple(None if t is None else (t.shape, t.stride(), t.dtype, t.device) for t in tensors)
+
+
+def _table_dtype(struct):
+    kinds = {ctypes.c_void_p: "u8", ctypes.c_int32: "i4"}
+    return np.dtype({"names": [n for n, _ in struct._fields_],
+                     "formats": [kinds[t] for _, t in struct._fields_],
+                     "offsets": [getattr(struct, n).offset for n, _ in struct._fields_],
+                     "itemsize": ctypes.sizeof(struct)})
+
+
+class _NoSpan:
+    def __call__(self, name):
+        return self
+
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *exc):
+        return False
+
+
+NO_SPAN = _NoSpan()
+
+
+class LaunchPlan:
+    """The calls ``steps`` = [(jobs, scale, mask)] over views of ``bases`` (problem field ->
+    base tensor). ``drop_p``: the dropout probability of every step (its seed comes with each
+    run)."""
+
+    def __init__(self, steps, bases, drop_p=0.0):
+        steps = [s for s in steps if s[0]]
+        self.bwd = bool(steps) and isinstance(steps[0][0][0], BwdJob)
+        self.struct = abi.BwdProblem if self.bwd else abi.FwdProblem
+        pack = _pack_bwd if self.bwd else _pack_fwd
+        drop = (drop_p, 0) if drop_p else None
+        self.drop = bool(drop_p)
+        self.steps, parts, lo = [], [], 0  # (layout, first row, rows, workspace bytes)
+        for jobs, scale, mask in steps:
+            lay, arr = pack(jobs, scale, mask, drop)
+            nbytes = (abi.lib().rmx_attn_bwd_workspace(ctypes.byref(lay), arr, len(jobs))
+                      if self.bwd else 0)
+            self.steps.append((lay, lo, len(jobs), nbytes))
+            parts.append(bytes(arr))
+            lo += len(jobs)
+        self.table = (np.frombuffer(bytearray(b"".join(parts)), dtype=_table_dtype(self.struct))
+                      if parts else None)
+        self.fields = []
+        for name, base in bases.items():
+            if self.table is None or base is None:
+                continue
+            col = self.table[name]
+            if not col.any():
+                continue
+            if not col.all():
+                raise AssertionError(f"{name} is set in some problems only")
+            col -= np.uint64(base.data_ptr())
+            self.fields.append(name)
+
+    def bind(self, bases):
+        """The problem tables at the addresses of ``bases``."""
+        t = self.table.copy()
+        for name in self.fields:
+            t[name] += np.uint64(bases[name].data_ptr())
+        return t
+
+    def _layout(self, lay, seed):
+        if not self.drop:
+            return lay
+        lay = abi.AttnLayout.from_buffer_copy(lay)
+        lay.drop_seed_lo, lay.drop_seed_hi = seed & 0xFFFFFFFF, (seed >> 32) & 0xFFFFFFFF
+        return lay
+
+    def problems(self, table, lo):
+        return ctypes.byref(self.struct.from_buffer(table.view(np.uint8), lo * table.itemsize))
+
+    def run_fwd(self, bases, seed, like, span):
+        """Launch the forward steps; ``span()`` brackets each (timing)."""
+        if self.table is None:
+            return
+        t, lib, stream = self.bind(bases), abi.lib(), abi.stream_of(like)
+        for lay, lo, n, _ in self.steps:
+            with span("attn_fwd"):
+                abi.check(lib.rmx_attn_fwd(ctypes.byref(self._layout(lay, seed)),
+                                           self.problems(t, lo), n, stream))
+
+    def run_bwd(self, bases, seed, like, span=None):
+        """Launch the backward steps: dK/dV then dQ of each, in one call, or in one call each
+        bracketed by ``span``."""
+        if self.table is None:
+            return
+        t, lib = self.bind(bases), abi.lib()
+        if span is None:
+            for lay, lo, n, nbytes in self.steps:
+                _launch_bwd(lib, self._layout(lay, seed), self.problems(t, lo), n, nbytes, like)
+            return
+        tk, tq = t.copy(), t
+        tk["dq_mode"] = tq["dkv_mode"] = abi.GRAD_NONE
+        for lay, lo, n, nbytes in self.steps:
+            lay = self._layout(lay, seed)
+            with span("attn_bwd_dkdv"):
+                _launch_bwd(lib, lay, self.problems(tk, lo), n, nbytes, like)
+            with span("attn_bwd_dq"):
+                _launch_bwd(lib, lay, self.problems(tq, lo), n, 0, like)
+
+
+def plan(key, build):
+    """The kept plan of ``key``, built (``build()``) on first use."""
+    with _plans_lock:
+        p = _plans.get(key)
+        if p is not None:
+            _plans.move_to_end(key)
+            return p
+    p = build()
+    with _plans_lock:
+        _plans[key] = p
+        while len(_plans) > PLANS_MAX:
+            _plans.popitem(last=False)
+    return p

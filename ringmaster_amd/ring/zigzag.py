@@ -134,6 +134,21 @@ class _Ctx:
                 start = torch.searchsorted(d2.contiguous(), d2.contiguous(), right=False)
                 self.kgidx = start[:, rows].permute(1, 0, 2).to(torch.int32).contiguous()
 
+    @property
+    def drop_p(self):
+        return 0.0 if self.dropout is None else float(self.dropout[0])
+
+    @property
+    def drop_seed(self):
+        return 0 if self.dropout is None else int(self.dropout[1]) & ((1 << 64) - 1)
+
+    def key(self, only_ranks):
+        """What the ring's launch plans depend on besides their tensors' signatures."""
+        return (self.layout, self.causal, self.scale, self.drop_p,
+                None if self.window is None else tuple(self.window),
+                None if self.right is None else tuple(self.right),
+                None if only_ranks is None else frozenset(only_ranks))
+
     def schedule(self, split_final: bool):
         if self.layout == "zigzag":
             return zigzag_schedule(self.P, self.L, split_final=split_final)
@@ -229,20 +244,6 @@ class KernelTimer:
         self.events.clear()
 
 
-class _NoTimer:
-    def __call__(self, name):
-        return self
-
-    def __enter__(self):
-        return None
-
-    def __exit__(self, *exc):
-        return False
-
-
-_NO_TIMER = _NoTimer()
-
-
 def _only(blocks, only_ranks):
     """The blocks the ranks in ``only_ranks`` compute (all blocks for None)."""
     return blocks if only_ranks is None else [bl for bl in blocks if bl.runs_on in only_ranks]
@@ -262,7 +263,7 @@ def ring_forward(q, k, v, scale: float, doc: torch.Tensor | None = None, timer=N
     computed (per-rank timing). ``window`` (contiguous layouts or document masks): one
     bound per rank on the global ``pos_q - pos_k`` of its queries; ``right`` (non-causal
     contiguous rings): one bound per rank on the global ``pos_k - pos_q``."""
-    timer = timer or _NO_TIMER
+    timer = timer or ops.NO_SPAN
     c = _Ctx(q, k, scale, doc, layout, causal, window, dropout, right)
     qd, kd, vd = q.transpose(2, 3), k.transpose(2, 3), v.transpose(2, 3)  # [P, b, L, H, d] views
     dev = q.device
@@ -272,23 +273,31 @@ def ring_forward(q, k, v, scale: float, doc: torch.Tensor | None = None, timer=N
     acc_lse = None
     if c.P > 1:
         acc_lse = torch.empty((c.P, c.b, c.hq, c.L), dtype=torch.float32, device=dev)
-    for s, blocks in enumerate(c.schedule(split_final=True)):
-        jobs = []
-        for bl in _only(blocks, only_ranks):
-            r, kr = bl.rank, bl.kv_rank
-            qs, ks = slice(bl.q_lo, bl.q_hi), slice(bl.k_lo, bl.k_hi)
-            jobs.append(ops.FwdJob(
-                q=qd[r][:, qs], k=kd[kr][:, ks], v=vd[kr][:, ks],
-                mode=_fwd_mode(bl.first, bl.last),
-                out=out[r][:, qs], lse=lse[r][:, :, qs],
-                acc_out=acc[r][:, qs],
-                acc_lse=None if acc_lse is None else acc_lse[r][:, :, qs],
-                q_gidx=c.idx(r, bl.q_lo, bl.q_hi), k_gidx=c.kidx(kr, bl.k_lo, bl.k_hi),
-                q_doc=c.docs(r, bl.q_lo, bl.q_hi), k_doc=c.docs(kr, bl.k_lo, bl.k_hi),
-                window=c.block_window(bl), right=c.block_right(bl),
-                **dict(zip(("drop_q0", "drop_k0"), c.block_drop(bl)))))
-        with timer("attn_fwd"):
-            ops.attn_fwd(jobs, scale=scale, mask=c.mask(s), dropout=c.dropout)
+    bases = dict(q=q, k=k, v=v, out=out, lse=lse, acc_out=acc, acc_lse=acc_lse,
+                 q_gidx=c.gidx, k_gidx=c.kgidx, q_doc=c.rdoc, k_doc=c.rdoc)
+
+    def build():
+        steps = []
+        for s, blocks in enumerate(c.schedule(split_final=True)):
+            jobs = []
+            for bl in _only(blocks, only_ranks):
+                r, kr = bl.rank, bl.kv_rank
+                qs, ks = slice(bl.q_lo, bl.q_hi), slice(bl.k_lo, bl.k_hi)
+                jobs.append(ops.FwdJob(
+                    q=qd[r][:, qs], k=kd[kr][:, ks], v=vd[kr][:, ks],
+                    mode=_fwd_mode(bl.first, bl.last),
+                    out=out[r][:, qs], lse=lse[r][:, :, qs],
+                    acc_out=acc[r][:, qs],
+                    acc_lse=None if acc_lse is None else acc_lse[r][:, :, qs],
+                    q_gidx=c.idx(r, bl.q_lo, bl.q_hi), k_gidx=c.kidx(kr, bl.k_lo, bl.k_hi),
+                    q_doc=c.docs(r, bl.q_lo, bl.q_hi), k_doc=c.docs(kr, bl.k_lo, bl.k_hi),
+                    window=c.block_window(bl), right=c.block_right(bl),
+                    **dict(zip(("drop_q0", "drop_k0"), c.block_drop(bl)))))
+            steps.append((jobs, scale, c.mask(s)))
+        return ops.LaunchPlan(steps, bases, c.drop_p)
+
+    plan = ops.plan(("ring_fwd", c.key(only_ranks), ops.signature(q, k, v, c.gidx)), build)
+    plan.run_fwd(bases, c.drop_seed, q, timer)
     return out, lse, acc
 
 
@@ -300,7 +309,7 @@ def ring_backward(dout, q, k, v, out, lse, scale: float, doc: torch.Tensor | Non
     Returns fp32 (dq [P, b, L, Hq, d], dk, dv [P, b, L, Hkv, d]). Each step launches the
     KV-major dK/dV kernel and the Q-major dQ kernel over all ranks (``only_ranks``: over
     those ranks only, as in :func:`ring_forward`; the gradients are then partial)."""
-    timer = timer or _NO_TIMER
+    timer = timer or ops.NO_SPAN
     c = _Ctx(q, k, scale, doc, layout, causal, window, dropout, right)
     qd, kd, vd = q.transpose(2, 3), k.transpose(2, 3), v.transpose(2, 3)
     dev = q.device
@@ -320,27 +329,31 @@ def ring_backward(dout, q, k, v, out, lse, scale: float, doc: torch.Tensor | Non
     dq = torch.empty((c.P, c.b, c.L, c.hq, c.d), dtype=torch.float32, device=dev)
     dk = torch.empty((c.P, c.b, c.L, c.hkv, c.d), dtype=torch.float32, device=dev)
     dv = torch.empty_like(dk)
-    for s, blocks in enumerate(c.schedule(split_final=False)):
-        mode = abi.GRAD_WRITE_F32 if s == 0 else abi.GRAD_ACC_F32
-        kv_jobs, q_jobs = [], []
-        for bl in _only(blocks, only_ranks):
-            r, kr = bl.rank, bl.kv_rank
-            qs, ks = slice(bl.q_lo, bl.q_hi), slice(bl.k_lo, bl.k_hi)
-            common = dict(
-                q=qd[r][:, qs], k=kd[kr][:, ks], v=vd[kr][:, ks], dout=dout[r][:, qs],
-                lse=lse[r][:, :, qs], delta=delta[r][:, :, qs], nlse=nlse[r][:, :, qs],
-                q_gidx=c.idx(r, bl.q_lo, bl.q_hi), k_gidx=c.kidx(kr, bl.k_lo, bl.k_hi),
-                q_doc=c.docs(r, bl.q_lo, bl.q_hi), k_doc=c.docs(kr, bl.k_lo, bl.k_hi),
-                window=c.block_window(bl), right=c.block_right(bl),
-                **dict(zip(("drop_q0", "drop_k0"), c.block_drop(bl))))
-            kv_jobs.append(ops.BwdJob(dq_mode=abi.GRAD_NONE, dkv_mode=mode,
-                                      dk_acc=dk[kr][:, ks], dv_acc=dv[kr][:, ks], **common))
-            q_jobs.append(ops.BwdJob(dq_mode=mode, dkv_mode=abi.GRAD_NONE,
-                                     dq_acc=dq[r][:, qs], **common))
-        with timer("attn_bwd_dkdv"):
-            ops.attn_bwd(kv_jobs, scale=scale, mask=c.mask(s), dropout=c.dropout)
-        with timer("attn_bwd_dq"):
-            ops.attn_bwd(q_jobs, scale=scale, mask=c.mask(s), dropout=c.dropout)
+    bases = dict(q=q, k=k, v=v, dout=dout, lse=lse, delta=delta, nlse=nlse, dq_acc=dq, dk_acc=dk,
+                 dv_acc=dv, q_gidx=c.gidx, k_gidx=c.kgidx, q_doc=c.rdoc, k_doc=c.rdoc)
+
+    def build():
+        steps = []
+        for s, blocks in enumerate(c.schedule(split_final=False)):
+            mode = abi.GRAD_WRITE_F32 if s == 0 else abi.GRAD_ACC_F32
+            jobs = []
+            for bl in _only(blocks, only_ranks):
+                r, kr = bl.rank, bl.kv_rank
+                qs, ks = slice(bl.q_lo, bl.q_hi), slice(bl.k_lo, bl.k_hi)
+                jobs.append(ops.BwdJob(
+                    q=qd[r][:, qs], k=kd[kr][:, ks], v=vd[kr][:, ks], dout=dout[r][:, qs],
+                    lse=lse[r][:, :, qs], delta=delta[r][:, :, qs], nlse=nlse[r][:, :, qs],
+                    q_gidx=c.idx(r, bl.q_lo, bl.q_hi), k_gidx=c.kidx(kr, bl.k_lo, bl.k_hi),
+                    q_doc=c.docs(r, bl.q_lo, bl.q_hi), k_doc=c.docs(kr, bl.k_lo, bl.k_hi),
+                    window=c.block_window(bl), right=c.block_right(bl),
+                    dq_mode=mode, dkv_mode=mode, dq_acc=dq[r][:, qs],
+                    dk_acc=dk[kr][:, ks], dv_acc=dv[kr][:, ks],
+                    **dict(zip(("drop_q0", "drop_k0"), c.block_drop(bl)))))
+            steps.append((jobs, scale, c.mask(s)))
+        return ops.LaunchPlan(steps, bases, c.drop_p)
+
+    plan = ops.plan(("ring_bwd", c.key(only_ranks), ops.signature(q, k, v, dout, c.gidx)), build)
+    plan.run_bwd(bases, c.drop_seed, q, None if timer is ops.NO_SPAN else timer)
     return dq, dk, dv
 
 
