@@ -606,8 +606,10 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_kernel(const BwdParams p
   __shared__ __attribute__((aligned(1024))) uint8_t sO[NB][C::QT];
   // nl = -lse log2(e) and delta of each tile
   __shared__ __attribute__((aligned(512))) float sM[NB][2 * BQ];
-  __shared__ int sQg[NB][BQ];
-  __shared__ int sQd[NB][BQ];
+  // RMX_MASK_DOC: global index and document of each tile's queries (rows past the end read 0:
+  // their Q and dO rows are 0, so they add nothing either way)
+  __shared__ __attribute__((aligned(256))) int sQg[NB][BQ];
+  __shared__ __attribute__((aligned(256))) int sQd[NB][BQ];
   __shared__ int sRange[2];
 
   const WgCoord wc = map_workgroup(prm.map, blockIdx.x);
@@ -686,7 +688,9 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_kernel(const BwdParams p
   if (ntile == 0 && P.dkv_mode == RMX_GRAD_ACC_F32) return;
   const int wave_klast = (kw0 + 31 < sk ? kw0 + 31 : sk - 1);
 
-  // ---- tile loads. Wave 0 first loads the tile's lse and delta (one dword per
+  // ---- tile loads. Wave 0 first loads the tile's lse and delta, and under document masks
+  // its queries' indices and documents (by LDS DMA too: as register loads their waits drained
+  // the tiles in flight, 7.96 against @ ms for 16384^2 unmasked pairs) (one dword per
   // lane; rows past the end read 0, where Q and dO rows are 0 as well, so they
   // add nothing), then every wave its share of the Q and dO rows (instruction n
   // fills LDS bytes [1024 n, 1024 n + 1024), lane L row n*RPK + L/CH, swizzled
@@ -724,6 +728,12 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_kernel(const BwdParams p
   }
   // part p of a tile's loads into buffer b: p = 0 also the metadata (wave 0), then the
   // wave's Q rows (p < NDMA) or dO rows; all 2 NDMA parts make the tile
+  auto dma_doc = [&](int b, int qa, uint32_t n) __attribute__((always_inline)) {
+    if (mask == RMX_MASK_DOC) {
+      dma4_async(make_rsrc(qgid + qa, n), lds_addr(sQg[b]), 4 * lane);
+      dma4_async(make_rsrc(qdoc + qa, n), lds_addr(sQd[b]), 4 * lane);
+    }
+  };
   auto dma_part = [&](int b, Cursor cu, bool live, int p) __attribute__((always_inline)) {
     const int qa = cu.qt * BQ;
     const int hi = live ? cu.hi : 0;
@@ -733,6 +743,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_kernel(const BwdParams p
       const uint32_t m = lds_addr(sM[b]);
       dma4_async(make_rsrc(nb0 + lo, n), m, 4 * lane);
       dma4_async(make_rsrc(db0 + lo, n), m + 4 * BQ, 4 * lane);
+      dma_doc(b, qa, n);
     }
     if (p < C::NDMA) {
       const i32x4 qrs = make_rsrc(qb0 + hi * qhs + qa * qss, live ? qspan - (uint32_t)(qa * qss) : 0u);
@@ -752,6 +763,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_kernel(const BwdParams p
       const uint32_t m = lds_addr(sM[b]);
       dma4_async(make_rsrc(nb0 + lo, n), m, 4 * lane);
       dma4_async(make_rsrc(db0 + lo, n), m + 4 * BQ, 4 * lane);
+      dma_doc(b, qa, n);
     }
     const int qo = hi * qhs + qa * qss, oo = hi * ohs + qa * oss;
     const i32x4 qrs = make_rsrc(qb0 + qo, live ? qspan - (uint32_t)(qa * qss) : 0u);
@@ -764,26 +776,6 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_kernel(const BwdParams p
       dma16_async(ors, od + 1024 * n, vo[i]);
     }
   };
-  int nqg = 0, nqd = 0;
-  auto doc_load = [&](Cursor cu) {
-    if (mask == RMX_MASK_DOC && tid < BQ) {
-      const int qq = cu.qt * BQ + tid;
-      if (qq < sq) {
-        nqg = qgid[qq];
-        nqd = qdoc[qq];
-      } else {
-        nqg = -2147483647;  // rows past the end: masked
-        nqd = -1;
-      }
-    }
-  };
-  auto doc_store = [&](int slot) {
-    if (mask == RMX_MASK_DOC && tid < BQ) {
-      sQg[slot][tid] = nqg;
-      sQd[slot][tid] = nqd;
-    }
-  };
-
   // per-lane LDS byte offsets (swizzle folded in): rows (A of S, dP'): query row
   // 32 mb + sigma(l32), chunk 2 kb + hl
   int raddr[NKB];
@@ -935,8 +927,6 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_kernel(const BwdParams p
   dma_tile(0, cur, ntile > 0);
   dma_tile(1, nx1, ntile > 1);
   dma_tile(2, nx2, ntile > 2);
-  doc_load(cur);
-  doc_store(0);
 
   f32x16 dv[NDB], dk[NDB], s[2], dp[2], nl[2];
   // dropout: delta of the tile's rows (the dP' accumulator then starts at 0, see pack_pair)
@@ -1038,7 +1028,6 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_kernel(const BwdParams p
   auto tile = [&](auto bc, int j) {
     constexpr int B = decltype(bc)::value;  // == j % NB
     constexpr int BN = (B + 1) % NB;
-    if (j + 1 < ntile) doc_load(nx1);
     bf16x8 pt[4], dst[4];
     int qa_next = 0;  // first query of tile j + 1 (set at the hand-over, read in phase 3)
     Cursor dcu = nx3;  // tile j + 3: its loads issue one part per step early in phase 2
@@ -1138,7 +1127,6 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_kernel(const BwdParams p
 
     // hand-over: tile j + 1 landed (tile j + 2 may stay in flight); tile j - 3's
     // buffer (last read in phase 2 of tile j - 3) takes tile j + 3
-    if (j + 1 < ntile) doc_store(BN);
     wait_vm_barrier<2 * C::NDMA>();
     if constexpr (DROP) dma_tile((B + 3) % NB, nx3, j + 3 < ntile);
     qa_next = nx1.qt * BQ;
@@ -1176,11 +1164,11 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_kernel(const BwdParams p
   // (one wait, not one memory round trip per row). A launch of one tile: 28.4 -> 12.8 us at
   // head dim 128, 19.4 -> 8.7 at 64.
   // Caller pointers below vector alignment take the element-wise form, straight from the
-  // accumulators; the document and dropout kernels a compact loop over the staged rows. The
-  // choice is the register allocator's: with the compact loop the FULL and causal main loops
-  // move 47 values per tile between VGPRs and AGPRs instead of 14 and run 1% slower, with the
-  // element-wise form the document loop takes 20 more VALU instructions per tile and the
-  // dropout kernels spill 192 registers (the compact form: none).
+  // accumulators; the dropout kernels a compact loop over the staged rows. The choice is the
+  // register allocator's: with the compact loop the FULL and causal main loops move 47 values
+  // per tile between VGPRs and AGPRs instead of 14 and run 1% slower (documents: 113 instead
+  // of 34, 8%), with the element-wise form the dropout kernels spill 192 registers (the
+  // compact form: none).
   constexpr int CPR = HD / 4;    // 16-byte chunks per fp32 row
   constexpr int RPI = 64 / CPR;  // rows per instruction of a wave
   constexpr int NI = 32 / RPI;   // instructions per wave and gradient
@@ -1193,7 +1181,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_kernel(const BwdParams p
   const bool w32 = mode == RMX_GRAD_WRITE_F32 || mode == RMX_GRAD_ACC_F32;
   const bool vec = (!(rd || w32) || (((uintptr_t)E.dv_acc | (uintptr_t)E.dk_acc) & 15) == 0) &&
                    (w32 || (((uintptr_t)E.dv | (uintptr_t)E.dk) & 7) == 0);
-  constexpr bool ELEMS = !DROP && MASK != RMX_MASK_DOC;
+  constexpr bool ELEMS = !DROP;
   if (ELEMS && !vec) {
     float prev[2][NDB][16];
     if (rd) {
@@ -1352,8 +1340,9 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_d256_kernel(const BwdPar
   uint8_t(*const sO)[QT] = reinterpret_cast<uint8_t(*)[QT]>(smem + NQB * QT);
   uint8_t* const sK = smem + (NQB + NOB) * QT;
   __shared__ __attribute__((aligned(256))) float sM[NOB][2][64];  // nl, delta (a DMA writes 64)
-  __shared__ int sQg[NOB][BQ];
-  __shared__ int sQd[NOB][BQ];
+  // RMX_MASK_DOC: as in the kernel above (a DMA writes 64)
+  __shared__ __attribute__((aligned(256))) int sQg[NOB][64];
+  __shared__ __attribute__((aligned(256))) int sQd[NOB][64];
   __shared__ int sRange[2];
 
   const WgCoord wc = map_workgroup(prm.map, blockIdx.x);
@@ -1469,6 +1458,10 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_d256_kernel(const BwdPar
       const uint32_t n = 4u * (uint32_t)(sq - qa);
       dma4_async(make_rsrc(nb0 + lo, n), lds_addr(&sM[bo][0][0]), 4 * lane);
       dma4_async(make_rsrc(db0 + lo, n), lds_addr(&sM[bo][1][0]), 4 * lane);
+      if (mask == RMX_MASK_DOC) {
+        dma4_async(make_rsrc(qgid + qa, n), lds_addr(&sQg[bo][0]), 4 * lane);
+        dma4_async(make_rsrc(qdoc + qa, n), lds_addr(&sQd[bo][0]), 4 * lane);
+      }
     }
     const i32x4 qrs = make_rsrc(qb0 + cu.hi * qhs + qa * qss, qspan - (uint32_t)(qa * qss));
     const i32x4 ors = make_rsrc(ob0 + cu.hi * ohs + qa * oss, ospan - (uint32_t)(qa * oss));
@@ -1480,26 +1473,6 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_d256_kernel(const BwdPar
       dma16_async(ors, od + 1024 * n, vo[i]);
     }
   };
-  int nqg = 0, nqd = 0;
-  auto doc_load = [&](Cursor cu) {
-    if (mask == RMX_MASK_DOC && tid < BQ) {
-      const int qq = cu.qt * BQ + tid;
-      if (qq < sq) {
-        nqg = qgid[qq];
-        nqd = qdoc[qq];
-      } else {
-        nqg = -2147483647;  // rows past the end: masked
-        nqd = -1;
-      }
-    }
-  };
-  auto doc_store = [&](int slot) {
-    if (mask == RMX_MASK_DOC && tid < BQ) {
-      sQg[slot][tid] = nqg;
-      sQd[slot][tid] = nqd;
-    }
-  };
-
   // ---- the K block (rows k0 .. k0 + BKV - 1) into LDS, once; -V of this wave's keys in
   // registers (lane: key row, dims 16 kb + 8 hl ..), MFMA operands from AGPRs
   {
@@ -1670,8 +1643,6 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_d256_kernel(const BwdPar
   Cursor nx1 = advance(cur), nx2 = advance(nx1);
   if (ntile > 0) dma_tile(0, 0, cur);
   if (ntile > 1) dma_tile(1, 1, nx1);
-  doc_load(cur);
-  doc_store(0);
   wait_all_loads();
   lds_barrier();
 
@@ -1736,7 +1707,6 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_d256_kernel(const BwdPar
     constexpr int BQ0 = JC % NQB, BO0 = JC % NOB;              // tile j
     constexpr int BQ1 = (JC + 1) % NQB, BO1 = (JC + 1) % NOB;  // tile j + 1
     constexpr int BQ2 = (JC + 2) % NQB;                        // tile j + 2's Q
-    if (j + 1 < ntile) doc_load(nx1);
     bf16x8 pt[2], dst[2];
     int qa_next = 0, hi_next = 0;  // tile j + 1 (set at the hand-over)
     // operand f of this tile (f >= F: the next tile's)
@@ -1812,7 +1782,6 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_d256_kernel(const BwdPar
 
     // hand-over: tile j + 1 has landed in every wave and this tile's dO slot (read last in
     // phase 1) and tile j - 1's Q buffer are free for tile j + 2
-    if (j + 1 < ntile) doc_store(BO1);
     wait_vm_barrier<0>();
     if (j + 2 < ntile) dma_tile(BQ2, BO0, nx2);
     qa_next = nx1.qt * BQ;
