@@ -74,8 +74,8 @@ struct BwdTiles {
 };
 
 // ---------------------------------------------------------------- dQ (Q-major)
-// One workgroup = 8 waves x 32 queries of one (problem, batch, head). Per key
-// tile (64 keys) and wave:
+// One workgroup = 8 waves x 32 queries of one (problem, batch, head), 4 waves where the
+// launch is small (half_workgroups). Per key tile (64 keys) and wave:
 //   S^T  = K Q^T    A = K rows (LDS), B = Q (VGPRs)        16 MFMAs
 //   dP^T = V dO^T   A = V rows (LDS), B = dO (VGPRs)       16 MFMAs
 //   P = exp2(S c - lse2), dS = P (dP - delta)  (lane = query: lse/delta per lane; the
@@ -98,11 +98,11 @@ struct BwdTiles {
 // (swizzle folded in) plus a compile-time offset below 64 KiB, with no address
 // arithmetic in the loop. Tiles past the end are issued as zero-length loads,
 // which keeps every wait count static.
-// At head dim 256 a workgroup is 4 waves (one per SIMD: Q, dO and the dQ accumulator
+// At head dim 256 a workgroup is always 4 waves (one per SIMD: Q, dO and the dQ accumulator
 // take 256 registers) and a key tile 32 keys, so four K/V buffers (16 KiB each) fit.
-template <int HD>
+template <int HD, int WAVES>
 struct DqCfg {
-  static constexpr int NW = HD == 256 ? 4 : 8;  // waves per workgroup
+  static constexpr int NW = WAVES;              // waves per workgroup
   static constexpr int NT = NW * 64;
   static constexpr int BQ = 32 * NW;            // queries per workgroup
   static constexpr int BK = HD == 256 ? 32 : 64;  // keys per tile
@@ -110,17 +110,17 @@ struct DqCfg {
   static constexpr int MDOC = BK < 64 ? 64 : BK;  // key metadata slots (a DMA writes 64)
 };
 
-template <int HD, int MASK, int DT, bool DROP>
-__global__ __launch_bounds__(DqCfg<HD>::NT, 1) void attn_bwd_dq_kernel(const BwdParams prm) {
+template <int HD, int WAVES, int MASK, int DT, bool DROP>
+__global__ __launch_bounds__(64 * WAVES, 1) void attn_bwd_dq_kernel(const BwdParams prm) {
   using T = BwdTiles<HD>;
-  constexpr int NW = DqCfg<HD>::NW, NT = DqCfg<HD>::NT, BQ = DqCfg<HD>::BQ, BK = DqCfg<HD>::BK;
+  constexpr int NW = DqCfg<HD, WAVES>::NW, NT = DqCfg<HD, WAVES>::NT, BQ = DqCfg<HD, WAVES>::BQ, BK = DqCfg<HD, WAVES>::BK;
   constexpr int MBK = BK / 32, KB2 = BK / 16;  // 32-key blocks of S^T, 16-key steps of dQ
   constexpr int CH = T::CH, NKB = T::NKB, NDB = T::NDB;
   constexpr int RB = HD * 2;              // LDS row bytes (unpadded, swizzled)
   constexpr int KT = BK * RB;             // bytes of one K (or V) tile
   constexpr int RPK = 1024 / RB;          // rows per 1 KiB DMA instruction
   constexpr int NDMA = KT / 1024 / NW;    // DMA instructions per wave, tile and operand
-  constexpr int NB = DqCfg<HD>::NB;       // tile buffers
+  constexpr int NB = DqCfg<HD, WAVES>::NB;       // tile buffers
   // K tiles at [0, NB KT), V tiles after them; V rows get their own base register when
   // the last V tile would sit past the 16-bit LDS instruction offset
   constexpr bool VBASE = 2 * NB * KT - KT / 2 > 65535;
@@ -129,8 +129,8 @@ __global__ __launch_bounds__(DqCfg<HD>::NT, 1) void attn_bwd_dq_kernel(const Bwd
   // K tiles, then V tiles; the epilogue stages the dQ rows here (NW x 32 x HD fp32)
   constexpr int NTB = 2 * NB > NW * 32 * HD * 4 / KT ? 2 * NB : NW * 32 * HD * 4 / KT;
   __shared__ __attribute__((aligned(1024))) uint8_t sT[NTB][KT];
-  __shared__ __attribute__((aligned(256))) int sKg[NB][DqCfg<HD>::MDOC];
-  __shared__ __attribute__((aligned(256))) int sKd[NB][DqCfg<HD>::MDOC];
+  __shared__ __attribute__((aligned(256))) int sKg[NB][DqCfg<HD, WAVES>::MDOC];
+  __shared__ __attribute__((aligned(256))) int sKd[NB][DqCfg<HD, WAVES>::MDOC];
   __shared__ int sRange[2];
 
   const WgCoord wc = map_workgroup(prm.map, blockIdx.x);
@@ -1882,10 +1882,28 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_d256_kernel(const BwdPar
   store(dk, -L.scale, P.dk_acc ? P.dk_acc + so : nullptr, P.dk);
 }
 
+// dQ of the n problems in prm.P (in launch order)
+template <int HD, int WAVES, int DT, bool DROP>
+static hipError_t launch_dq(BwdParams& prm, int n, hipStream_t stream) {
+  using C = DqCfg<HD, WAVES>;
+  const rmx_attn_layout& L = prm.L;
+  int ntile[RMX_MAX_BATCHED];
+  for (int i = 0; i < n; ++i) ntile[i] = (prm.P[i].sq + C::BQ - 1) / C::BQ;
+  const dim3 grid(plan_workgroups(prm.map, n, L.batch * L.hq, L.hq / L.hkv, ntile,
+                                  L.mask == RMX_MASK_CAUSAL));
+  if (L.mask == RMX_MASK_CAUSAL)
+    hipLaunchKernelGGL((attn_bwd_dq_kernel<HD, WAVES, RMX_MASK_CAUSAL, DT, DROP>), grid, dim3(C::NT), 0, stream, prm);
+  else if (L.mask == RMX_MASK_DOC)
+    hipLaunchKernelGGL((attn_bwd_dq_kernel<HD, WAVES, RMX_MASK_DOC, DT, DROP>), grid, dim3(C::NT), 0, stream, prm);
+  else
+    hipLaunchKernelGGL((attn_bwd_dq_kernel<HD, WAVES, RMX_MASK_FULL, DT, DROP>), grid, dim3(C::NT), 0, stream, prm);
+  return hipGetLastError();
+}
+
 template <int HD, int DT, bool DROP>
 hipError_t launch_bwd_t(const rmx_attn_layout& L, const rmx_bwd_problem* probs, int n,
                         const DkdvSplit& split, void* ws, hipStream_t stream) {
-  constexpr int BQ_DQ = DqCfg<HD>::BQ, BKV = HD == 256 ? 128 : DkdvCfg<HD>::BKV;
+  constexpr int BKV = HD == 256 ? 128 : DkdvCfg<HD>::BKV;
   BwdParams pq, pk;
   pq.L = L;
   pk.L = L;
@@ -1912,11 +1930,7 @@ hipError_t launch_bwd_t(const rmx_attn_layout& L, const rmx_bwd_problem* probs, 
   int oq[RMX_MAX_BATCHED], ok[RMX_MAX_BATCHED], ntile[RMX_MAX_BATCHED];
   order_by_cost(nq, cq, oq);
   order_by_cost(nk, ck, ok);
-  for (int i = 0; i < nq; ++i) {
-    pq.P[i] = probs[iq[oq[i]]];
-    ntile[i] = (pq.P[i].sq + BQ_DQ - 1) / BQ_DQ;
-  }
-  const int tq = plan_workgroups(pq.map, nq, L.batch * L.hq, G, ntile, L.mask == RMX_MASK_CAUSAL);
+  for (int i = 0; i < nq; ++i) pq.P[i] = probs[iq[oq[i]]];
   pq.nsplit = 1;
   pq.split_stride = 0;
   pk.nsplit = split.n;
@@ -1968,17 +1982,13 @@ hipError_t launch_bwd_t(const rmx_attn_layout& L, const rmx_bwd_problem* probs, 
     const hipError_t e = launch_dkdv_fold(L, fold, nk, split, ws, stream);
     if (e != hipSuccess) return e;
   }
-  if (tq > 0) {
-    const dim3 grid(tq);
-    if (L.mask == RMX_MASK_CAUSAL)
-      hipLaunchKernelGGL((attn_bwd_dq_kernel<HD, RMX_MASK_CAUSAL, DT, DROP>), grid, dim3(DqCfg<HD>::NT), 0, stream, pq);
-    else if (L.mask == RMX_MASK_DOC)
-      hipLaunchKernelGGL((attn_bwd_dq_kernel<HD, RMX_MASK_DOC, DT, DROP>), grid, dim3(DqCfg<HD>::NT), 0, stream, pq);
-    else
-      hipLaunchKernelGGL((attn_bwd_dq_kernel<HD, RMX_MASK_FULL, DT, DROP>), grid, dim3(DqCfg<HD>::NT), 0, stream, pq);
-    return hipGetLastError();
-  }
-  return hipSuccess;
+  if (nq == 0) return hipSuccess;
+  if constexpr (HD == 256)
+    return launch_dq<HD, 4, DT, DROP>(pq, nq, stream);
+  else if (half_workgroups(L, pq.P, nq))
+    return launch_dq<HD, 4, DT, DROP>(pq, nq, stream);
+  else
+    return launch_dq<HD, 8, DT, DROP>(pq, nq, stream);
 }
 
 }  // namespace rmx

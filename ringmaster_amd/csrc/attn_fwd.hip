@@ -8,7 +8,8 @@
 // (ring/merge.py:20-31, ring/zigzag.py:49-67).
 //
 // Work decomposition: one workgroup = 8 waves = 256 queries of one
-// (problem, batch, head); each wave owns 32 queries and walks the key tiles
+// (problem, batch, head), or 4 waves = 128 where the launch is small
+// (half_workgroups); each wave owns 32 queries and walks the key tiles
 // (64 keys) that the mask leaves. At head dim 256 a workgroup is 4 waves (one per
 // SIMD: the Q operand and the O accumulator alone take 192 registers) and a key tile
 // 32 keys (the seven tile buffers then take 112 KiB of LDS).
@@ -51,9 +52,9 @@ struct FwdParams {
   float drop_scale;   // 1 / (1 - p)
 };
 
-template <int HD>
+template <int HD, int WAVES>
 struct FwdCfg {
-  static constexpr int NW = HD == 256 ? 4 : 8;  // waves per workgroup
+  static constexpr int NW = WAVES;            // waves per workgroup
   static constexpr int NT = NW * 64;
   static constexpr int BQ = 32 * NW;          // queries per workgroup
   static constexpr int BK = HD == 256 ? 32 : 64;  // keys per tile
@@ -71,9 +72,9 @@ struct FwdCfg {
 
 constexpr float kRescaleSlack = 8.0f;  // log2 units: P <= 2^8 between rescales
 
-template <int HD, int MASK, int DT, bool DROP>
-__global__ __launch_bounds__(FwdCfg<HD>::NT, 1) void attn_fwd_kernel(const FwdParams prm) {
-  using C = FwdCfg<HD>;
+template <int HD, int WAVES, int MASK, int DT, bool DROP>
+__global__ __launch_bounds__(64 * WAVES, 1) void attn_fwd_kernel(const FwdParams prm) {
+  using C = FwdCfg<HD, WAVES>;
   constexpr int BK = C::BK, MB = C::MB, NKB = C::NKB, NDB = C::NDB, CH = C::CH, RB = C::RB;
   constexpr int NDMA = C::NDMA;
 
@@ -649,10 +650,10 @@ __global__ __launch_bounds__(FwdCfg<HD>::NT, 1) void attn_fwd_kernel(const FwdPa
   }
 }
 
-template <int HD, int DT, bool DROP>
+template <int HD, int WAVES, int DT, bool DROP>
 static hipError_t launch_fwd_t(const rmx_attn_layout& L, const rmx_fwd_problem* probs, int n,
                                hipStream_t stream) {
-  constexpr int BQ = FwdCfg<HD>::BQ;
+  using C = FwdCfg<HD, WAVES>;
   FwdParams prm;
   prm.L = L;
   prm.scale_log2 = L.scale * kLog2e;
@@ -664,29 +665,33 @@ static hipError_t launch_fwd_t(const rmx_attn_layout& L, const rmx_fwd_problem* 
   order_by_cost(n, cost, order);
   for (int i = 0; i < n; ++i) {
     prm.P[i] = probs[order[i]];
-    ntile[i] = (prm.P[i].sq + BQ - 1) / BQ;
+    ntile[i] = (prm.P[i].sq + C::BQ - 1) / C::BQ;
   }
   const int grid = plan_workgroups(prm.map, n, L.batch * L.hq, L.hq / L.hkv, ntile,
                                    L.mask == RMX_MASK_CAUSAL);
   if (grid == 0) return hipSuccess;
   if (L.mask == RMX_MASK_CAUSAL)
-    hipLaunchKernelGGL((attn_fwd_kernel<HD, RMX_MASK_CAUSAL, DT, DROP>), dim3(grid),
-                       dim3(FwdCfg<HD>::NT), 0, stream, prm);
+    hipLaunchKernelGGL((attn_fwd_kernel<HD, WAVES, RMX_MASK_CAUSAL, DT, DROP>), dim3(grid),
+                       dim3(C::NT), 0, stream, prm);
   else if (L.mask == RMX_MASK_DOC)
-    hipLaunchKernelGGL((attn_fwd_kernel<HD, RMX_MASK_DOC, DT, DROP>), dim3(grid),
-                       dim3(FwdCfg<HD>::NT), 0, stream, prm);
+    hipLaunchKernelGGL((attn_fwd_kernel<HD, WAVES, RMX_MASK_DOC, DT, DROP>), dim3(grid),
+                       dim3(C::NT), 0, stream, prm);
   else
-    hipLaunchKernelGGL((attn_fwd_kernel<HD, RMX_MASK_FULL, DT, DROP>), dim3(grid),
-                       dim3(FwdCfg<HD>::NT), 0, stream, prm);
+    hipLaunchKernelGGL((attn_fwd_kernel<HD, WAVES, RMX_MASK_FULL, DT, DROP>), dim3(grid),
+                       dim3(C::NT), 0, stream, prm);
   return hipGetLastError();
 }
 
 template <int DT, bool DROP>
 static hipError_t launch_fwd_hd(const rmx_attn_layout& L, const rmx_fwd_problem* probs, int n,
                                 hipStream_t stream) {
-  if (L.head_dim > 128) return launch_fwd_t<256, DT, DROP>(L, probs, n, stream);
-  if (L.head_dim > 64) return launch_fwd_t<128, DT, DROP>(L, probs, n, stream);
-  return launch_fwd_t<64, DT, DROP>(L, probs, n, stream);
+  if (L.head_dim > 128) return launch_fwd_t<256, 4, DT, DROP>(L, probs, n, stream);
+  const bool half = half_workgroups(L, probs, n);
+  if (L.head_dim > 64)
+    return half ? launch_fwd_t<128, 4, DT, DROP>(L, probs, n, stream)
+                : launch_fwd_t<128, 8, DT, DROP>(L, probs, n, stream);
+  return half ? launch_fwd_t<64, 4, DT, DROP>(L, probs, n, stream)
+              : launch_fwd_t<64, 8, DT, DROP>(L, probs, n, stream);
 }
 
 hipError_t launch_attn_fwd(const rmx_attn_layout& L, const rmx_fwd_problem* probs, int n,

@@ -180,6 +180,19 @@ __device__ __forceinline__ bool drop_keep(uint32_t qterm, uint32_t kterm, uint32
   return fmix32(qterm ^ kterm) >= thr;
 }
 
+// Host side: whether a forward or dQ launch (head dims up to 128) runs workgroups of 4 waves
+// (128 queries) instead of 8 (256): while they are at most one per CU. A 4-wave workgroup has
+// one wave per SIMD and takes about 0.75 of an 8-wave one's time for the same keys, so twice the
+// workgroups win as long as they run at once: forward / dQ, us, 8 -> 4 waves: 2048^2 causal, 8
+// heads of 128 (64 workgroups of 8) 63 -> 49 / 69 -> 55, 16 heads (128) 66 -> 53 / 73 -> 58; past
+// that, 4096^2 unmasked of 16 heads (256) 146 -> 194 / 181 -> 188.
+template <class Prob>
+inline bool half_workgroups(const rmx_attn_layout& L, const Prob* probs, int n) {
+  int64_t wgs = 0;
+  for (int i = 0; i < n; ++i) wgs += (int64_t)L.batch * L.hq * ((probs[i].sq + 127) / 128);
+  return wgs <= 256;
+}
+
 // Host side: the keep threshold floor(p 2^32) and the scale 1 / (1 - p) of dropout p.
 inline void drop_params(float p, uint32_t* thr, float* scale) {
   if (!(p > 0.f)) {
