@@ -17,9 +17,9 @@
 //   backward: chunk sums of g_cum into g_dt at each chunk's first token / those turned into
 //     what enters each chunk / the chunks, each reading its own first token before the
 //     barrier that precedes its stores.
-// A sequence of one chunk is one launch. At 8 rows x 8192 x 64 the three launches take 28 + 5 + 9
-// us forward and 5 + 5 + 35 us backward; the first and the last of these are bound by the VALU
-// work of softplus (25 MB and 42 MB moved).
+// A sequence of one chunk is one launch. At 8 rows x 8192 x 64 the three launches take 19 + 5 + 9
+// us forward and 5 + 5 + 29 us backward, 25 MB and 42 MB moved by the first and the last of these;
+// cum_A's rms error falls from 1e-6 to 6e-8 (shorter chains of sums).
 #include "rmx_kernels.h"
 
 namespace rmx {
@@ -47,7 +47,27 @@ __device__ __forceinline__ float dt_at(const DtArgs& a, int64_t i) {
   return a.dt_f32 ? reinterpret_cast<const float*>(a.dt)[i]
                   : bf2f(reinterpret_cast<const uint16_t*>(a.dt)[i]);
 }
-__device__ __forceinline__ float softplus_t(float x) { return x > 20.f ? x : log1pf(expf(x)); }
+// softplus(x) = max(x, 0) + log1p(z) and its derivative, with z = exp(-|x|). log1p(z) =
+// 2 atanh(s) with s = z / (2 + z) <= 1/3, and 2 s = z - s z: z - s (z - R), R the atanh series
+// past its first term (cut at 2e-9 of the whole), so the rounding of s and R only enters a
+// second-order term: as accurate as the library's log1pf (e's rms error 3.6e-8 with either), and
+// the first forward kernel takes 19 us instead of 28, the last backward one 29 instead of 35. (A
+// shorter exp too, the hardware's exp2 with a first-order correction: 18 and 27 us, but an rms
+// error of 4.4e-8.)
+__device__ __forceinline__ float log1p_unit(float z) {  // 0 <= z <= 1
+  const float s = z * __builtin_amdgcn_rcpf(2.f + z), q = s * s;
+  float a = 2.f / 15.f;
+  a = fmaf(a, q, 2.f / 13.f);
+  a = fmaf(a, q, 2.f / 11.f);
+  a = fmaf(a, q, 2.f / 9.f);
+  a = fmaf(a, q, 2.f / 7.f);
+  a = fmaf(a, q, 2.f / 5.f);
+  a = fmaf(a, q, 2.f / 3.f);
+  return fmaf(-s, fmaf(-a, q, z), z);
+}
+__device__ __forceinline__ float softplus_t(float x) {
+  return x > 20.f ? x : fmaxf(x, 0.f) + log1p_unit(expf(-fabsf(x)));
+}
 
 constexpr int kDtThreads = 512;
 constexpr int kDtRun = 16;  // tokens per thread
@@ -255,9 +275,11 @@ __global__ __launch_bounds__(kDtThreads) void mamba2_dt_bwd_kernel(const DtArgs 
     const float ge = Ah * R + d[i];
     float e = x[i], gdt = ge;
     if (a.softplus) {
-      const float z = expf(y);
-      e = y > 20.f ? y : log1pf(z);
-      gdt = y > 20.f ? ge : ge * (z / (z + 1.f));
+      const float z = expf(-fabsf(y)), d = 1.f + z;
+      e = y > 20.f ? y : fmaxf(y, 0.f) + log1p_unit(z);
+      float r = __builtin_amdgcn_rcpf(d);
+      r = fmaf(fmaf(-d, r, 1.f), r, r);
+      gdt = y > 20.f ? ge : ge * (y >= 0.f ? r : z * r);
     }
     if (i < p.n) {
       pa += R * e;
