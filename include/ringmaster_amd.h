@@ -43,7 +43,7 @@ extern "C" {
                               17: rmx_linear_scan_status;
                               18: right-bounded windows (problem window_right), and since,
                                   as additions: rmx_mamba2_dt_cumsum_state_bwd,
-                                  rmx_attn_bwd_ws */
+                                  rmx_attn_bwd_ws, rmx_cast_half */
 
 /* error codes */
 #define RMX_OK 0
@@ -253,6 +253,15 @@ int32_t rmx_lse_merge(float* out, float* lse, const void* blk_out, int32_t blk_t
                       const int64_t* l_strides /*3*/, const int64_t* bo_strides /*3*/,
                       const int64_t* bl_strides /*2: batch, head*/, int32_t init,
                       void* stream);
+
+/*
+ * dst[i][j] = src[i][j] rounded to nearest even, for up to RMX_CAST_MAX contiguous arrays in one
+ * launch: n[i] elements (a multiple of 8), 16-byte aligned, dst of type RMX_DTYPE_*. The cast
+ * of the reverse ring's accumulated gradients to the inputs' type (ring/zigzag.py:253-254).
+ */
+#define RMX_CAST_MAX 4
+int32_t rmx_cast_half(const float* const* src, uint16_t* const* dst, const int64_t* n,
+                      int32_t count, int32_t dtype, void* stream);
 
 /*
  * Zigzag (head_tail) shard of `batch` rows of `seq` tokens over `world` ranks:

@@ -103,6 +103,8 @@ SIGNATURES = {
     "rmx_lse_merge": (_i32, [_vp, _vp, _vp, _i32, _vp, _i32, _i32, _i32, _i32,
                              ctypes.POINTER(_i64), ctypes.POINTER(_i64), ctypes.POINTER(_i64),
                              ctypes.POINTER(_i64), _i32, _vp]),
+    "rmx_cast_half": (_i32, [ctypes.POINTER(_vp), ctypes.POINTER(_vp), ctypes.POINTER(_i64), _i32,
+                             _i32, _vp]),
     "rmx_zigzag_gather": (_i32, [_vp, _vp, _i32, _i32, _i32, _i32, _i64, _i64, _vp, _vp]),
     "rmx_zigzag_scatter": (_i32, [_vp, _vp, _i32, _i32, _i32, _i64, _i64, _vp]),
     "rmx_linear_scan_fwd": (_i32, [_vp] * 5 + [_i32] * 5 + [_vp, ctypes.c_size_t, _vp]),

@@ -282,6 +282,28 @@ int32_t rmx_lse_merge(float* out, float* lse, const void* blk_out, int32_t blk_t
                     "rmx_lse_merge launch");
 }
 
+int32_t rmx_cast_half(const float* const* src, uint16_t* const* dst, const int64_t* n,
+                      int32_t count, int32_t dtype, void* stream) {
+  if (count < 0 || count > RMX_CAST_MAX)
+    return fail(RMX_EINVAL, "count must lie in [0, %d] (got %d)", RMX_CAST_MAX, count);
+  if (dtype != RMX_DTYPE_BF16 && dtype != RMX_DTYPE_F16)
+    return fail(RMX_EINVAL, "unknown element type %d", dtype);
+  if (count == 0) return RMX_OK;
+  if (!src || !dst || !n) return fail(RMX_EINVAL, "NULL array list");
+  for (int i = 0; i < count; ++i) {
+    if (n[i] < 0 || n[i] % 8)
+      return fail(RMX_EINVAL, "array %d: %lld elements (a multiple of 8)", i, (long long)n[i]);
+    if (n[i] / 2048 >= 2147483647LL)
+      return fail(RMX_EUNSUPPORTED, "array %d: more than 2^31 workgroups", i);
+    if (n[i] && (!src[i] || !dst[i])) return fail(RMX_EINVAL, "array %d is NULL", i);
+    if (!aligned(src[i], 16) || !aligned(dst[i], 16))
+      return fail(RMX_EINVAL, "array %d must be 16-byte aligned", i);
+  }
+  return dev_status(rmx::launch_cast_half(src, dst, n, count, dtype == RMX_DTYPE_F16,
+                                          (hipStream_t)stream),
+                    "rmx_cast_half launch");
+}
+
 int32_t rmx_zigzag_gather(const void* src, void* dst, int32_t batch, int32_t seq, int32_t world,
                           int32_t rank, int64_t row_bytes, int64_t src_bstride,
                           const void* pad_row, void* stream) {

@@ -157,4 +157,48 @@ hipError_t launch_lse_merge(float* out, float* lse, const void* blk_out, int blk
   return hipGetLastError();
 }
 
+// ---------------------------------------------------------------- fp32 -> 16 bits
+// The ring backward's fp32 accumulators to the gradients' type, all arrays of a call in one
+// launch (blockIdx.y): three separate casts were three launches of 4-5 us each beside 2-3 us of
+// data in a small ring. HBM-bound: 8 elements per thread, each byte touched once.
+struct CastParams {
+  const float* src[RMX_CAST_MAX];
+  uint16_t* dst[RMX_CAST_MAX];
+  int64_t n8[RMX_CAST_MAX];  // 8-element units
+};
+
+template <int DT>
+__global__ __launch_bounds__(256) void cast_half_kernel(const CastParams prm) {
+  const int y = blockIdx.y;
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= prm.n8[y]) return;
+  const f32x4 a = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(prm.src[y] + 8 * i));
+  const f32x4 b = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(prm.src[y] + 8 * i + 4));
+  u32x4 u;
+  u[0] = cvt_pk<DT>(a[0], a[1]);
+  u[1] = cvt_pk<DT>(a[2], a[3]);
+  u[2] = cvt_pk<DT>(b[0], b[1]);
+  u[3] = cvt_pk<DT>(b[2], b[3]);
+  *reinterpret_cast<u32x4*>(prm.dst[y] + 8 * i) = u;
+}
+
+hipError_t launch_cast_half(const float* const* src, uint16_t* const* dst, const int64_t* n,
+                            int count, int f16, hipStream_t stream) {
+  CastParams prm{};
+  int64_t most = 0;
+  for (int i = 0; i < count; ++i) {
+    prm.src[i] = src[i];
+    prm.dst[i] = dst[i];
+    prm.n8[i] = n[i] / 8;
+    most = prm.n8[i] > most ? prm.n8[i] : most;
+  }
+  if (most == 0) return hipSuccess;
+  const dim3 grid((unsigned)((most + 255) / 256), count);
+  if (f16)
+    hipLaunchKernelGGL((cast_half_kernel<RMX_DTYPE_F16>), grid, dim3(256), 0, stream, prm);
+  else
+    hipLaunchKernelGGL((cast_half_kernel<RMX_DTYPE_BF16>), grid, dim3(256), 0, stream, prm);
+  return hipGetLastError();
+}
+
 }  // namespace rmx

@@ -32,6 +32,8 @@ hipError_t launch_lse_merge(float* out, float* lse, const void* blk_out, int blk
                             const float* blk_lse, int batch, int seq, int heads, int head_dim,
                             const int64_t* os, const int64_t* ls, const int64_t* bos,
                             const int64_t* bls, int init, hipStream_t stream);
+hipError_t launch_cast_half(const float* const* src, uint16_t* const* dst, const int64_t* n,
+                            int count, int f16, hipStream_t stream);
 hipError_t launch_zigzag(const void* src, void* dst, int batch, int seq, int world, int rank,
                          int64_t row_bytes, int64_t bstride, const void* pad_row, int scatter,
                          hipStream_t stream);

@@ -303,6 +303,18 @@ def _launch_bwd(lib, lay, problems, n, nbytes, like):
                                   abi.stream_of(like)))
 
 
+def cast_half(tensors, dtype):
+    """Contiguous fp32 tensors (element counts multiples of 8) as bf16 or fp16, one launch."""
+    outs = [torch.empty(t.shape, dtype=dtype, device=t.device) for t in tensors]
+    n = len(tensors)
+    abi.check(abi.lib().rmx_cast_half(
+        (ctypes.c_void_p * n)(*(t.data_ptr() for t in tensors)),
+        (ctypes.c_void_p * n)(*(t.data_ptr() for t in outs)),
+        (ctypes.c_int64 * n)(*(t.numel() for t in tensors)), n, _DTYPES[dtype],
+        abi.stream_of(tensors[0])))
+    return outs
+
+
 # ---------------------------------------------------------------- launch plans
 # Building a call's jobs (views, checks, strides) takes 20-40 us of host time per job, more
 # than a small ring step's kernels. A plan keeps what those jobs come to for one signature of

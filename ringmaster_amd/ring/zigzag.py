@@ -378,8 +378,9 @@ class EmulatedRing(torch.autograd.Function):
                                    ctx.layout, ctx.causal, window=ctx.window, dropout=ctx.dropout,
                                    right=ctx.right)
         # fp32 accumulators -> q.dtype, returned in the interface layout [P, b, H, L, d]
-        return (dq.to(q.dtype).transpose(2, 3), dk.to(k.dtype).transpose(2, 3),
-                dv.to(v.dtype).transpose(2, 3), None, None, None, None, None, None, None, None)
+        dq, dk, dv = ops.cast_half((dq, dk, dv), q.dtype)
+        return (dq.transpose(2, 3), dk.transpose(2, 3), dv.transpose(2, 3), None, None, None, None,
+                None, None, None, None)
 
 
 def check_ring_inputs(q, k, v):
