@@ -507,13 +507,33 @@ __global__ __launch_bounds__(64 * WAVES, 1) void attn_bwd_dq_kernel(const BwdPar
   const bool colok = 4 * ch < D;
   float* const abase = P.dq_acc ? P.dq_acc + bb * L.a_sb + head * L.a_sh + 4 * ch : nullptr;
   uint16_t* const bbase = P.dq ? P.dq + bb * L.o_sb + head * L.o_sh + 4 * ch : nullptr;
-  // the accumulating modes read a group's prior values before its first store (one wait,
-  // not one memory round trip per row)
   const int mode = P.dq_mode;
   const bool rd = mode == RMX_GRAD_ACC_F32 || mode == RMX_GRAD_ACC_FINAL;
-  // the prior value is added: the store is a write (f32) or a conversion (16-bit)
-  const int wmode = mode == RMX_GRAD_ACC_F32 ? RMX_GRAD_WRITE_F32
-                    : mode == RMX_GRAD_ACC_FINAL ? RMX_GRAD_WRITE_BF16 : mode;
+  const bool w32 = mode == RMX_GRAD_WRITE_F32 || mode == RMX_GRAD_ACC_F32;
+  if (!rd) {  // a short loop (as the forward's)
+    float* ap = w32 ? abase + (int64_t)(qw0 + rr) * L.a_ss : nullptr;
+    uint16_t* bp = w32 ? nullptr : bbase + (int64_t)(qw0 + rr) * L.o_ss;
+    const int rows = colok ? sq - qw0 - rr : 0;
+#pragma unroll 4
+    for (int r = 0; r < 32; r += RPI) {
+      if (r >= rows) break;
+      const int row = r + rr;
+      const f32x4 v = *reinterpret_cast<const f32x4*>(stg + row * (HD * 4) + 16 * (ch ^ (row % CPR)));
+      if (w32) {
+        *reinterpret_cast<f32x4*>(ap) = v;
+        ap += RPI * L.a_ss;
+      } else {
+        u32x2 w;
+        w[0] = cvt_pk<DT>(v[0], v[1]);
+        w[1] = cvt_pk<DT>(v[2], v[3]);
+        *reinterpret_cast<u32x2*>(bp) = w;
+        bp += RPI * L.o_ss;
+      }
+    }
+    return;
+  }
+  // the accumulating modes read a group's prior values before its first store (one wait,
+  // not one memory round trip per row)
 #pragma unroll
   for (int g = 0; g < NI; g += GI) {
     f32x4 v[GI], prev[GI];
@@ -521,16 +541,23 @@ __global__ __launch_bounds__(64 * WAVES, 1) void attn_bwd_dq_kernel(const BwdPar
     for (int i = 0; i < GI; ++i) {
       const int row = RPI * (g + i) + rr, qq = qw0 + row;
       v[i] = *reinterpret_cast<const f32x4*>(stg + row * (HD * 4) + 16 * (ch ^ (row % CPR)));
-      prev[i] = rd && colok && qq < sq ? *reinterpret_cast<const f32x4*>(abase + (int64_t)qq * L.a_ss)
-                                       : f32x4{};
+      prev[i] = colok && qq < sq ? *reinterpret_cast<const f32x4*>(abase + (int64_t)qq * L.a_ss)
+                                 : f32x4{};
     }
 #pragma unroll
     for (int i = 0; i < GI; ++i) {
       const int qq = qw0 + RPI * (g + i) + rr;
       if (!colok || qq >= sq) continue;
-      if (rd) v[i] += prev[i];
-      grad_store4<DT>(wmode, abase ? abase + (int64_t)qq * L.a_ss : nullptr,
-                      bbase ? bbase + (int64_t)qq * L.o_ss : nullptr, v[i]);
+      v[i] += prev[i];
+      // the prior value is added: the store is a write (f32) or a conversion (16-bit)
+      if (w32) {
+        *reinterpret_cast<f32x4*>(abase + (int64_t)qq * L.a_ss) = v[i];
+      } else {
+        u32x2 w;
+        w[0] = cvt_pk<DT>(v[i][0], v[i][1]);
+        w[1] = cvt_pk<DT>(v[i][2], v[i][3]);
+        *reinterpret_cast<u32x2*>(bbase + (int64_t)qq * L.o_ss) = w;
+      }
     }
   }
 }
