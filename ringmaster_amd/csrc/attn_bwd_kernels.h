@@ -717,7 +717,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_kernel(const BwdParams p
 
   // ---- tile loads. Wave 0 first loads the tile's lse and delta, and under document masks
   // its queries' indices and documents (by LDS DMA too: as register loads their waits drained
-  // the tiles in flight, 7.96 against @ ms for 16384^2 unmasked pairs) (one dword per
+  // the tiles in flight, 7.96 against 7.56 ms for 16384^2 unmasked pairs) (one dword per
   // lane; rows past the end read 0, where Q and dO rows are 0 as well, so they
   // add nothing), then every wave its share of the Q and dO rows (instruction n
   // fills LDS bytes [1024 n, 1024 n + 1024), lane L row n*RPK + L/CH, swizzled

@@ -92,7 +92,7 @@ class _Ctx:
         self.P, self.b, self.hq, self.L, self.d = q.shape
         self.hkv = k.shape[2]
         self.half = self.L // 2
-        self.scale = scale
+        self.scale = float(scale)  # (a plan's key: by value, not a tensor by identity)
         self.doc = doc
         self.layout, self.causal = layout, causal
         self.window = None if window is None else [int(w) for w in window]

@@ -87,6 +87,23 @@ def test_ring_plans_follow_their_base_tensors(monkeypatch, layout, causal, docs,
                 assert ((ta[f] == 0) == (tc[f] == 0)).all(), f
 
 
+def test_ring_plans_take_the_scale_by_value(monkeypatch):
+    """A scale given as a tensor that the program changes in place: the second pass takes its
+    new value, and no plan keeps the tensor."""
+    q = torch.randn(2, 1, 2, 16, 64).to(torch.bfloat16)
+    scale = torch.tensor(0.125)
+    ops._plans.clear()
+
+    def scales():
+        calls = _recorded(monkeypatch, lambda: zigzag.ring_forward(q, q, q, scale))
+        return {abi.AttnLayout.from_buffer_copy(c[1]).scale for c in calls}
+
+    assert scales() == {0.125}
+    scale.mul_(2)
+    assert scales() == {0.25}
+    ops._plans.clear()
+
+
 def test_plans_are_bounded():
     ops._plans.clear()
     for i in range(ops.PLANS_MAX + 9):
