@@ -489,7 +489,7 @@ static int check_mamba_bwd(int32_t batch, int32_t T, int32_t nheads, int32_t hea
 size_t rmx_mamba2_cp_correction_bwd_workspace(int32_t batch, int32_t T, int32_t nheads,
                                               int32_t head_dim, int32_t ngroups, int32_t d_state) {
   if (check_mamba_bwd(batch, T, nheads, head_dim, ngroups, d_state)) return 0;
-  return rmx::mamba2_bwd_workspace(batch, T, nheads, head_dim, d_state);
+  return rmx::mamba2_bwd_workspace(batch, T, nheads, head_dim, ngroups, d_state);
 }
 
 // Shared argument checks of the two correction-backward entry points (1 = nothing to do).
@@ -520,7 +520,7 @@ int32_t rmx_mamba2_cp_correction_bwd(const uint16_t* gy, const float* ghf, const
                                 head_dim, ngroups, d_state);
   if (rc) return rc < 0 ? rc : RMX_OK;
   if (!workspace) return fail(RMX_EINVAL, "NULL workspace");
-  const size_t need = rmx::mamba2_bwd_workspace(batch, T, nheads, head_dim, d_state);
+  const size_t need = rmx::mamba2_bwd_workspace(batch, T, nheads, head_dim, ngroups, d_state);
   if (workspace_bytes < need)
     return fail(RMX_EINVAL, "workspace of %zu bytes is below the %zu required", workspace_bytes, need);
   return dev_status(rmx::launch_mamba2_correction_bwd(gy, ghf, C, cum_A, h_prev, seq_idx, gC, g_cumA,
@@ -540,7 +540,7 @@ int32_t rmx_mamba2_cp_correction_bwd_noalloc(const uint16_t* gy, const float* gh
   int rc = check_mamba_bwd_args(gy, ghf, C, cum_A, h_prev, gC, g_cumA, g_hprev, batch, T, nheads,
                                 head_dim, ngroups, d_state);
   if (rc) return rc < 0 ? rc : RMX_OK;
-  const size_t need = rmx::mamba2_bwd_workspace(batch, T, nheads, head_dim, d_state);
+  const size_t need = rmx::mamba2_bwd_workspace(batch, T, nheads, head_dim, ngroups, d_state);
   if (need > RMX_MAMBA2_BWD_SCRATCH_MAX)
     return fail(RMX_EINVAL,
                 "the shape needs a %zu-byte workspace, above the %zu bytes of the allocation-free "

@@ -13,7 +13,7 @@
 // row's last token starts a fresh sequence, :131). With P[t,h,n] = sum_d G[t,h,d]
 // H_in[h,d,n], both dC and the sum in dcumA are contractions of P:
 //   dC[t,g,n] = sum_{h in g} e[t,h] P[t,h,n],  sum_d G S = sum_n C[t,g(h),n] P[t,h,n].
-// Five launches:
+// Five launches (six where the dC kernel is split):
 //  1. prep: H_in^T split into three bf16 parts hi + mid + lo ([B,H,n,d]); then e
 //     transposed to [B,H,T] by a kernel of its own (64-token x 64-head tiles);
 //  2. unit kernel: per head slice of 64 channels walking a token block, the block's
@@ -49,10 +49,13 @@ struct MambaBwdArgs {
   uint16_t* ht_mid;
   uint16_t* ht_lo;
   float* eT;        // [B][H][T]
-  int batch, T, nheads, head_dim, ngroups, d_state, ntb;
+  float* cpart;     // [nhs][B][T][G][n] dC partials of the dC kernel's head splits (nhs > 1)
+  int batch, T, nheads, head_dim, ngroups, d_state;
+  int tpw, ntb;     // unit kernel: tokens per workgroup (a multiple of 32), token blocks
+  int nhs;          // dC kernel: head splits
 };
 
-constexpr int kMambaBwdTokensPerWg = 4096;  // unit kernel token block
+constexpr int kMambaBwdTokensPerWg = 4096;  // unit kernel token block of a full chip
 constexpr int kMambaBwdCTokens = 256;       // dC kernel token tile (8 waves x 32)
 
 // Chunk swizzle for LDS tiles read both row-wise (8 consecutive rows, one
@@ -158,7 +161,7 @@ __global__ __launch_bounds__(256) void mamba2_bwd_et_kernel(const MambaBwdArgs a
 // ---------------------------------------------------------------------------
 // 2. unit kernel. A unit is 64 channels of one head (head_dim 64: one head,
 // 128: half a head); a workgroup holds 4 units of heads in one C group and
-// walks kMambaBwdTokensPerWg tokens, 32 per step, with the forward's DMA rings
+// walks a.tpw tokens, 32 per step, with the forward's DMA rings
 // (C and aux shared, G per wave, two steps ahead). Per wave and step:
 //   dH^T partial (64 ch x N) += (G e)^T C  4 N/32 MFMAs per 16 tokens: A = G^T e
 //       split into hi/lo (transposed reads of the G stage), B = C (transposed
@@ -200,8 +203,8 @@ __global__ __launch_bounds__(256, 1) void mamba2_bwd_unit_kernel(const MambaBwdA
   const int uph = HD / SL, hpw = 4 / uph, h0 = 4 * ug / uph;
   const int unit = 4 * ug + wave, h = unit / uph, sl = unit % uph, hw = wave / uph;
   const int g = h0 / (H / G);
-  const int tbeg = tb * kMambaBwdTokensPerWg;
-  const int tend = tbeg + kMambaBwdTokensPerWg < T ? tbeg + kMambaBwdTokensPerWg : T;
+  const int tbeg = tb * a.tpw;
+  const int tend = tbeg + a.tpw < T ? tbeg + a.tpw : T;
   const int nstep = (tend - tbeg + 31) / 32;
   const int64_t HHD = (int64_t)H * HD;
 
@@ -353,7 +356,9 @@ __global__ __launch_bounds__(256) void mamba2_bwd_reduce_kernel(const MambaBwdAr
 //   q    += sum_n C P               (C of the lane's token and rows, registers)
 // and after a head's last chunk dcumA[t,h] = e q (both lane halves' rows). The next
 // chunk's H_in^T (shared) and G (per wave) tiles load by DMA during the current one,
-// its e (from the transposed eT rows) into registers.
+// its e (from the transposed eT rows) into registers. A chunk takes 3.2 us whatever the launch's
+// size, so with few token tiles the group's heads are split over nhs workgroups (the rule at
+// mamba2_bwd_plan), whose fp32 sums mamba2_bwd_cfold_kernel adds in order.
 template <int N>
 struct MambaBwdCCfg {
   static constexpr int NW = 8;                 // waves, 32 tokens each
@@ -378,9 +383,12 @@ __global__ __launch_bounds__(512, 1) void mamba2_bwd_c_kernel(const MambaBwdArgs
   const int nwg = gridDim.x;
   if ((nwg & 7) == 0) id = (id & 7) * (nwg >> 3) + (id >> 3);
   const int tt = id % ntt, rest = id / ntt;
-  const int g = rest % a.ngroups, bb = rest / a.ngroups;
+  const int sp = rest % a.nhs, gb = rest / a.nhs;
+  const int g = gb % a.ngroups, bb = gb / a.ngroups;
   const int T = a.T, H = a.nheads, HD = a.head_dim;
-  const int hpg = H / a.ngroups, cph = HD / 64, nchunk = hpg * cph;
+  const int hpg = H / a.ngroups, cph = HD / 64;
+  const int hbeg = hpg * sp / a.nhs, nchunk = (hpg * (sp + 1) / a.nhs - hbeg) * cph;
+  const int hfirst = g * hpg + hbeg;
   const int tid = threadIdx.x, lane = tid & 63, hl = lane >> 5, l32 = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int t0 = tt * kMambaBwdCTokens;
@@ -390,9 +398,9 @@ __global__ __launch_bounds__(512, 1) void mamba2_bwd_c_kernel(const MambaBwdArgs
 
   const i32x4 rG = make_rsrc(a.gy + (int64_t)bb * T * HHD, span_bytes(T, ostride, (int)(HHD * 2)));
   const uint32_t ldsH = lds_addr(sH), ldsG = lds_addr(sG + wave * 2 * GS);
-  // chunk j: head hg = g * hpg + j / cph, channels 64 (j % cph) .. + 63
+  // chunk j: head hg = hfirst + j / cph, channels 64 (j % cph) .. + 63
   auto issue = [&](int st, int j) __attribute__((always_inline)) {
-    const int hg = g * hpg + j / cph, c0 = 64 * (j % cph);
+    const int hg = hfirst + j / cph, c0 = 64 * (j % cph);
     const int64_t ho = ((int64_t)bb * H + hg) * N * HD + c0;
     const i32x4 rh = make_rsrc(a.ht_hi + ho, span_bytes(N, HD * 2, 128));
     const i32x4 rm = make_rsrc(a.ht_mid + ho, span_bytes(N, HD * 2, 128));
@@ -416,7 +424,7 @@ __global__ __launch_bounds__(512, 1) void mamba2_bwd_c_kernel(const MambaBwdArgs
   };
   // e of the lane's token for the head of chunk j (0 past the sequence end)
   auto load_e = [&](int j) __attribute__((always_inline)) -> float {
-    const float* et = a.eT + ((int64_t)bb * H + g * hpg + j / cph) * T;
+    const float* et = a.eT + ((int64_t)bb * H + hfirst + j / cph) * T;
     return t < T ? et[t] : 0.f;
   };
 
@@ -477,7 +485,7 @@ __global__ __launch_bounds__(512, 1) void mamba2_bwd_c_kernel(const MambaBwdArgs
     }
     if (j % cph == cph - 1) {  // the head's last chunk: dcumA of its tokens
       const float tot = q + xhalf(q);
-      if (hl == 0 && t < T) a.g_cumA[((int64_t)bb * T + t) * H + g * hpg + j / cph] = ecur * tot;
+      if (hl == 0 && t < T) a.g_cumA[((int64_t)bb * T + t) * H + hfirst + j / cph] = ecur * tot;
       q = 0.f;
     }
     ecur = enext;
@@ -485,7 +493,18 @@ __global__ __launch_bounds__(512, 1) void mamba2_bwd_c_kernel(const MambaBwdArgs
 
   // dC[b, t, g, n]: lane (hl, l32) reg r of nb = token 32 wave + l32,
   // n = 32 nb + 16 (r / 8) + 8 hl + r % 8 (sigma-permuted A rows)
-  if (t < T) {
+  if (t < T && a.nhs > 1) {
+    float* dst = a.cpart + ((((int64_t)sp * a.batch + bb) * T + t) * a.ngroups + g) * N + 8 * hl;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        f32x4 v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = acc[nb][4 * q4 + i];
+        *reinterpret_cast<f32x4*>(dst + 32 * nb + 16 * (q4 >> 1) + 4 * (q4 & 1)) = v;
+      }
+  } else if (t < T) {
     uint16_t* dst = a.gC + (((int64_t)bb * T + t) * a.ngroups + g) * N + 8 * hl;
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb)
@@ -497,6 +516,21 @@ __global__ __launch_bounds__(512, 1) void mamba2_bwd_c_kernel(const MambaBwdArgs
         *reinterpret_cast<bf16x8*>(dst + 32 * nb + 16 * half) = pack8_hw(v);
       }
   }
+}
+
+// dC = sum of the head splits' partials, 8 elements per thread; bound by its traffic
+__global__ __launch_bounds__(256) void mamba2_bwd_cfold_kernel(const MambaBwdArgs a, int64_t n) {
+  const int64_t i = 8 * ((int64_t)blockIdx.x * 256 + threadIdx.x);
+  if (i >= n) return;
+  f32x4 lo = *reinterpret_cast<const f32x4*>(a.cpart + i);
+  f32x4 hi = *reinterpret_cast<const f32x4*>(a.cpart + i + 4);
+#pragma unroll 4
+  for (int s = 1; s < a.nhs; ++s) {
+    lo += *reinterpret_cast<const f32x4*>(a.cpart + s * n + i);
+    hi += *reinterpret_cast<const f32x4*>(a.cpart + s * n + i + 4);
+  }
+  const float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+  *reinterpret_cast<bf16x8*>(a.gC + i) = pack8_hw(v);
 }
 
 // ---------------------------------------------------------------------------
@@ -531,10 +565,48 @@ hipError_t mamba2_bwd_scratch(void** out) {
   return hipSuccess;
 }
 
-size_t mamba2_bwd_workspace(int batch, int T, int nheads, int head_dim, int d_state) {
+// How a call's two MFMA kernels are cut, and the workspace that takes.
+struct MambaBwdPlan {
+  int tpw, ntb, nhs;
+  size_t bytes;
+};
+
+// Both kernels walk serially (the unit kernel its token block, the dC kernel its group's heads)
+// at one workgroup per CU, so a call with fewer workgroups than CUs is as slow as one that fills
+// the chip. Until there are 256 of them, the unit kernel's 4096-token blocks are halved (down to
+// 256 tokens: a block also writes a state's partial) and the dC kernel's heads split. Both
+// stop where the workspace would pass the allocation-free entry's array, which so takes every
+// shape that the whole cut fits.
+// Whole -> cut, us a backward (batch x T x heads x head dim, groups, d_state): 2x128x64x64, 1, 128
+// 195 -> 53; 8x1024x64x64, 1, 128 238 -> 103; 4x2048x16x128, 2, 64 114 -> 70; 2x4096x64x64, 2, 128
+// 264 -> 106; 8x4096x64x64, 1, 128 365 -> 299; 8x8192x64x64 fills the chip and stays whole (417).
+static MambaBwdPlan mamba2_bwd_plan(int batch, int T, int nheads, int head_dim, int ngroups,
+                                    int d_state) {
+  constexpr int kCu = 256;
   const size_t state = (size_t)batch * nheads * head_dim * d_state;
-  const size_t ntb = (size_t)((T + kMambaBwdTokensPerWg - 1) / kMambaBwdTokensPerWg);
-  return ntb * state * 4 + 3 * state * 2 + (size_t)batch * nheads * T * 4 + 256;
+  const size_t dc = (size_t)batch * T * ngroups * d_state;
+  auto bytes = [&](int64_t ntb, int64_t nhs) -> size_t {
+    return (size_t)ntb * state * 4 + 3 * state * 2 + (size_t)batch * nheads * T * 4 + 256 +
+           (nhs > 1 ? 16 + (size_t)nhs * dc * 4 : 0);
+  };
+  MambaBwdPlan p{kMambaBwdTokensPerWg, 0, 1, 0};
+  auto blocks = [&](int tpw) -> int { return (int)(((int64_t)T + tpw - 1) / tpw); };
+  const int64_t units = (int64_t)nheads * (head_dim / 64) / 4 * batch;
+  while (p.tpw > 256 && units * blocks(p.tpw) < kCu &&
+         bytes(blocks(p.tpw / 2), 1) <= RMX_MAMBA2_BWD_SCRATCH_MAX)
+    p.tpw /= 2;
+  p.ntb = blocks(p.tpw);
+  const int64_t wgs = (int64_t)((T + kMambaBwdCTokens - 1) / kMambaBwdCTokens) * ngroups * batch;
+  const int hpg = nheads / ngroups;
+  const int64_t want = wgs > 0 ? kCu / wgs : 1;
+  p.nhs = want < 2 || hpg < 2 ? 1 : want < hpg ? (int)want : hpg;
+  while (p.nhs > 1 && bytes(p.ntb, p.nhs) > RMX_MAMBA2_BWD_SCRATCH_MAX) --p.nhs;
+  p.bytes = bytes(p.ntb, p.nhs);
+  return p;
+}
+
+size_t mamba2_bwd_workspace(int batch, int T, int nheads, int head_dim, int ngroups, int d_state) {
+  return mamba2_bwd_plan(batch, T, nheads, head_dim, ngroups, d_state).bytes;
 }
 
 hipError_t launch_mamba2_correction_bwd(const uint16_t* gy, const float* ghf, const uint16_t* C,
@@ -544,7 +616,8 @@ hipError_t launch_mamba2_correction_bwd(const uint16_t* gy, const float* ghf, co
                                         int nheads, int head_dim, int ngroups, int d_state,
                                         hipStream_t stream) {
   const size_t state = (size_t)batch * nheads * head_dim * d_state;
-  const int ntb = (T + kMambaBwdTokensPerWg - 1) / kMambaBwdTokensPerWg;
+  const MambaBwdPlan p = mamba2_bwd_plan(batch, T, nheads, head_dim, ngroups, d_state);
+  const int ntb = p.ntb;
   uint8_t* ws = reinterpret_cast<uint8_t*>(((uintptr_t)workspace + 255) & ~(uintptr_t)255);
   MambaBwdArgs a{gy, ghf, C, cum_A, h_prev, seq_idx, gC, g_cumA, g_hprev,
                  reinterpret_cast<float*>(ws),
@@ -552,7 +625,11 @@ hipError_t launch_mamba2_correction_bwd(const uint16_t* gy, const float* ghf, co
                  reinterpret_cast<uint16_t*>(ws + ntb * state * 4 + state * 2),
                  reinterpret_cast<uint16_t*>(ws + ntb * state * 4 + state * 4),
                  reinterpret_cast<float*>(ws + ntb * state * 4 + state * 6),
-                 batch, T, nheads, head_dim, ngroups, d_state, ntb};
+                 nullptr, batch, T, nheads, head_dim, ngroups, d_state, p.tpw, ntb, p.nhs};
+  const int64_t dc = (int64_t)batch * T * ngroups * d_state;
+  if (p.nhs > 1)
+    a.cpart = reinterpret_cast<float*>(
+        ((uintptr_t)(a.eT + (size_t)batch * nheads * T) + 15) & ~(uintptr_t)15);
   const int uph = head_dim / 64, nug = nheads * uph / 4;
   const int ntt = (T + kMambaBwdCTokens - 1) / kMambaBwdCTokens;
   auto run = [&](auto hd, auto n) {
@@ -563,8 +640,11 @@ hipError_t launch_mamba2_correction_bwd(const uint16_t* gy, const float* ghf, co
     hipLaunchKernelGGL((mamba2_bwd_unit_kernel<Nc>), dim3((unsigned)(nug * ntb * batch)), dim3(256), 0,
                        stream, a, nug);
     // the dC kernel writes dcumA, to which the reduce then adds the state term
-    hipLaunchKernelGGL((mamba2_bwd_c_kernel<Nc>), dim3((unsigned)(ntt * ngroups * batch)),
+    hipLaunchKernelGGL((mamba2_bwd_c_kernel<Nc>), dim3((unsigned)(ntt * ngroups * batch * a.nhs)),
                        dim3(64 * MambaBwdCCfg<Nc>::NW), 0, stream, a, ntt);
+    if (a.nhs > 1)
+      hipLaunchKernelGGL(mamba2_bwd_cfold_kernel, dim3((unsigned)((dc / 8 + 255) / 256)), dim3(256), 0,
+                         stream, a, dc);
     hipLaunchKernelGGL((mamba2_bwd_reduce_kernel<HDc, Nc>), dim3(nheads, batch), dim3(256), 0, stream, a);
     return hipGetLastError();
   };
