@@ -28,7 +28,7 @@
 extern "C" {
 #endif
 
-#define RMX_ABI_VERSION 18 /* 3: Mamba2 correction bwd; 4: nlse; 5: CP conv1d; 6: dt cumsum;
+#define RMX_ABI_VERSION 19 /* 3: Mamba2 correction bwd; 4: nlse; 5: CP conv1d; 6: dt cumsum;
                               7: effective dt in/out of the dt cumsum, shard final state;
                               8: allocation-free Mamba2 correction bwd;
                               9: carried-in state h_in / dh_in of the linear scan;
@@ -41,9 +41,9 @@ extern "C" {
                               16: per-batch-row document metadata (layout m_sb),
                                   dropout with document masks;
                               17: rmx_linear_scan_status;
-                              18: right-bounded windows (problem window_right), and since,
-                                  as additions: rmx_mamba2_dt_cumsum_state_bwd,
-                                  rmx_attn_bwd_ws, rmx_cast_half */
+                              18: right-bounded windows (problem window_right);
+                              19: rmx_attn_bwd_workspace, rmx_attn_bwd_ws, rmx_cast_half,
+                                  rmx_mamba2_dt_cumsum_state_bwd */
 
 /* error codes */
 #define RMX_OK 0

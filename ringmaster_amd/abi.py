@@ -17,7 +17,7 @@ from pathlib import Path
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libringmaster_amd.so"
-ABI_VERSION = 18  # RMX_ABI_VERSION of include/ringmaster_amd.h
+ABI_VERSION = 19  # RMX_ABI_VERSION of include/ringmaster_amd.h
 
 RMX_OK = 0
 RMX_EINVAL = -1
@@ -144,12 +144,13 @@ def lib() -> ctypes.CDLL:
                         f"ringmaster_amd native library missing ({LIB_PATH}); build it with "
                         "`python -c 'import __graft_entry__ as g; g.build()'`")
                 handle = ctypes.CDLL(str(LIB_PATH))
+                # before any other symbol: an older library may lack some
+                if handle.rmx_abi_version() != ABI_VERSION:
+                    raise RuntimeError("ringmaster_amd ABI version mismatch")
                 for name, (res, args) in SIGNATURES.items():
                     fn = getattr(handle, name)
                     fn.restype = res
                     fn.argtypes = args
-                if handle.rmx_abi_version() != ABI_VERSION:
-                    raise RuntimeError("ringmaster_amd ABI version mismatch")
                 _lib = handle
     return _lib
 

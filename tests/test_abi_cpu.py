@@ -30,8 +30,22 @@ def test_library_exports_every_declared_symbol():
 
 def test_abi_version_and_error_string():
     lib = abi.lib()
-    assert lib.rmx_abi_version() == abi.ABI_VERSION == 18
+    assert lib.rmx_abi_version() == abi.ABI_VERSION == 19
     assert isinstance(lib.rmx_last_error(), bytes)
+
+
+def test_older_library_is_refused_by_its_version(monkeypatch):
+    """A library of the version before, without the symbols added since: the error names the
+    version, not the first symbol that is missing."""
+    class Older:
+        @staticmethod
+        def rmx_abi_version():
+            return 18
+
+    monkeypatch.setattr(abi, "_lib", None)
+    monkeypatch.setattr(abi.ctypes, "CDLL", lambda path: Older())
+    with pytest.raises(RuntimeError, match="version"):
+        abi.lib()
 
 
 def _layout(**kw):
