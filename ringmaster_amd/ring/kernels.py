@@ -147,6 +147,12 @@ def _drop_of(dropout):
     return float(dropout[0]), int(dropout[1]) & _M64
 
 
+def _by_value(scale, window):
+    """A block's scale and window bound as numbers: a plan's key holds them by value, where a
+    tensor that the program changes in place would stand for its old value."""
+    return float(scale), None if window is None else int(window)
+
+
 def block_forward(q, k, v, scale: float, causal: bool, keep_f32: bool = False, window=None,
                   dropout=None, right=None):
     """(out [b, sq, hq, d] in q's dtype, lse fp32 [b, hq, sq]) of one block; with ``keep_f32`` also
@@ -159,6 +165,7 @@ def block_forward(q, k, v, scale: float, causal: bool, keep_f32: bool = False, w
     out32 = torch.empty((b, sq, hq, d), dtype=torch.float32, device=q.device) if keep_f32 else None
     mask, shift = _mask_of(causal, right)
     p, seed = _drop_of(dropout)
+    scale, window = _by_value(scale, window)
     bases = dict(q=q, k=k, v=v, out=out, lse=lse, acc_out=out32)
     plan = ops.plan(
         ("block_fwd", mask, shift, window, scale, p, keep_f32, ops.signature(q, k, v)),
@@ -189,6 +196,7 @@ def block_backward(dout, q, k, v, out, lse, scale: float, causal: bool, dq=None,
     dv_t = dv if (dv is not None and dv.stride() == dk_t.stride()) else torch.empty_like(dk_t)
     mask, shift = _mask_of(causal, right)
     p, seed = _drop_of(dropout)
+    scale, window = _by_value(scale, window)
     bases = dict(q=q, k=k, v=v, dout=dout, lse=lse, delta=delta, nlse=nlse, dq=dq_t, dk=dk_t, dv=dv_t)
     plan = ops.plan(
         ("block_bwd", mask, shift, window, scale, p,

@@ -104,6 +104,30 @@ def test_ring_plans_take_the_scale_by_value(monkeypatch):
     ops._plans.clear()
 
 
+def test_block_plans_take_scale_and_window_by_value(monkeypatch):
+    """The same of a block's scale and window bound, forward and backward."""
+    from ringmaster_amd.ring.kernels import block_backward, block_forward
+
+    q = torch.randn(1, 16, 2, 64).to(torch.bfloat16)
+    scale, window = torch.tensor(0.125), torch.tensor(5)
+    ops._plans.clear()
+
+    def seen():
+        def passes():
+            out, lse = block_forward(q, q, q, scale, True, window=window)
+            block_backward(q, q, q, q, out, lse, scale, True, window=window)
+
+        return {(abi.AttnLayout.from_buffer_copy(c[1]).scale,
+                 (abi.FwdProblem if c[0] == "fwd" else abi.BwdProblem).from_buffer_copy(c[2]).window_left)
+                for c in _recorded(monkeypatch, passes)}
+
+    assert seen() == {(0.125, 5)}
+    scale.mul_(2)
+    window.add_(4)
+    assert seen() == {(0.25, 9)}
+    ops._plans.clear()
+
+
 def test_plans_are_bounded():
     ops._plans.clear()
     for i in range(ops.PLANS_MAX + 9):
