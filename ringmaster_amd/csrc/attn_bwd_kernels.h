@@ -1916,14 +1916,15 @@ static hipError_t launch_dq(BwdParams& prm, int n, hipStream_t stream) {
   const rmx_attn_layout& L = prm.L;
   int ntile[RMX_MAX_BATCHED];
   for (int i = 0; i < n; ++i) ntile[i] = (prm.P[i].sq + C::BQ - 1) / C::BQ;
-  const dim3 grid(plan_workgroups(prm.map, n, L.batch * L.hq, L.hq / L.hkv, ntile,
-                                  L.mask == RMX_MASK_CAUSAL));
+  const int grid = plan_workgroups(prm.map, n, L.batch * L.hq, L.hq / L.hkv, ntile,
+                                   L.mask == RMX_MASK_CAUSAL);
+  if (grid == 0) return hipSuccess;  // an empty batch
   if (L.mask == RMX_MASK_CAUSAL)
-    hipLaunchKernelGGL((attn_bwd_dq_kernel<HD, WAVES, RMX_MASK_CAUSAL, DT, DROP>), grid, dim3(C::NT), 0, stream, prm);
+    hipLaunchKernelGGL((attn_bwd_dq_kernel<HD, WAVES, RMX_MASK_CAUSAL, DT, DROP>), dim3(grid), dim3(C::NT), 0, stream, prm);
   else if (L.mask == RMX_MASK_DOC)
-    hipLaunchKernelGGL((attn_bwd_dq_kernel<HD, WAVES, RMX_MASK_DOC, DT, DROP>), grid, dim3(C::NT), 0, stream, prm);
+    hipLaunchKernelGGL((attn_bwd_dq_kernel<HD, WAVES, RMX_MASK_DOC, DT, DROP>), dim3(grid), dim3(C::NT), 0, stream, prm);
   else
-    hipLaunchKernelGGL((attn_bwd_dq_kernel<HD, WAVES, RMX_MASK_FULL, DT, DROP>), grid, dim3(C::NT), 0, stream, prm);
+    hipLaunchKernelGGL((attn_bwd_dq_kernel<HD, WAVES, RMX_MASK_FULL, DT, DROP>), dim3(grid), dim3(C::NT), 0, stream, prm);
   return hipGetLastError();
 }
 

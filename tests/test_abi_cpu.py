@@ -421,3 +421,24 @@ def test_window_bounds_keep_the_flash_pairs():
                     mask2, shift2 = _mask_of(causal, right2)
                     got2 = _band(sq, sk, False, left2, shift2 if mask2 == abi.MASK_CAUSAL else None)
                     assert torch.equal(got2, ref), (sq, sk, causal, w)
+
+
+@pytest.mark.parametrize("head_dim", [64, 128, 256])
+def test_empty_batch_launches_nothing(head_dim):
+    """batch 0 with tensors in hand is a call with nothing to do, forward and backward."""
+    lay = _layout(batch=0, head_dim=head_dim)
+    for name in ("q", "k", "v", "o", "dk", "a", "ka"):
+        for s in ("sb", "ss", "sh"):
+            setattr(lay, f"{name}_{s}", 1024)
+    lib, at = abi.lib(), 1 << 20  # an address, never read
+    fwd, bwd = (abi.FwdProblem * 1)(), (abi.BwdProblem * 1)()
+    for p in (fwd[0], bwd[0]):
+        for field, kind in p._fields_:
+            if kind is ctypes.c_void_p:
+                setattr(p, field, at)
+        p.sq, p.sk = 300, 200
+    fwd[0].mode = abi.FWD_WRITE
+    bwd[0].dq_mode = bwd[0].dkv_mode = abi.GRAD_WRITE_BF16
+    assert lib.rmx_attn_fwd(ctypes.byref(lay), fwd, 1, None) == abi.RMX_OK
+    assert lib.rmx_attn_bwd(ctypes.byref(lay), bwd, 1, None) == abi.RMX_OK
+    assert lib.rmx_attn_bwd_ws(ctypes.byref(lay), bwd, 1, at, 0, None) == abi.RMX_OK
