@@ -28,7 +28,7 @@
 extern "C" {
 #endif
 
-#define RMX_ABI_VERSION 19 /* 3: Mamba2 correction bwd; 4: nlse; 5: CP conv1d; 6: dt cumsum;
+#define RMX_ABI_VERSION 20 /* 3: Mamba2 correction bwd; 4: nlse; 5: CP conv1d; 6: dt cumsum;
                               7: effective dt in/out of the dt cumsum, shard final state;
                               8: allocation-free Mamba2 correction bwd;
                               9: carried-in state h_in / dh_in of the linear scan;
@@ -43,7 +43,9 @@ extern "C" {
                               17: rmx_linear_scan_status;
                               18: right-bounded windows (problem window_right);
                               19: rmx_attn_bwd_workspace, rmx_attn_bwd_ws, rmx_cast_half,
-                                  rmx_mamba2_dt_cumsum_state_bwd */
+                                  rmx_mamba2_dt_cumsum_state_bwd;
+                              20: rmx_mamba2_dt_cumsum_bwd_workspace,
+                                  rmx_mamba2_dt_cumsum_bwd_ws */
 
 /* error codes */
 #define RMX_OK 0
@@ -443,6 +445,23 @@ int32_t rmx_mamba2_dt_cumsum_state_bwd(const void* dt, int32_t dt_is_f32, const 
                                        const float* g_e, float* g_dt, float* g_A,
                                        float* g_dt_bias, int32_t rows, int32_t T, int32_t nheads,
                                        void* stream);
+
+/*
+ * Both of the above (state = 0 or 1; with 1, g_decay is NULL) with device memory for the partial
+ * sums of dL/dA and dL/ddt_bias: those are then added in a fixed order and a call on zeroed
+ * outputs repeats bit for bit, where the forms above repeat for one or two rows only (and walk
+ * such a row's tokens in one workgroup per 64 heads). rmx_mamba2_dt_cumsum_bwd_workspace
+ * returns the bytes the call can use (0: none); the workspace (nullable, 16-byte aligned) is
+ * scratch of this call, its contents on entry do not matter, and one smaller than that is not
+ * used. No counterpart in the reference.
+ */
+size_t rmx_mamba2_dt_cumsum_bwd_workspace(int32_t rows, int32_t T, int32_t nheads);
+int32_t rmx_mamba2_dt_cumsum_bwd_ws(const void* dt, int32_t dt_is_f32, const float* dt_bias,
+                                    const float* A, int32_t dt_softplus, const float* g_cum_A,
+                                    const float* g_e, const float* g_decay, const float* decay,
+                                    float* g_dt, float* g_A, float* g_dt_bias, int32_t rows,
+                                    int32_t T, int32_t nheads, int32_t state, void* workspace,
+                                    size_t workspace_bytes, void* stream);
 
 /*
  * Mamba2 shard final state from x, B and dt: the final_states of mamba-ssm's

@@ -17,7 +17,7 @@ from pathlib import Path
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libringmaster_amd.so"
-ABI_VERSION = 19  # RMX_ABI_VERSION of include/ringmaster_amd.h
+ABI_VERSION = 20  # RMX_ABI_VERSION of include/ringmaster_amd.h
 
 RMX_OK = 0
 RMX_EINVAL = -1
@@ -122,6 +122,9 @@ SIGNATURES = {
                                  + [_i32, _i32, _i32, _vp]),
     "rmx_mamba2_dt_cumsum_state_bwd": (_i32, [_vp, _i32, _vp, _vp, _i32] + [_vp] * 5
                                        + [_i32, _i32, _i32, _vp]),
+    "rmx_mamba2_dt_cumsum_bwd_workspace": (ctypes.c_size_t, [_i32] * 3),
+    "rmx_mamba2_dt_cumsum_bwd_ws": (_i32, [_vp, _i32, _vp, _vp, _i32] + [_vp] * 7
+                                    + [_i32, _i32, _i32, _i32, _vp, ctypes.c_size_t, _vp]),
     "rmx_mamba2_chunk_state": (_i32, [_vp] * 6 + [_i32] * 6 + [_vp]),
     "rmx_mamba2_chunk_state_bwd_workspace": (ctypes.c_size_t, [_i32] * 4),
     "rmx_mamba2_chunk_state_bwd": (_i32, [_vp] * 10 + [_i32] * 6 + [_vp, ctypes.c_size_t, _vp]),

@@ -596,16 +596,38 @@ static int dt_cumsum_bwd(const void* dt, int32_t dt_is_f32, const float* dt_bias
                          int32_t dt_softplus, const float* g_cum_A, const float* g_e,
                          const float* g_decay, const float* decay, float* g_dt, float* g_A,
                          float* g_dt_bias, int32_t rows, int32_t T, int32_t nheads, int closed,
-                         void* stream, const char* what) {
+                         void* workspace, size_t workspace_bytes, void* stream, const char* what) {
   int rc = check_dt(dt, dt_is_f32, A, dt_softplus, rows, T, nheads);
   if (rc) return rc;
   if ((int64_t)rows * T * nheads == 0) return RMX_OK;
-  if (!g_dt || !g_A || (g_decay && !decay)) return fail(RMX_EINVAL, "NULL tensor pointer");
-  return dev_status(rmx::launch_mamba2_dt_cumsum_bwd(dt, dt_is_f32, dt_bias, A, dt_softplus,
-                                                     g_cum_A, g_e, g_decay, decay, g_dt, g_A,
-                                                     g_dt_bias, rows, T, nheads, closed,
-                                                     (hipStream_t)stream),
+  if (!g_dt || !g_A || (g_decay && !decay) || (closed && (!g_cum_A || !g_e)))
+    return fail(RMX_EINVAL, "NULL tensor pointer");
+  if (workspace && !aligned(workspace, 16))
+    return fail(RMX_EINVAL, "workspace must be 16-byte aligned");
+  const size_t need = rmx::mamba2_dt_bwd_workspace(rows, T, nheads);
+  return dev_status(rmx::launch_mamba2_dt_cumsum_bwd(
+                        dt, dt_is_f32, dt_bias, A, dt_softplus, g_cum_A, g_e, g_decay, decay, g_dt,
+                        g_A, g_dt_bias, rows, T, nheads, closed,
+                        need && workspace_bytes >= need ? workspace : nullptr, (hipStream_t)stream),
                     what);
+}
+
+size_t rmx_mamba2_dt_cumsum_bwd_workspace(int32_t rows, int32_t T, int32_t nheads) {
+  if (rows <= 0 || T <= 0 || nheads <= 0) return 0;
+  return rmx::mamba2_dt_bwd_workspace(rows, T, nheads);
+}
+
+int32_t rmx_mamba2_dt_cumsum_bwd_ws(const void* dt, int32_t dt_is_f32, const float* dt_bias,
+                                    const float* A, int32_t dt_softplus, const float* g_cum_A,
+                                    const float* g_e, const float* g_decay, const float* decay,
+                                    float* g_dt, float* g_A, float* g_dt_bias, int32_t rows,
+                                    int32_t T, int32_t nheads, int32_t state, void* workspace,
+                                    size_t workspace_bytes, void* stream) {
+  if (state != 0 && state != 1) return fail(RMX_EINVAL, "state must be 0 or 1");
+  if (state && g_decay) return fail(RMX_EINVAL, "the state form takes no decay gradient");
+  return dt_cumsum_bwd(dt, dt_is_f32, dt_bias, A, dt_softplus, g_cum_A, g_e, g_decay, decay, g_dt,
+                       g_A, g_dt_bias, rows, T, nheads, state, workspace, workspace_bytes, stream,
+                       "rmx_mamba2_dt_cumsum_bwd_ws launch");
 }
 
 int32_t rmx_mamba2_dt_cumsum_bwd(const void* dt, int32_t dt_is_f32, const float* dt_bias,
@@ -614,7 +636,7 @@ int32_t rmx_mamba2_dt_cumsum_bwd(const void* dt, int32_t dt_is_f32, const float*
                                  float* g_dt, float* g_A, float* g_dt_bias, int32_t rows,
                                  int32_t T, int32_t nheads, void* stream) {
   return dt_cumsum_bwd(dt, dt_is_f32, dt_bias, A, dt_softplus, g_cum_A, g_e, g_decay, decay, g_dt,
-                       g_A, g_dt_bias, rows, T, nheads, 0, stream,
+                       g_A, g_dt_bias, rows, T, nheads, 0, nullptr, 0, stream,
                        "rmx_mamba2_dt_cumsum_bwd launch");
 }
 
@@ -623,10 +645,8 @@ int32_t rmx_mamba2_dt_cumsum_state_bwd(const void* dt, int32_t dt_is_f32, const 
                                        const float* g_e, float* g_dt, float* g_A,
                                        float* g_dt_bias, int32_t rows, int32_t T, int32_t nheads,
                                        void* stream) {
-  if ((int64_t)rows * T * nheads > 0 && (!g_cum_A || !g_e))
-    return fail(RMX_EINVAL, "NULL tensor pointer");
   return dt_cumsum_bwd(dt, dt_is_f32, dt_bias, A, dt_softplus, g_cum_A, g_e, nullptr, nullptr, g_dt,
-                       g_A, g_dt_bias, rows, T, nheads, 1, stream,
+                       g_A, g_dt_bias, rows, T, nheads, 1, nullptr, 0, stream,
                        "rmx_mamba2_dt_cumsum_state_bwd launch");
 }
 

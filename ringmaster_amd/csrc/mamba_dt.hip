@@ -16,9 +16,11 @@
 //     every other token plus the last token of the chunk before;
 //   backward: chunk sums of g_cum into g_dt at each chunk's first token / those turned into
 //     what enters each chunk / the chunks, each reading its own first token before the
-//     barrier that precedes its stores.
+//     barrier that precedes its stores; with a workspace they leave their parts of dA and
+//     d(bias) there and a fourth launch adds those in order (see mamba2_dt_fold_kernel).
 // A sequence of one chunk is one launch. At 8 rows x 8192 x 64 the three launches take 19 + 5 + 9
-// us forward and 5 + 5 + 29 us backward, 25 MB and 42 MB moved by the first and the last of these;
+// us forward and the four 4 + 5 + 24 + 4 us backward, 25 MB and 42 MB moved by the first and the
+// third of these;
 // cum_A's rms error falls from 1e-6 to 6e-8 (shorter chains of sums).
 #include "rmx_kernels.h"
 
@@ -39,6 +41,7 @@ struct DtArgs {
   float* g_dt;           // bwd out [rows, T, H] (fp32)
   float* g_A;            // bwd += [H]
   float* g_bias;         // bwd += [H] (softplus only) or null
+  float* part;           // bwd workspace or null: dA and d(bias) parts [2][rows * nchunk][H]
   int rows, T, H;
   int nchunk;
 };
@@ -83,10 +86,10 @@ struct DtPos {
   int row, h, s, c, n;
   bool hv;
   int64_t t0, base;  // element of (row, t0, h)
-  __device__ __forceinline__ explicit DtPos(const DtArgs& a) {
+  // of workgroup rb (row, head block) and chunk ci
+  __device__ __forceinline__ DtPos(const DtArgs& a, int rb, int ci) {
     const int hb = (a.H + HT - 1) / HT;
-    c = blockIdx.x % a.nchunk;
-    const int rb = blockIdx.x / a.nchunk;
+    c = ci;
     row = rb / hb;
     h = (rb % hb) * HT + (int)(threadIdx.x % HT);
     s = threadIdx.x / HT;
@@ -95,6 +98,8 @@ struct DtPos {
     n = !hv || t0 >= a.T ? 0 : (a.T - t0 < kDtRun ? (int)(a.T - t0) : kDtRun);
     base = ((int64_t)row * a.T + t0) * a.H + h;
   }
+  __device__ __forceinline__ explicit DtPos(const DtArgs& a)
+      : DtPos(a, blockIdx.x / a.nchunk, blockIdx.x % a.nchunk) {}
 };
 
 // sum of the values of the runs before s (or after s) at this thread's head
@@ -227,21 +232,11 @@ __global__ __launch_bounds__(kDtThreads) void mamba2_dt_sums_kernel(const DtArgs
 // the small R of early tokens keep their precision;
 // g_e_s = A R_s (+ the direct g_e_s);  g_A += sum_s R_s e_s;  g_dt_s = g_e_s softplus'(dt_s + bias)
 // (or g_e_s);  g_bias += sum_s g_dt_s (softplus only).
+// One chunk, `in` entering it: g_dt of the thread's run and its parts of g_A and g_bias, added to
+// pa and pb.
 template <int HT, bool CLOSED>
-__global__ __launch_bounds__(kDtThreads) void mamba2_dt_bwd_kernel(const DtArgs a) {
-  __shared__ float part[DtCfg<HT>::NS][HT];
-  __shared__ float red[2][DtCfg<HT>::NS][HT];
-  const DtPos<HT> p(a);
-  const int col = threadIdx.x % HT;
-  const float Ah = p.hv ? a.A[p.h] : 0.f;
-  const float bh = (p.hv && a.bias) ? a.bias[p.h] : 0.f;
-  float in = 0.f;  // what enters the chunk
-  if (p.hv) {
-    if (a.nchunk > 1 && a.g_cum)
-      in = a.g_dt[((int64_t)p.row * a.T + (int64_t)p.c * DtCfg<HT>::CT) * a.H + p.h];
-    else if (!CLOSED && a.g_decay)
-      in = a.g_decay[(int64_t)p.row * a.H + p.h] * a.decay[(int64_t)p.row * a.H + p.h];
-  }
+__device__ __forceinline__ void dt_bwd_chunk(const DtArgs& a, const DtPos<HT>& p, float Ah, float bh,
+                                             float in, float (*part)[HT], float& pa, float& pb) {
   float g[kDtRun], x[kDtRun], d[kDtRun];
 #pragma unroll
   for (int i = 0; i < kDtRun; ++i) {
@@ -265,10 +260,9 @@ __global__ __launch_bounds__(kDtThreads) void mamba2_dt_bwd_kernel(const DtArgs 
       g[i] = run;
     }
   }
-  part[p.s][col] = run;
+  part[p.s][threadIdx.x % HT] = run;
   __syncthreads();  // (also: every thread has read the chunk's first g_dt)
   in += dt_other_runs<HT, !CLOSED>(part, p.s);
-  float pa = 0.f, pb = 0.f;
 #pragma unroll
   for (int i = 0; i < kDtRun; ++i) {
     const float R = in + g[i], y = x[i] + bh;
@@ -287,13 +281,103 @@ __global__ __launch_bounds__(kDtThreads) void mamba2_dt_bwd_kernel(const DtArgs 
       a.g_dt[p.base + (int64_t)i * a.H] = gdt;
     }
   }
-  red[0][p.s][col] = pa;
-  red[1][p.s][col] = pb;
+}
+
+// The runs' sums of g_A and g_bias at this thread's head, valid in run 0.
+template <int HT>
+__device__ __forceinline__ void dt_runs_total(float (*red)[DtCfg<HT>::NS][HT], int s, float& pa,
+                                              float& pb) {
+  const int col = threadIdx.x % HT;
+  red[0][s][col] = pa;
+  red[1][s][col] = pb;
   __syncthreads();
-  if (p.s == 0 && p.hv) {
-    atomicAdd(a.g_A + p.h, pa + dt_other_runs<HT, true>(red[0], 0));
-    if (a.softplus && a.g_bias) atomicAdd(a.g_bias + p.h, pb + dt_other_runs<HT, true>(red[1], 0));
+  if (s == 0) {
+    pa += dt_other_runs<HT, true>(red[0], 0);
+    pb += dt_other_runs<HT, true>(red[1], 0);
   }
+}
+
+template <int HT, bool CLOSED>
+__global__ __launch_bounds__(kDtThreads) void mamba2_dt_bwd_kernel(const DtArgs a) {
+  __shared__ float part[DtCfg<HT>::NS][HT];
+  __shared__ float red[2][DtCfg<HT>::NS][HT];
+  const DtPos<HT> p(a);
+  const float Ah = p.hv ? a.A[p.h] : 0.f;
+  const float bh = (p.hv && a.bias) ? a.bias[p.h] : 0.f;
+  float in = 0.f;  // what enters the chunk
+  if (p.hv) {
+    if (a.nchunk > 1 && a.g_cum)
+      in = a.g_dt[((int64_t)p.row * a.T + (int64_t)p.c * DtCfg<HT>::CT) * a.H + p.h];
+    else if (!CLOSED && a.g_decay)
+      in = a.g_decay[(int64_t)p.row * a.H + p.h] * a.decay[(int64_t)p.row * a.H + p.h];
+  }
+  float pa = 0.f, pb = 0.f;
+  dt_bwd_chunk<HT, CLOSED>(a, p, Ah, bh, in, part, pa, pb);
+  dt_runs_total<HT>(red, p.s, pa, pb);
+  if (p.s != 0 || !p.hv) return;
+  const bool gb = a.softplus && a.g_bias;
+  if (a.part) {
+    const int64_t n = (int64_t)a.rows * a.nchunk, at = ((int64_t)p.row * a.nchunk + p.c) * a.H + p.h;
+    a.part[at] = pa;
+    if (gb) a.part[n * a.H + at] = pb;
+  } else {
+    atomicAdd(a.g_A + p.h, pa);
+    if (gb) atomicAdd(a.g_bias + p.h, pb);
+  }
+}
+
+// One workgroup walks all chunks of a row, so that each head's dA and d(bias) are one sum.
+template <int HT, bool CLOSED>
+__global__ __launch_bounds__(kDtThreads) void mamba2_dt_bwd_serial_kernel(const DtArgs a) {
+  __shared__ float part[DtCfg<HT>::NS][HT];
+  __shared__ float red[2][DtCfg<HT>::NS][HT];
+  const DtPos<HT> p0(a, blockIdx.x, 0);
+  const float Ah = p0.hv ? a.A[p0.h] : 0.f;
+  const float bh = (p0.hv && a.bias) ? a.bias[p0.h] : 0.f;
+  float in = 0.f;
+  if (!CLOSED && p0.hv && a.g_decay)
+    in = a.g_decay[(int64_t)p0.row * a.H + p0.h] * a.decay[(int64_t)p0.row * a.H + p0.h];
+  float pa = 0.f, pb = 0.f;
+  for (int i = 0; i < a.nchunk; ++i) {
+    const DtPos<HT> p(a, blockIdx.x, CLOSED ? i : a.nchunk - 1 - i);
+    dt_bwd_chunk<HT, CLOSED>(a, p, Ah, bh, in, part, pa, pb);
+    in += part[0][threadIdx.x % HT] + dt_other_runs<HT, true>(part, 0);
+    __syncthreads();  // the next chunk writes part
+  }
+  dt_runs_total<HT>(red, p0.s, pa, pb);
+  if (p0.s != 0 || !p0.hv) return;
+  atomicAdd(a.g_A + p0.h, pa);
+  if (a.softplus && a.g_bias) atomicAdd(a.g_bias + p0.h, pb);
+}
+
+// dA (blockIdx.y 0) and d(bias) (1) += the chunks' parts, in a fixed order, so that a call
+// repeats bit for bit: added by atomics, chunks arrive in any order. 16 heads by 64 shares of the
+// parts per workgroup. 512 parts of 64 heads: 4 us, and the chunk kernel, without the atomics
+// of 512 workgroups on 128 words, 24 us instead of 29.
+__global__ __launch_bounds__(1024) void mamba2_dt_fold_kernel(const DtArgs a) {
+  __shared__ float sum[64][16];
+  const int col = threadIdx.x % 16, share = threadIdx.x / 16;
+  const int h = blockIdx.x * 16 + col;
+  const int64_t n = (int64_t)a.rows * a.nchunk;
+  const float* x = a.part + blockIdx.y * n * a.H + h;
+  float v = 0.f;
+  if (h < a.H) {
+    const int64_t hi = n * (share + 1) / 64;
+#pragma unroll 8
+    for (int64_t i = n * share / 64; i < hi; ++i) v += x[i * a.H];
+  }
+  sum[share][col] = v;
+  __syncthreads();
+  if (share < 8) {
+    v = 0.f;
+    for (int i = 0; i < 8; ++i) v += sum[8 * share + i][col];
+  }
+  __syncthreads();
+  if (share < 8) sum[share][col] = v;
+  __syncthreads();
+  if (share || h >= a.H) return;
+  for (int i = 1; i < 8; ++i) v += sum[i][col];
+  atomicAdd((blockIdx.y ? a.g_bias : a.g_A) + h, v);
 }
 
 // ---------------------------------------------------------------- launchers
@@ -313,48 +397,71 @@ static void launch_dt_fwd(DtArgs a, hipStream_t stream) {
   hipLaunchKernelGGL((mamba2_dt_carry_kernel<HT>), dim3(grid), dim3(kDtThreads), 0, stream, a);
 }
 
+// Heads per workgroup: the least that covers H.
+static int dt_heads(int H) { return H <= 8 ? 8 : H <= 16 ? 16 : H <= 32 ? 32 : 64; }
+
+size_t mamba2_dt_bwd_workspace(int rows, int T, int H) {
+  const int64_t CT = kDtThreads / dt_heads(H) * kDtRun, nchunk = ((int64_t)T + CT - 1) / CT;
+  return nchunk > 1 ? (size_t)rows * nchunk * H * 8 : 0;
+}
+
 template <int HT, bool CLOSED>
 static void launch_dt_bwd(DtArgs a, hipStream_t stream) {
   const unsigned grid = (unsigned)dt_grid<HT>(a), rows = (unsigned)(a.rows * ((a.H + 63) / 64));
+  // Without a workspace the chunks' parts are added by atomics. One or two rows go chunk by
+  // chunk instead: with one sum per row and head they repeat bit for bit (two sums added to zero
+  // commute). 1 x 8192 x 64: 608 us (one workgroup),
+  // with the workspace 18.
+  if (a.nchunk > 1 && !a.part && a.rows <= 2) {
+    hipLaunchKernelGGL((mamba2_dt_bwd_serial_kernel<HT, CLOSED>), dim3(grid / a.nchunk),
+                       dim3(kDtThreads), 0, stream, a);
+    return;
+  }
   if (a.nchunk > 1 && a.g_cum) {
     hipLaunchKernelGGL((mamba2_dt_sums_kernel<HT>), dim3(grid), dim3(kDtThreads), 0, stream, a);
     hipLaunchKernelGGL((mamba2_dt_chunks_kernel<CLOSED ? kDtNegPrefix : kDtSuffix>), dim3(rows),
                        dim3(1024), 0, stream, a, a.g_dt, DtCfg<HT>::CT, 0);
   }
   hipLaunchKernelGGL((mamba2_dt_bwd_kernel<HT, CLOSED>), dim3(grid), dim3(kDtThreads), 0, stream, a);
+  if (a.part)
+    hipLaunchKernelGGL(mamba2_dt_fold_kernel, dim3((a.H + 15) / 16, a.softplus && a.g_bias ? 2 : 1),
+                       dim3(1024), 0, stream, a);
+}
+
+template <class F>
+static void by_heads(int H, F f) {
+  switch (dt_heads(H)) {
+    case 8: f(std::integral_constant<int, 8>{}); break;
+    case 16: f(std::integral_constant<int, 16>{}); break;
+    case 32: f(std::integral_constant<int, 32>{}); break;
+    default: f(std::integral_constant<int, 64>{});
+  }
 }
 
 hipError_t launch_mamba2_dt_cumsum(const void* dt, int dt_f32, const float* bias, const float* A,
                                    int softplus, float* cum_A, float* e, float* decay, int rows,
                                    int T, int H, hipStream_t stream) {
   const DtArgs a{dt, dt_f32, bias, A, softplus, cum_A, e, nullptr, decay, nullptr, nullptr, nullptr,
-                 nullptr, nullptr, rows, T, H, 0};
+                 nullptr, nullptr, nullptr, rows, T, H, 0};
   if ((int64_t)rows * T * H == 0) return hipSuccess;
-  if (H <= 8) launch_dt_fwd<8>(a, stream);
-  else if (H <= 16) launch_dt_fwd<16>(a, stream);
-  else if (H <= 32) launch_dt_fwd<32>(a, stream);
-  else launch_dt_fwd<64>(a, stream);
+  by_heads(H, [&](auto ht) { launch_dt_fwd<ht.value>(a, stream); });
   return hipGetLastError();
-}
-
-template <bool CLOSED>
-static void launch_dt_bwd_h(const DtArgs& a, hipStream_t stream) {
-  if (a.H <= 8) launch_dt_bwd<8, CLOSED>(a, stream);
-  else if (a.H <= 16) launch_dt_bwd<16, CLOSED>(a, stream);
-  else if (a.H <= 32) launch_dt_bwd<32, CLOSED>(a, stream);
-  else launch_dt_bwd<64, CLOSED>(a, stream);
 }
 
 hipError_t launch_mamba2_dt_cumsum_bwd(const void* dt, int dt_f32, const float* bias,
                                        const float* A, int softplus, const float* g_cum,
                                        const float* g_e, const float* g_decay, const float* decay,
                                        float* g_dt, float* g_A, float* g_bias, int rows, int T,
-                                       int H, int closed, hipStream_t stream) {
+                                       int H, int closed, void* ws, hipStream_t stream) {
   const DtArgs a{dt, dt_f32, bias, A, softplus, nullptr, nullptr, g_e, const_cast<float*>(decay),
-                 g_cum, g_decay, g_dt, g_A, g_bias, rows, T, H, 0};
+                 g_cum, g_decay, g_dt, g_A, g_bias, static_cast<float*>(ws), rows, T, H, 0};
   if ((int64_t)rows * T * H == 0) return hipSuccess;
-  if (closed) launch_dt_bwd_h<true>(a, stream);
-  else launch_dt_bwd_h<false>(a, stream);
+  by_heads(H, [&](auto ht) {
+    if (closed)
+      launch_dt_bwd<ht.value, true>(a, stream);
+    else
+      launch_dt_bwd<ht.value, false>(a, stream);
+  });
   return hipGetLastError();
 }
 

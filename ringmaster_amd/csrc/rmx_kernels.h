@@ -82,7 +82,8 @@ hipError_t launch_mamba2_dt_cumsum_bwd(const void* dt, int dt_f32, const float* 
                                        const float* A, int softplus, const float* g_cum,
                                        const float* g_e, const float* g_decay, const float* decay,
                                        float* g_dt, float* g_A, float* g_bias, int rows, int T,
-                                       int H, int closed, hipStream_t stream);
+                                       int H, int closed, void* ws, hipStream_t stream);
+size_t mamba2_dt_bwd_workspace(int rows, int T, int H);
 hipError_t launch_mamba2_chunk_state(const uint16_t* x, const uint16_t* B, const float* e,
                                      const float* cum_A, const int32_t* t0, float* state,
                                      int rows, int T, int H, int D, int G, int N,

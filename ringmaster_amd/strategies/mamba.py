@@ -142,6 +142,24 @@ def _dt_forward(dt, A, dt_bias, softplus, want_e):
     return cum, decay, e
 
 
+def _dt_backward(dt, A, dt_bias, softplus, g_cum, g_e, g_decay, decay, state):
+    """(g_dt in dt's type, g_A, g_bias or None) of ``_dt_forward``; ``state``: g_cum and g_e as the
+    shard state's backward leaves them."""
+    rows, T, H = dt.shape
+    g_dt = torch.empty((rows, T, H), dtype=torch.float32, device=dt.device)
+    g_A = torch.zeros(H, dtype=torch.float32, device=dt.device)
+    g_b = torch.zeros(H, dtype=torch.float32, device=dt.device) if dt_bias is not None else None
+    lib = abi.lib()
+    ws_bytes = lib.rmx_mamba2_dt_cumsum_bwd_workspace(rows, T, H)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dt.device) if ws_bytes else None
+    abi.check(lib.rmx_mamba2_dt_cumsum_bwd_ws(
+        dt.data_ptr(), int(dt.dtype == torch.float32), abi.ptr(dt_bias), A.data_ptr(),
+        int(softplus), abi.ptr(g_cum), abi.ptr(g_e), abi.ptr(g_decay), abi.ptr(decay),
+        g_dt.data_ptr(), g_A.data_ptr(), abi.ptr(g_b), rows, T, H, int(state), abi.ptr(ws),
+        ws_bytes, abi.stream_of(dt)))
+    return g_dt.to(dt.dtype), g_A, g_b
+
+
 class _DtCumsum(torch.autograd.Function):
     """(cum_A, decay) from dt."""
 
@@ -156,19 +174,12 @@ class _DtCumsum(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g_cum, g_decay):
         dt, A, dt_bias, decay = ctx.saved_tensors
-        rows, T, H = dt.shape
         if g_cum is None and g_decay is None:
             return None, None, None, None
         g_cum = None if g_cum is None else g_cum.contiguous().float()
         g_decay = None if g_decay is None else g_decay.contiguous().float()
-        g_dt = torch.empty((rows, T, H), dtype=torch.float32, device=dt.device)
-        g_A = torch.zeros(H, dtype=torch.float32, device=dt.device)
-        g_b = torch.zeros(H, dtype=torch.float32, device=dt.device) if dt_bias is not None else None
-        abi.check(abi.lib().rmx_mamba2_dt_cumsum_bwd(
-            dt.data_ptr(), int(dt.dtype == torch.float32), abi.ptr(dt_bias), A.data_ptr(),
-            int(ctx.softplus), abi.ptr(g_cum), None, abi.ptr(g_decay), decay.data_ptr(),
-            g_dt.data_ptr(), g_A.data_ptr(), abi.ptr(g_b), rows, T, H, abi.stream_of(dt)))
-        return g_dt.to(dt.dtype), g_A, g_b, None
+        return (*_dt_backward(dt, A, dt_bias, ctx.softplus, g_cum, None, g_decay, decay, False),
+                None)
 
 
 def mamba2_chunk_decay(dt: torch.Tensor, A: torch.Tensor, dt_bias: torch.Tensor | None = None,
@@ -229,15 +240,9 @@ class _ChunkState(torch.autograd.Function):
             x.data_ptr(), B.data_ptr(), e.data_ptr(), cum_A.data_ptr(), abi.ptr(t0),
             g.data_ptr(), g_x.data_ptr(), g_B.data_ptr(), g_e.data_ptr(), g_cum.data_ptr(),
             rows, T, H, D, G, N, abi.ptr(ws), ws_bytes, abi.stream_of(x)))
-        g_dt = torch.empty_like(g_e)
-        g_A = torch.zeros(H, dtype=torch.float32, device=x.device)
-        g_b = torch.zeros(H, dtype=torch.float32, device=x.device) if dt_bias is not None else None
         # (g_cum at T-1, on which every weight depends, is minus the sum of the others there)
-        abi.check(lib.rmx_mamba2_dt_cumsum_state_bwd(
-            dt.data_ptr(), int(dt.dtype == torch.float32), abi.ptr(dt_bias), A.data_ptr(),
-            int(ctx.softplus), g_cum.data_ptr(), g_e.data_ptr(), g_dt.data_ptr(), g_A.data_ptr(),
-            abi.ptr(g_b), rows, T, H, abi.stream_of(x)))
-        return g_x, g_B, g_dt.to(dt.dtype), g_A, g_b, None, None
+        return (g_x, g_B, *_dt_backward(dt, A, dt_bias, ctx.softplus, g_cum, g_e, None, None, True),
+                None, None)
 
 
 def last_document_start(seq_idx: torch.Tensor) -> torch.Tensor:

@@ -30,7 +30,7 @@ def test_library_exports_every_declared_symbol():
 
 def test_abi_version_and_error_string():
     lib = abi.lib()
-    assert lib.rmx_abi_version() == abi.ABI_VERSION == 19
+    assert lib.rmx_abi_version() == abi.ABI_VERSION == 20
     assert isinstance(lib.rmx_last_error(), bytes)
 
 
@@ -442,3 +442,19 @@ def test_empty_batch_launches_nothing(head_dim):
     assert lib.rmx_attn_fwd(ctypes.byref(lay), fwd, 1, None) == abi.RMX_OK
     assert lib.rmx_attn_bwd(ctypes.byref(lay), bwd, 1, None) == abi.RMX_OK
     assert lib.rmx_attn_bwd_ws(ctypes.byref(lay), bwd, 1, at, 0, None) == abi.RMX_OK
+
+
+def test_dt_cumsum_bwd_workspace_contract():
+    """Sizes: nothing for one chunk of tokens, two floats per row, chunk and head otherwise; a
+    misaligned workspace and a decay gradient of the state form are refused."""
+    lib, at = abi.lib(), 1 << 20  # an address, never read
+    size = lib.rmx_mamba2_dt_cumsum_bwd_workspace
+    for H, chunk in ((8, 1024), (16, 512), (32, 256), (33, 128), (64, 128), (65, 128)):
+        assert size(3, chunk, H) == 0
+        assert size(3, chunk + 1, H) == 3 * 2 * H * 8
+    assert size(0, 4096, 8) == size(-1, 4096, 8) == size(1, 0, 8) == 0
+    call = lambda state, decay, ws: lib.rmx_mamba2_dt_cumsum_bwd_ws(  # noqa: E731
+        at, 1, at, at, 1, at, at, decay, decay, at, at, at, 1, 4096, 8, state, ws, 1 << 20, None)
+    assert call(0, None, at + 4) == abi.RMX_EINVAL
+    assert call(1, at, at) == abi.RMX_EINVAL
+    assert call(2, None, at) == abi.RMX_EINVAL

@@ -79,3 +79,68 @@ def test_dt_cumsum_chunks(rows, T, H, softplus, f32):
         assert ((g_A.cpu() - grads[1]).abs() <= bar_A).all()
         if softplus:
             assert ((g_b.cpu() - grads[2]).abs() <= bar.sum((0, 1))).all()
+
+
+@pytest.mark.parametrize("rows,T,H", [(1, 4096, 8), (1, 1025, 3), (2, 2000, 16), (1, 300, 24),
+                                      (5, 400, 64), (3, 2000, 65), (1, 8192, 64)])
+@pytest.mark.parametrize("state", [False, True])
+def test_parameter_gradients_repeat(rows, T, H, state):
+    """dA and d(bias) of several chunks: with the workspace they repeat bit for bit, without it
+    for one or two rows; both forms within 32 roundings of their absolute sums of each other; a
+    workspace below the queried size is left alone."""
+    from ringmaster_amd import abi
+
+    print(f"case dt repeat rows={rows} T={T} H={H} state={state}", flush=True)
+    lib = abi.lib()
+    dt, bias, A = seeded((rows, T, H), 1).cuda(), (seeded((H,), 2) - 2).cuda(), -torch.exp(
+        seeded((H,), 3)).cuda()
+    g_cum, g_e = seeded((rows, T, H), 4).cuda(), seeded((rows, T, H), 5).cuda()
+    need = lib.rmx_mamba2_dt_cumsum_bwd_workspace(rows, T, H)
+    assert need > 0
+
+    def call(ws_bytes, ws):
+        g_dt, g_A, g_b = torch.empty_like(dt), torch.zeros_like(A), torch.zeros_like(A)
+        abi.check(lib.rmx_mamba2_dt_cumsum_bwd_ws(
+            dt.data_ptr(), 1, bias.data_ptr(), A.data_ptr(), 1, g_cum.data_ptr(), g_e.data_ptr(),
+            None, None, g_dt.data_ptr(), g_A.data_ptr(), g_b.data_ptr(), rows, T, H, int(state),
+            abi.ptr(ws), ws_bytes, abi.stream_of(dt)))
+        return g_dt, g_A, g_b
+
+    ws = torch.full((need + 64,), 0x5A, dtype=torch.uint8, device="cuda")
+    plain, again = call(need - 4, ws), [call(need - 4, ws) for _ in range(4)]
+    assert (ws == 0x5A).all(), "a workspace below the queried size was written"
+    if rows <= 2:
+        assert all(torch.equal(x, y) for other in again for x, y in zip(plain, other))
+    first, again = call(need, ws), [call(need, ws) for _ in range(4)]
+    assert (ws[need:] == 0x5A).all(), "written past the workspace"
+    assert all(torch.equal(x, y) for other in again for x, y in zip(first, other))
+    # R e and g_dt summed in absolute value bound every partial sum of either order
+    e = torch.nn.functional.softplus(dt.double() + bias)
+    g_abs = g_cum.double().abs().sum(1, keepdim=True)
+    bar_A = 32 * 2.0 ** -23 * (g_abs * e).sum((0, 1))
+    bar_b = 32 * 2.0 ** -23 * (A.double().abs() * g_abs + g_e.double().abs()).sum((0, 1))
+    assert ((first[1] - plain[1]).abs() <= bar_A).all()
+    assert ((first[2] - plain[2]).abs() <= bar_b).all()
+
+
+def test_one_row_calls_repeat():
+    """The public calls on one row (what a rank of a real run has): dA and d(bias) repeat."""
+    from ringmaster_amd.strategies.mamba import mamba2_chunk_decay, mamba2_chunk_state
+
+    T, H = 4096, 24
+    dt = seeded((1, T, H), 1).to(torch.bfloat16).cuda().requires_grad_(True)
+    A = (-torch.exp(seeded((H,), 2))).cuda().requires_grad_(True)
+    bias = (seeded((H,), 3) - 4).cuda().requires_grad_(True)
+    x = seeded((1, T, H, 64), 4).to(torch.bfloat16).cuda()
+    B = seeded((1, T, 1, 64), 5).to(torch.bfloat16).cuda()
+    g_cum, g_st = seeded((1, T, H), 6).cuda(), seeded((1, H, 64, 64), 7).cuda()
+
+    def grads():
+        cum, _ = mamba2_chunk_decay(dt, A, bias, True)
+        st = mamba2_chunk_state(x, dt, A, B, dt_bias=bias, dt_softplus=True)
+        return (*torch.autograd.grad(cum, (dt, A, bias), g_cum),
+                *torch.autograd.grad(st, (dt, A, bias), g_st))
+
+    first = grads()
+    for _ in range(8):
+        assert all(torch.equal(a, b) for a, b in zip(first, grads()))
