@@ -132,7 +132,7 @@ hipError_t launch_attn_bwd_delta(const rmx_attn_layout& L, const void* out, int 
 // 32 KV heads fills the chip and would go from 321 to 419 in two.
 DkdvSplit dkdv_split(const rmx_attn_layout& L, const rmx_bwd_problem* probs, int n) {
   constexpr int kCu = 256, kBkv = 128, kMaxSplit = 16;
-  DkdvSplit out{1, 0, 0};
+  DkdvSplit out{1, 0};
   const int hd = L.head_dim > 128 ? 256 : L.head_dim > 64 ? 128 : 64;
   const int bq = hd == 256 ? 32 : 64, G = L.hq / L.hkv;
   // us: per tile, per workgroup, of the fold launch
@@ -140,14 +140,11 @@ DkdvSplit dkdv_split(const rmx_attn_layout& L, const rmx_bwd_problem* probs, int
                fold = 5.;
   const int64_t per = (int64_t)L.batch * L.hkv;
   int64_t blocks = 0, keys = 0;
-  int skmax = 0, np = 0;
   for (int i = 0; i < n; ++i) {
     const rmx_bwd_problem& p = probs[i];
     if (p.sq == 0 || p.sk == 0 || p.dkv_mode == RMX_GRAD_NONE) continue;
-    blocks += per * ((p.sk + kBkv - 1) / kBkv);
+    blocks += per * split_key_blocks(p.sk);
     keys += per * p.sk;
-    skmax = p.sk > skmax ? p.sk : skmax;
-    ++np;
   }
   if (blocks == 0 || blocks >= 4 * kCu) return out;
   int64_t tiles = 0;  // of all blocks
@@ -184,41 +181,39 @@ DkdvSplit dkdv_split(const rmx_attn_layout& L, const rmx_bwd_problem* probs, int
       out.n = s;
     }
   }
-  if (out.n > 1) {
-    out.prob = per * skmax * (int64_t)L.head_dim;
-    out.grad = out.prob * np;
-  }
+  out.grad = keys * L.head_dim;
   return out;
 }
 
 struct FoldParams {
   rmx_attn_layout L;
   rmx_bwd_problem P[RMX_MAX_BATCHED];
-  const float* ws;
-  int nsplit, skmax;
-  int64_t prob, grad;
+  SplitParts parts;
+  int n, nsplit;
 };
 
-// Sum of the splits' partial dV (blockIdx.y even) and dK (odd) rows of one problem, stored in
-// its mode. Bound by its traffic (nsplit fp32 reads per element); a thread owns 4 columns of a
-// row, HD / 4 threads a row, the splits' loads four at a time in flight.
+// Sum of the splits' partial dV (blockIdx.y 0) and dK (1) rows, stored in their problem's mode.
+// Bound by its traffic (nsplit fp32 reads per element); a thread owns 4 columns of a row, HD / 4
+// threads a row, the splits' loads four at a time in flight.
 template <int HD, int DT>
 __global__ __launch_bounds__(256) void dkdv_fold_kernel(const FoldParams prm) {
   constexpr int CPR = HD / 4, RPB = 256 / CPR;
   const rmx_attn_layout& L = prm.L;
-  const rmx_bwd_problem& P = prm.P[blockIdx.y >> 1];
-  const int g = blockIdx.y & 1, D = L.head_dim;
+  const int g = blockIdx.y, D = L.head_dim, per = L.batch * L.hkv;
   const int col = 4 * (threadIdx.x % CPR);
-  const int64_t row = (int64_t)blockIdx.x * RPB + threadIdx.x / CPR;  // (batch, kv head, key)
-  if (col >= D || row >= (int64_t)L.batch * L.hkv * P.sk) return;
-  const int bh = (int)(row / P.sk), key = (int)(row - (int64_t)bh * P.sk);
+  const int64_t row = (int64_t)blockIdx.x * RPB + threadIdx.x / CPR;
+  int64_t local = row;  // (key, batch, kv head) of problem p
+  int p = 0;
+  for (; p < prm.n && local >= (int64_t)per * prm.P[p].sk; ++p) local -= (int64_t)per * prm.P[p].sk;
+  if (col >= D || p == prm.n) return;
+  const rmx_bwd_problem& P = prm.P[p];
+  const int key = (int)(local / per), bh = (int)(local - (int64_t)key * per);
   const int bb = bh / L.hkv, h = bh % L.hkv;
-  const float* src = prm.ws + (blockIdx.y >> 1) * prm.prob + g * prm.grad +
-                     ((int64_t)bh * prm.skmax + key) * D + col;
+  const float* src = prm.parts.base + g * prm.parts.grad + row * D + col;
   f32x4 v = *reinterpret_cast<const f32x4*>(src);
 #pragma unroll 4
   for (int s = 1; s < prm.nsplit; ++s)
-    v += *reinterpret_cast<const f32x4*>(src + s * 2 * prm.grad);
+    v += *reinterpret_cast<const f32x4*>(src + s * 2 * prm.parts.grad);
   const int mode = P.dkv_mode;
   const bool rd = mode == RMX_GRAD_ACC_F32 || mode == RMX_GRAD_ACC_FINAL;
   const bool w32 = mode == RMX_GRAD_WRITE_F32 || mode == RMX_GRAD_ACC_F32;
@@ -247,9 +242,9 @@ __global__ __launch_bounds__(256) void dkdv_fold_kernel(const FoldParams prm) {
 }
 
 template <int HD>
-static void launch_fold_t(const FoldParams& prm, int n, int64_t rows, bool f16, hipStream_t stream) {
+static void launch_fold_t(const FoldParams& prm, int64_t rows, bool f16, hipStream_t stream) {
   constexpr int RPB = 256 / (HD / 4);
-  const dim3 grid((unsigned)((rows + RPB - 1) / RPB), 2 * n);
+  const dim3 grid((unsigned)((rows + RPB - 1) / RPB), 2);
   if (f16)
     hipLaunchKernelGGL((dkdv_fold_kernel<HD, RMX_DTYPE_F16>), grid, dim3(256), 0, stream, prm);
   else
@@ -257,24 +252,21 @@ static void launch_fold_t(const FoldParams& prm, int n, int64_t rows, bool f16, 
 }
 
 hipError_t launch_dkdv_fold(const rmx_attn_layout& L, const rmx_bwd_problem* probs, int n,
-                            const DkdvSplit& split, const void* ws, hipStream_t stream) {
+                            const DkdvSplit& split, void* ws, hipStream_t stream) {
   FoldParams prm;
   prm.L = L;
   for (int i = 0; i < n; ++i) prm.P[i] = probs[i];
-  prm.ws = static_cast<const float*>(ws);
+  prm.parts = split.at(ws);
+  prm.n = n;
   prm.nsplit = split.n;
-  const int64_t per = (int64_t)L.batch * L.hkv;
-  prm.skmax = (int)(split.prob / (per * L.head_dim));
-  prm.prob = split.prob;
-  prm.grad = split.grad;
-  const int64_t rows = per * prm.skmax;
+  const int64_t rows = split.grad / L.head_dim;
   const bool f16 = L.dtype == RMX_DTYPE_F16;
   if (L.head_dim > 128)
-    launch_fold_t<256>(prm, n, rows, f16, stream);
+    launch_fold_t<256>(prm, rows, f16, stream);
   else if (L.head_dim > 64)
-    launch_fold_t<128>(prm, n, rows, f16, stream);
+    launch_fold_t<128>(prm, rows, f16, stream);
   else
-    launch_fold_t<64>(prm, n, rows, f16, stream);
+    launch_fold_t<64>(prm, rows, f16, stream);
   return hipGetLastError();
 }
 

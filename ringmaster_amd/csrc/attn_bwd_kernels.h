@@ -36,10 +36,10 @@ struct BwdParams {
   float scale_log2;
   uint32_t drop_thr;  // dropout: keep when the element's hash >= drop_thr
   float drop_scale;   // 1 / (1 - p)
-  // dK/dV: workgroups per key block (see the split notes at the dK/dV kernel) and the elements
-  // between the partial gradients of two splits
+  // dK/dV: workgroups per key block (see the split notes at the dK/dV kernel) and the splits'
+  // partial gradients
   int nsplit;
-  int64_t split_stride;
+  SplitParts parts;
 };
 
 // ---------------------------------------------------------------- shared helpers
@@ -60,8 +60,30 @@ __device__ __forceinline__ void grad_store4(int mode, float* acc, uint16_t* bf, 
 }
 
 // first of n items of share i of s
-__device__ __forceinline__ int split_lo(int n, int i, int s) {
-  return s == 1 ? (i ? n : 0) : (int)((int64_t)n * i / s);
+__device__ __forceinline__ int split_lo(int n, int i, int s) { return (int)((int64_t)n * i / s); }
+
+// ---------------------------------------------------------------- dK/dV splits
+// Partial gradients are rows [problem][key][batch, kv head] of head_dim: a problem's rows follow
+// those of the problems before it, and the strides are the same for all of them.
+// rows of the workspace before problem p
+__device__ __forceinline__ int64_t split_row0(const BwdParams& prm, int p) {
+  int64_t keys = 0;
+  for (int j = 0; j < p; ++j) keys += prm.P[j].sk;
+  return keys * prm.L.batch * prm.L.hkv;
+}
+
+// Where a workgroup's fp32 dK and dV go: the problem's accumulators or the split's partial rows.
+struct GradOut {
+  float *dv, *dk;
+  int64_t sb, ss, sh;
+};
+__device__ __forceinline__ GradOut grad_out(const BwdParams& prm, const rmx_bwd_problem& P, int p,
+                                            int share) {
+  const rmx_attn_layout& L = prm.L;
+  if (share < 0) return {P.dv_acc, P.dk_acc, L.ka_sb, L.ka_ss, L.ka_sh};
+  const int64_t D = L.head_dim, grad = prm.parts.grad;
+  float* const dv = prm.parts.base + 2 * grad * share + split_row0(prm, p) * D;
+  return {dv, dv + grad, L.hkv * D, (int64_t)L.batch * L.hkv * D, D};
 }
 
 // ---------------------------------------------------------------- tiles
@@ -654,7 +676,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_kernel(const BwdParams p
   const int G = L.hq / L.hkv;
   const int sq = P.sq, sk = P.sk;
   constexpr int mask = MASK;
-  const int split = wc.tile % prm.nsplit, k0 = wc.tile / prm.nsplit * C::BKV;
+  const int k0 = wc.tile / prm.nsplit * C::BKV;
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (SGPR)
@@ -707,12 +729,16 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_kernel(const BwdParams p
     qt_end = sRange[1] + 1;
     if (qt_end < qt_begin) qt_end = qt_begin;
   }
-  // (q head, query tile) pairs, q head major: this split's share [t_lo, t_lo + ntile)
+  // (q head, query tile) pairs, q head major: this workgroup's are [t_lo, t_lo + ntile)
   const int nqr = qt_end - qt_begin;
-  const int t_lo = split_lo(nqr * G, split, prm.nsplit);
-  const int ntile = split_lo(nqr * G, split + 1, prm.nsplit) - t_lo;
+  int t_lo = 0, ntile = nqr * G, share = -1;  // share: of a split block's tiles (-1: whole)
+  if (prm.nsplit > 1) {
+    share = wc.tile % prm.nsplit;
+    t_lo = split_lo(nqr * G, share, prm.nsplit);
+    ntile = split_lo(nqr * G, share + 1, prm.nsplit) - t_lo;
+  }
   // no query tile: accumulated dK and dV keep their values
-  if (ntile == 0 && P.dkv_mode == RMX_GRAD_ACC_F32) return;
+  if (ntile == 0 && share < 0 && P.dkv_mode == RMX_GRAD_ACC_F32) return;
   const int wave_klast = (kw0 + 31 < sk ? kw0 + 31 : sk - 1);
 
   // ---- tile loads. Wave 0 first loads the tile's lse and delta, and under document masks
@@ -1203,11 +1229,12 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_kernel(const BwdParams p
   int pe = wc.p;  // read the problem anew: its pointers are not kept in SGPRs across the loop
   asm volatile("" : "+s"(pe));
   const rmx_bwd_problem& E = prm.P[pe];
-  const int mode = E.dkv_mode;
+  const int mode = share >= 0 ? RMX_GRAD_WRITE_F32 : E.dkv_mode;
   const bool rd = mode == RMX_GRAD_ACC_F32 || mode == RMX_GRAD_ACC_FINAL;
   const bool w32 = mode == RMX_GRAD_WRITE_F32 || mode == RMX_GRAD_ACC_F32;
-  const bool vec = (!(rd || w32) || (((uintptr_t)E.dv_acc | (uintptr_t)E.dk_acc) & 15) == 0) &&
-                   (w32 || (((uintptr_t)E.dv | (uintptr_t)E.dk) & 7) == 0);
+  const bool vec = share >= 0 ||
+                   ((!(rd || w32) || (((uintptr_t)E.dv_acc | (uintptr_t)E.dk_acc) & 15) == 0) &&
+                    (w32 || (((uintptr_t)E.dv | (uintptr_t)E.dk) & 7) == 0));
   constexpr bool ELEMS = !DROP;
   if (ELEMS && !vec) {
     float prev[2][NDB][16];
@@ -1275,10 +1302,11 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_kernel(const BwdParams p
   __syncthreads();
   const int ch = el % CPR, rr = el / CPR;
   if (4 * ch >= L.head_dim) return;  // columns past the head dim are not stored
+  const GradOut O = grad_out(prm, E, pe, share);
 #pragma unroll 1
   for (int g = 0; g < 2; ++g) {
     const float* const stg = reinterpret_cast<const float*>(g == 0 ? &sQ[0][0] : &sO[0][0]) + 32 * wave * HD;
-    float* const gacc = (g == 0 ? E.dv_acc : E.dk_acc) + split * prm.split_stride + bb * L.ka_sb + kvh * L.ka_sh + 4 * ch;
+    float* const gacc = (g == 0 ? O.dv : O.dk) + bb * O.sb + kvh * O.sh + 4 * ch;
     uint16_t* const gbf = (g == 0 ? E.dv : E.dk) + bb * L.dk_sb + kvh * L.dk_sh + 4 * ch;
     if (!ELEMS && !vec) {
 #pragma unroll 1
@@ -1287,7 +1315,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_kernel(const BwdParams p
         const float* const src = stg + row * HD + 4 * (ch ^ (8 * ((row >> 2) & 1)));
 #pragma unroll 1
         for (int e = 0; e < 4; ++e) {
-          float* const x = gacc + kk * L.ka_ss + e;
+          float* const x = gacc + kk * O.ss + e;
           const float gv = rd ? *x + src[e] : src[e];
           if (w32)
             *x = gv;
@@ -1308,7 +1336,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_kernel(const BwdParams p
 #pragma unroll
       for (int i = 0; i < NI; ++i) {
         const int kk = kw0 + RPI * i + rr;
-        prev[i] = kk < sk ? *reinterpret_cast<const f32x4*>(gacc + (int64_t)kk * L.ka_ss) : f32x4{};
+        prev[i] = kk < sk ? *reinterpret_cast<const f32x4*>(gacc + (int64_t)kk * O.ss) : f32x4{};
       }
 #pragma unroll
       for (int i = 0; i < NI; ++i) v[i] += prev[i];
@@ -1318,7 +1346,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_kernel(const BwdParams p
       const int kk = kw0 + RPI * i + rr;
       if (kk >= sk) continue;
       if (w32) {
-        *reinterpret_cast<f32x4*>(gacc + (int64_t)kk * L.ka_ss) = v[i];
+        *reinterpret_cast<f32x4*>(gacc + (int64_t)kk * O.ss) = v[i];
       } else {
         u32x2 w;
         w[0] = cvt_pk<DT>(v[i][0], v[i][1]);
@@ -1387,7 +1415,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_d256_kernel(const BwdPar
   const int G = L.hq / L.hkv;
   const int sq = P.sq, sk = P.sk;
   constexpr int mask = MASK;
-  const int split = wc.tile % prm.nsplit, k0 = wc.tile / prm.nsplit * BKV;
+  const int k0 = wc.tile / prm.nsplit * BKV;
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (SGPR)
@@ -1440,12 +1468,16 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_d256_kernel(const BwdPar
     qt_end = sRange[1] + 1;
     if (qt_end < qt_begin) qt_end = qt_begin;
   }
-  // (q head, query tile) pairs, q head major: this split's share [t_lo, t_lo + ntile)
+  // (q head, query tile) pairs, q head major: this workgroup's are [t_lo, t_lo + ntile)
   const int nqr = qt_end - qt_begin;
-  const int t_lo = split_lo(nqr * G, split, prm.nsplit);
-  const int ntile = split_lo(nqr * G, split + 1, prm.nsplit) - t_lo;
+  int t_lo = 0, ntile = nqr * G, share = -1;  // share: of a split block's tiles (-1: whole)
+  if (prm.nsplit > 1) {
+    share = wc.tile % prm.nsplit;
+    t_lo = split_lo(nqr * G, share, prm.nsplit);
+    ntile = split_lo(nqr * G, share + 1, prm.nsplit) - t_lo;
+  }
   // no query tile: accumulated dK and dV keep their values
-  if (ntile == 0 && P.dkv_mode == RMX_GRAD_ACC_F32) return;
+  if (ntile == 0 && share < 0 && P.dkv_mode == RMX_GRAD_ACC_F32) return;
   const int wave_klast = (kw0 + 31 < sk ? kw0 + 31 : sk - 1);
 
   struct Cursor {
@@ -1840,7 +1872,8 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_d256_kernel(const BwdPar
   // ---- epilogue: lane (hl, l32) holds column d = 32 db + l32 of keys kw0 + c_row(hl, r).
   // Each gradient is staged through LDS as [key][d] fp32 rows (the tiles are dead) and
   // stored as 4-column runs of whole rows: one mode test per run, not per element.
-  const int mode = P.dkv_mode;
+  const int mode = share >= 0 ? RMX_GRAD_WRITE_F32 : P.dkv_mode;
+  const GradOut O = grad_out(prm, P, wc.p, share);
   float* const stg = reinterpret_cast<float*>(smem);
   const int col = 4 * (tid & 63), rw = tid >> 6;  // columns col .. col + 3 of rows rw + 4 i
   auto store = [&](const f32x16* acc, float sc, float* gacc, uint16_t* gbf) {
@@ -1852,9 +1885,9 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_d256_kernel(const BwdPar
         stg[(32 * wave + c_row(hl, r)) * HD + 32 * db + l32] = acc[db][r] * sc;
     __syncthreads();
     if (col >= D) return;  // columns past the head dim are not stored
-    const bool vf = ((uintptr_t)gacc & 15) == 0, vb = ((uintptr_t)gbf & 7) == 0;
+    const bool vf = ((uintptr_t)gacc & 15) == 0, vb = share >= 0 || ((uintptr_t)gbf & 7) == 0;
     auto gptr = [&](int kk) {
-      return gacc ? gacc + bb * L.ka_sb + (int64_t)kk * L.ka_ss + kvh * L.ka_sh + col : nullptr;
+      return gacc ? gacc + bb * O.sb + (int64_t)kk * O.ss + kvh * O.sh + col : nullptr;
     };
     auto bptr = [&](int kk) {
       return gbf ? gbf + bb * L.dk_sb + (int64_t)kk * L.dk_ss + kvh * L.dk_sh + col : nullptr;
@@ -1904,9 +1937,8 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_d256_kernel(const BwdPar
       }
     }
   };
-  const int64_t so = split * prm.split_stride;
-  store(dv, 1.f, P.dv_acc ? P.dv_acc + so : nullptr, P.dv);
-  store(dk, -L.scale, P.dk_acc ? P.dk_acc + so : nullptr, P.dk);
+  store(dv, 1.f, O.dv, P.dv);
+  store(dk, -L.scale, O.dk, P.dk);
 }
 
 // dQ of the n problems in prm.P (in launch order)
@@ -1932,6 +1964,7 @@ template <int HD, int DT, bool DROP>
 hipError_t launch_bwd_t(const rmx_attn_layout& L, const rmx_bwd_problem* probs, int n,
                         const DkdvSplit& split, void* ws, hipStream_t stream) {
   constexpr int BKV = HD == 256 ? 128 : DkdvCfg<HD>::BKV;
+  static_assert(split_key_blocks(BKV) == 1 && split_key_blocks(BKV + 1) == 2, "key blocks");
   BwdParams pq, pk;
   pq.L = L;
   pk.L = L;
@@ -1960,25 +1993,11 @@ hipError_t launch_bwd_t(const rmx_attn_layout& L, const rmx_bwd_problem* probs, 
   order_by_cost(nk, ck, ok);
   for (int i = 0; i < nq; ++i) pq.P[i] = probs[iq[oq[i]]];
   pq.nsplit = 1;
-  pq.split_stride = 0;
   pk.nsplit = split.n;
-  pk.split_stride = split.n > 1 ? 2 * split.grad : 0;
+  pq.parts = pk.parts = split.n > 1 ? split.at(ws) : SplitParts{};
   for (int i = 0; i < nk; ++i) {
     pk.P[i] = probs[ik[ok[i]]];
     ntile[i] = (pk.P[i].sk + BKV - 1) / BKV * split.n;
-  }
-  rmx_bwd_problem fold[RMX_MAX_BATCHED];
-  if (split.n > 1) {  // the kernels write partial gradients, the fold kernel the call's outputs
-    for (int i = 0; i < nk; ++i) {
-      fold[i] = pk.P[i];
-      pk.P[i].dkv_mode = RMX_GRAD_WRITE_F32;
-      pk.P[i].dv_acc = static_cast<float*>(ws) + i * split.prob;
-      pk.P[i].dk_acc = pk.P[i].dv_acc + split.grad;
-      pk.P[i].dv = pk.P[i].dk = nullptr;
-    }
-    pk.L.ka_ss = L.head_dim;
-    pk.L.ka_sh = split.prob / ((int64_t)L.batch * L.hkv);
-    pk.L.ka_sb = pk.L.ka_sh * L.hkv;
   }
   const int tk = plan_workgroups(pk.map, nk, L.batch * L.hkv, 1, ntile, L.mask == RMX_MASK_CAUSAL);
   if constexpr (HD == 256) {
@@ -2007,7 +2026,7 @@ hipError_t launch_bwd_t(const rmx_attn_layout& L, const rmx_bwd_problem* probs, 
     }
   }
   if (tk > 0 && split.n > 1) {
-    const hipError_t e = launch_dkdv_fold(L, fold, nk, split, ws, stream);
+    const hipError_t e = launch_dkdv_fold(L, pk.P, nk, split, ws, stream);
     if (e != hipSuccess) return e;
   }
   if (nq == 0) return hipSuccess;

@@ -14,17 +14,24 @@ hipError_t launch_attn_fwd(const rmx_attn_layout& L, const rmx_fwd_problem* prob
 hipError_t launch_attn_bwd_delta(const rmx_attn_layout& L, const void* out, int out_f32,
                                  const uint16_t* dout, float* delta, const float* lse, float* nlse,
                                  int sq, hipStream_t stream);
-// How a launch's key blocks are split over workgroups (n = 1: not at all): elements of one
-// problem's partial gradient (rows [batch, hkv, longest sk] of head_dim) and of all problems',
-// and the workspace: n splits x (dV, dK).
+// A split dK/dV launch's workspace: `base` holds n splits x (dV, dK) of `grad` elements each, a
+// gradient being rows [problem][key][batch, kv head] of head_dim.
+struct SplitParts {
+  float* base;
+  int64_t grad;
+};
+__host__ __device__ constexpr int split_key_blocks(int sk) { return (sk + 127) / 128; }
+// How a launch's key blocks are split over workgroups (n = 1: not at all) and the elements of its
+// dK (or dV).
 struct DkdvSplit {
   int n;
-  int64_t prob, grad;
+  int64_t grad;
   size_t bytes() const { return n > 1 ? (size_t)n * 2 * (size_t)grad * 4 : 0; }
+  SplitParts at(void* ws) const { return {static_cast<float*>(ws), grad}; }
 };
 DkdvSplit dkdv_split(const rmx_attn_layout& L, const rmx_bwd_problem* probs, int n);
 hipError_t launch_dkdv_fold(const rmx_attn_layout& L, const rmx_bwd_problem* probs, int n,
-                            const DkdvSplit& split, const void* ws, hipStream_t stream);
+                            const DkdvSplit& split, void* ws, hipStream_t stream);
 // ws: split.bytes() of workspace
 hipError_t launch_attn_bwd(const rmx_attn_layout& L, const rmx_bwd_problem* probs, int n,
                            const DkdvSplit& split, void* ws, hipStream_t stream);

@@ -458,3 +458,24 @@ def test_dt_cumsum_bwd_workspace_contract():
     assert call(0, None, at + 4) == abi.RMX_EINVAL
     assert call(1, at, at) == abi.RMX_EINVAL
     assert call(2, None, at) == abi.RMX_EINVAL
+
+
+def test_split_workspace_follows_the_keys():
+    """Problems of very different lengths take the rows they have, not the longest one's: the
+    splits' two fp32 gradients of every key."""
+    d = 128
+    lay = _layout(hq=8, hkv=1, head_dim=d)
+    for name in ("q", "k", "v", "o", "dk", "a", "ka"):
+        for s in ("sb", "ss", "sh"):
+            setattr(lay, f"{name}_{s}", 1024)
+    arr = (abi.BwdProblem * 16)()
+    for i, p in enumerate(arr):
+        for field, kind in p._fields_:
+            if kind is ctypes.c_void_p:
+                setattr(p, field, 1 << 20)  # an address, never read
+        p.sq, p.sk = 512, 4096 if i == 0 else 8
+        p.dq_mode, p.dkv_mode = abi.GRAD_NONE, abi.GRAD_WRITE_F32
+    keys = 4096 + 15 * 8
+    need = abi.lib().rmx_attn_bwd_workspace(ctypes.byref(lay), arr, 16)
+    splits, rest = divmod(need, 8 * keys * d)
+    assert rest == 0 and 2 <= splits <= 16

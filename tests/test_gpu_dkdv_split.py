@@ -95,6 +95,63 @@ def test_split_equals_whole(b, sq, sk, hq, hkv, d, kind, x, off):
             assert a.abs().sum() > 0 and rel_l2(c.cpu(), a.cpu()) < bar
 
 
+@pytest.mark.parametrize("kind", ["causal", "doc"])
+def test_workspace_contract(kind):
+    """A workspace below the queried size is not touched and the call runs unsplit, one of that
+    size is not written past its end, a misaligned one is refused; problems of different
+    lengths keep to their own rows."""
+    from ringmaster_amd import abi
+    from ringmaster_amd.ring import ops
+    from ringmaster_amd.ring.kernels import block_forward
+
+    print(f"case workspace contract {kind}", flush=True)
+    b, sq, hq, hkv, d = 1, 700, 8, 2, 128
+    q, k, v, do = (bf16_pair((b, sq, h, d), s)[1] for h, s in ((hq, 1), (hkv, 2), (hkv, 3), (hq, 4)))
+    _, lse, out32 = block_forward(q, k, v, d ** -0.5, True, keep_f32=True)
+    delta = torch.empty((b, hq, sq), device="cuda")
+    nlse = torch.empty_like(delta)
+    ops.attn_bwd_delta(out32, do, delta, hkv, lse=lse, nlse=nlse)
+    ar = torch.arange(sq, dtype=torch.int32, device="cuda")
+    jobs, outs = [], []
+    for n in (129, 700, 33):
+        dk, dv = (torch.empty((b, n, hkv, d), device="cuda") for _ in range(2))
+        meta = dict(q_gidx=ar, k_gidx=ar[:n], q_doc=ar // 250, k_doc=ar[:n] // 250) \
+            if kind == "doc" else {}
+        jobs.append(ops.BwdJob(q=q, k=k[:, :n], v=v[:, :n], dout=do, lse=lse, delta=delta,
+                               nlse=nlse, dq_mode=abi.GRAD_NONE, dkv_mode=abi.GRAD_WRITE_F32,
+                               dk_acc=dk, dv_acc=dv, **meta))
+        outs += [dk, dv]
+    # one call has one set of strides: give every problem the longest one's buffers
+    big = [torch.empty((b, 700, hkv, d), device="cuda") for _ in outs]
+    for i, j in enumerate(jobs):
+        n = j.k.shape[1]
+        j.dk_acc, j.dv_acc = big[2 * i][:, :n], big[2 * i + 1][:, :n]
+    mask = abi.MASK_DOC if kind == "doc" else abi.MASK_CAUSAL
+    lay, arr = ops._pack_bwd(jobs, d ** -0.5, mask, None)
+    lib = abi.lib()
+    need = lib.rmx_attn_bwd_workspace(ctypes.byref(lay), arr, len(jobs))
+    assert need > 16
+    ws = torch.full((need + 4096,), 0xFF, dtype=torch.uint8, device="cuda")
+
+    def call(ptr, nbytes):
+        for t in big:
+            t.fill_(7.0)
+        rc = lib.rmx_attn_bwd_ws(ctypes.byref(lay), arr, len(jobs), ptr, nbytes, abi.stream_of(q))
+        torch.cuda.synchronize()
+        return rc, [t.clone() for t in big]
+
+    _, whole = call(None, 0)
+    rc, small = call(ws.data_ptr(), need - 1)
+    assert rc == abi.RMX_OK and (ws == 0xFF).all()
+    assert all(torch.equal(a, c) for a, c in zip(whole, small))
+    assert call(ws.data_ptr() + 4, need)[0] == abi.RMX_EINVAL
+    rc, split = call(ws.data_ptr(), need)
+    assert rc == abi.RMX_OK and (ws[need:] == 0xFF).all() and not (ws[:need] == 0xFF).all()
+    for i, (a, c) in enumerate(zip(whole, split)):
+        n = jobs[i // 2].k.shape[1]
+        assert (c[:, n:] == 7.0).all() and rel_l2(c[:, :n].cpu(), a[:, :n].cpu()) < 1e-6
+
+
 def test_refused_arguments_and_small_workspaces():
     """The workspace query of a refused call is 0 and the call itself still refuses."""
     from ringmaster_amd import abi
