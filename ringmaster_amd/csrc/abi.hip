@@ -239,9 +239,9 @@ int32_t rmx_attn_bwd_ws(const rmx_attn_layout* layout, const rmx_bwd_problem* pr
     return fail(RMX_EINVAL, "workspace must be 16-byte aligned");
   for (int i = 0; i < nproblems; i += RMX_MAX_BATCHED) {
     const int n = std::min(nproblems - i, RMX_MAX_BATCHED);
-    rmx::DkdvSplit split{1, 0};
+    rmx::DkdvSplit split{1, 0, 0};
     if (workspace) split = rmx::dkdv_split(*layout, problems + i, n);
-    if (split.bytes() > workspace_bytes) split = rmx::DkdvSplit{1, 0};
+    if (split.bytes() > workspace_bytes) split = rmx::DkdvSplit{1, 0, 0};
     rc = dev_status(rmx::launch_attn_bwd(*layout, problems + i, n, split, workspace,
                                          (hipStream_t)stream),
                     "rmx_attn_bwd launch");

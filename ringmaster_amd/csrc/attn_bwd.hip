@@ -123,16 +123,20 @@ hipError_t launch_attn_bwd_delta(const rmx_attn_layout& L, const void* out, int 
 
 // ---------------------------------------------------------------- dK/dV splits
 // Workgroups per key block of a dK/dV launch. The launch's time is estimated for every
-// number of splits from the tile counts of its key blocks (the masks' own ranges; documents
-// count as causal): a tile and a workgroup cost what the kernels measure on a lone CU,
+// number of splits from the tile counts of its key blocks (the masks' own ranges; documents,
+// whose ranges only the device knows, count as causal: the longest they can be): a tile and a
+// workgroup cost what the kernels measure on a lone CU,
 // workgroups run in rounds over the CUs, and a split launch adds the fold kernel and the
 // partial gradients' traffic. Launches of many rounds stay whole. Whole -> split, us a launch:
 // 4096^2 causal 32/8 heads of 128 403 -> 314 (2), 2048^2 189 -> 101 (3), 512^2 58 -> 34 (4);
 // 4096^2 causal 16/4 heads of 256 821 -> 343 (4), of 64 253 -> 102 (4); the same 4096^2 with
 // 32 KV heads fills the chip and would go from 321 to 419 in two.
+// A packed ring's backward (every kernel of it), whole -> split: 4 ranks x 1024 tokens, 8/2 heads of
+// 128, documents of 64 tokens 269 -> 214, of 2048 504 -> 321; 8 x 766, 4/2 heads of 64, of 364 217 -> 209;
+// over 22 rings of the range at most 1.02 of the whole one's time.
 DkdvSplit dkdv_split(const rmx_attn_layout& L, const rmx_bwd_problem* probs, int n) {
   constexpr int kCu = 256, kBkv = 128, kMaxSplit = 16;
-  DkdvSplit out{1, 0};
+  DkdvSplit out{1, 0, 0};
   const int hd = L.head_dim > 128 ? 256 : L.head_dim > 64 ? 128 : 64;
   const int bq = hd == 256 ? 32 : 64, G = L.hq / L.hkv;
   // us: per tile, per workgroup, of the fold launch
@@ -182,6 +186,7 @@ DkdvSplit dkdv_split(const rmx_attn_layout& L, const rmx_bwd_problem* probs, int
     }
   }
   out.grad = keys * L.head_dim;
+  out.blocks = blocks;
   return out;
 }
 
@@ -203,12 +208,17 @@ __global__ __launch_bounds__(256) void dkdv_fold_kernel(const FoldParams prm) {
   const int col = 4 * (threadIdx.x % CPR);
   const int64_t row = (int64_t)blockIdx.x * RPB + threadIdx.x / CPR;
   int64_t local = row;  // (key, batch, kv head) of problem p
-  int p = 0;
-  for (; p < prm.n && local >= (int64_t)per * prm.P[p].sk; ++p) local -= (int64_t)per * prm.P[p].sk;
+  int p = 0, block = 0;
+  for (; p < prm.n && local >= (int64_t)per * prm.P[p].sk; ++p) {
+    local -= (int64_t)per * prm.P[p].sk;
+    block += per * split_key_blocks(prm.P[p].sk);
+  }
   if (col >= D || p == prm.n) return;
   const rmx_bwd_problem& P = prm.P[p];
   const int key = (int)(local / per), bh = (int)(local - (int64_t)key * per);
   const int bb = bh / L.hkv, h = bh % L.hkv;
+  // (an empty block is its first workgroup's, which has stored it if the mode writes)
+  if (L.mask == RMX_MASK_DOC && prm.parts.empty[block + bh * split_key_blocks(P.sk) + key / 128]) return;
   const float* src = prm.parts.base + g * prm.parts.grad + row * D + col;
   f32x4 v = *reinterpret_cast<const f32x4*>(src);
 #pragma unroll 4

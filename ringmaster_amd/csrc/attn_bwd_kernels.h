@@ -36,8 +36,8 @@ struct BwdParams {
   float scale_log2;
   uint32_t drop_thr;  // dropout: keep when the element's hash >= drop_thr
   float drop_scale;   // 1 / (1 - p)
-  // dK/dV: workgroups per key block (see the split notes at the dK/dV kernel) and the splits'
-  // partial gradients
+  // dK/dV: workgroups per key block (see the split notes at the dK/dV kernel), the splits'
+  // partial gradients and which blocks have none (RMX_MASK_DOC)
   int nsplit;
   SplitParts parts;
 };
@@ -84,6 +84,14 @@ __device__ __forceinline__ GradOut grad_out(const BwdParams& prm, const rmx_bwd_
   const int64_t D = L.head_dim, grad = prm.parts.grad;
   float* const dv = prm.parts.base + 2 * grad * share + split_row0(prm, p) * D;
   return {dv, dv + grad, L.hkv * D, (int64_t)L.batch * L.hkv * D, D};
+}
+
+// index of key block kb of (problem p, group = batch * hkv + kv head)
+__device__ __forceinline__ int split_block(const BwdParams& prm, int p, int group, int kb) {
+  const int per = prm.L.batch * prm.L.hkv;
+  int at = 0;
+  for (int j = 0; j < p; ++j) at += per * split_key_blocks(prm.P[j].sk);
+  return at + group * split_key_blocks(prm.P[p].sk) + kb;
 }
 
 // ---------------------------------------------------------------- tiles
@@ -621,7 +629,10 @@ __global__ __launch_bounds__(64 * WAVES, 1) void attn_bwd_dq_kernel(const BwdPar
 // idle behind long workgroups. The launcher then gives each block nsplit workgroups with
 // equal shares of its tiles. They write fp32 partial gradients to the caller's workspace,
 // which dkdv_fold_kernel adds in split order (deterministic) and stores in the call's mode
-// (the rule and its measurements: dkdv_split in attn_bwd.hip).
+// (the rule and its measurements: dkdv_split in attn_bwd.hip). Only the device knows how far a
+// block's documents reach, and past a ring's first step most blocks reach no query: such a block
+// is left to its first workgroup, as an unsplit one (the accumulating mode touches no memory), and
+// the fold passes it over. (So left with up to 4 or 12 tiles: 0-5% and up to 44% slower.)
 // Q/dO tiles (with lse, delta) arrive by LDS DMA into four buffers; a tile is
 // issued three barriers before it is read. Tiles past the end are issued as
 // zero-length loads (they write zeros to a free buffer and touch no memory),
@@ -734,8 +745,17 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_kernel(const BwdParams p
   int t_lo = 0, ntile = nqr * G, share = -1;  // share: of a split block's tiles (-1: whole)
   if (prm.nsplit > 1) {
     share = wc.tile % prm.nsplit;
-    t_lo = split_lo(nqr * G, share, prm.nsplit);
-    ntile = split_lo(nqr * G, share + 1, prm.nsplit) - t_lo;
+    if (mask == RMX_MASK_DOC) {
+      const bool empty = ntile == 0;
+      if (share == 0 && tid == 0)
+        prm.parts.empty[split_block(prm, wc.p, wc.group, wc.tile / prm.nsplit)] = empty;
+      if (empty && share > 0) return;
+      if (empty) share = -1;
+    }
+    if (share >= 0) {
+      t_lo = split_lo(nqr * G, share, prm.nsplit);
+      ntile = split_lo(nqr * G, share + 1, prm.nsplit) - t_lo;
+    }
   }
   // no query tile: accumulated dK and dV keep their values
   if (ntile == 0 && share < 0 && P.dkv_mode == RMX_GRAD_ACC_F32) return;
@@ -1473,8 +1493,17 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_d256_kernel(const BwdPar
   int t_lo = 0, ntile = nqr * G, share = -1;  // share: of a split block's tiles (-1: whole)
   if (prm.nsplit > 1) {
     share = wc.tile % prm.nsplit;
-    t_lo = split_lo(nqr * G, share, prm.nsplit);
-    ntile = split_lo(nqr * G, share + 1, prm.nsplit) - t_lo;
+    if (mask == RMX_MASK_DOC) {
+      const bool empty = ntile == 0;
+      if (share == 0 && tid == 0)
+        prm.parts.empty[split_block(prm, wc.p, wc.group, wc.tile / prm.nsplit)] = empty;
+      if (empty && share > 0) return;
+      if (empty) share = -1;
+    }
+    if (share >= 0) {
+      t_lo = split_lo(nqr * G, share, prm.nsplit);
+      ntile = split_lo(nqr * G, share + 1, prm.nsplit) - t_lo;
+    }
   }
   // no query tile: accumulated dK and dV keep their values
   if (ntile == 0 && share < 0 && P.dkv_mode == RMX_GRAD_ACC_F32) return;

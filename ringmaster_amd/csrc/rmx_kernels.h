@@ -15,19 +15,24 @@ hipError_t launch_attn_bwd_delta(const rmx_attn_layout& L, const void* out, int 
                                  const uint16_t* dout, float* delta, const float* lse, float* nlse,
                                  int sq, hipStream_t stream);
 // A split dK/dV launch's workspace: `base` holds n splits x (dV, dK) of `grad` elements each, a
-// gradient being rows [problem][key][batch, kv head] of head_dim.
+// gradient being rows [problem][key][batch, kv head] of head_dim; `empty` one word per key block
+// ([problem][batch, kv head][block], RMX_MASK_DOC only): 1 where no query attends it.
 struct SplitParts {
   float* base;
+  int32_t* empty;
   int64_t grad;
 };
 __host__ __device__ constexpr int split_key_blocks(int sk) { return (sk + 127) / 128; }
-// How a launch's key blocks are split over workgroups (n = 1: not at all) and the elements of its
-// dK (or dV).
+// How a launch's key blocks are split over workgroups (n = 1: not at all), the elements of its
+// dK (or dV) and its key blocks.
 struct DkdvSplit {
   int n;
-  int64_t grad;
-  size_t bytes() const { return n > 1 ? (size_t)n * 2 * (size_t)grad * 4 : 0; }
-  SplitParts at(void* ws) const { return {static_cast<float*>(ws), grad}; }
+  int64_t grad, blocks;
+  size_t bytes() const { return n > 1 ? (size_t)n * 2 * (size_t)grad * 4 + (size_t)blocks * 4 : 0; }
+  SplitParts at(void* ws) const {
+    float* const base = static_cast<float*>(ws);
+    return {base, reinterpret_cast<int32_t*>(base + n * 2 * grad), grad};
+  }
 };
 DkdvSplit dkdv_split(const rmx_attn_layout& L, const rmx_bwd_problem* probs, int n);
 hipError_t launch_dkdv_fold(const rmx_attn_layout& L, const rmx_bwd_problem* probs, int n,

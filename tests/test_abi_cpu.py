@@ -462,7 +462,7 @@ def test_dt_cumsum_bwd_workspace_contract():
 
 def test_split_workspace_follows_the_keys():
     """Problems of very different lengths take the rows they have, not the longest one's: the
-    splits' two fp32 gradients of every key."""
+    splits' two fp32 gradients of every key and a word per key block."""
     d = 128
     lay = _layout(hq=8, hkv=1, head_dim=d)
     for name in ("q", "k", "v", "o", "dk", "a", "ka"):
@@ -475,7 +475,7 @@ def test_split_workspace_follows_the_keys():
                 setattr(p, field, 1 << 20)  # an address, never read
         p.sq, p.sk = 512, 4096 if i == 0 else 8
         p.dq_mode, p.dkv_mode = abi.GRAD_NONE, abi.GRAD_WRITE_F32
-    keys = 4096 + 15 * 8
+    keys, blocks = 4096 + 15 * 8, 32 + 15
     need = abi.lib().rmx_attn_bwd_workspace(ctypes.byref(lay), arr, 16)
-    splits, rest = divmod(need, 8 * keys * d)
+    splits, rest = divmod(need - 4 * blocks, 8 * keys * d)
     assert rest == 0 and 2 <= splits <= 16

@@ -95,6 +95,85 @@ def test_split_equals_whole(b, sq, sk, hq, hkv, d, kind, x, off):
             assert a.abs().sum() > 0 and rel_l2(c.cpu(), a.cpu()) < bar
 
 
+@pytest.mark.parametrize("d,docs", [(64, 40), (128, 40), (128, 300), (256, 40), (128, 5000)])
+@pytest.mark.parametrize("layout,causal", [("zigzag", True), ("contiguous", False)])
+def test_packed_ring_split_equals_whole(monkeypatch, d, docs, layout, causal):
+    """A packed ring backward whose steps the rule splits: most key blocks past the first step have
+    no query of their documents (all of them at 40 tokens), which the splits leave as the
+    unsplit kernel does, whatever the workspace holds."""
+    from ringmaster_amd import abi
+    from ringmaster_amd.ring import ops, zigzag
+
+    print(f"case packed split d={d} docs={docs} {layout} causal={causal}", flush=True)
+    P, L, hq, hkv = 4, 640, 8, 2
+    mk = lambda h, s: bf16_pair((P, 1, h, L, d), s)[1]  # noqa: E731
+    q, k, v, do = mk(hq, 1), mk(hkv, 2), mk(hkv, 3), mk(hq, 4).transpose(2, 3).contiguous()
+    doc = torch.arange(P * L, dtype=torch.int32, device="cuda") // docs
+    kw = dict(layout=layout, causal=causal)
+    out, lse, o32 = zigzag.ring_forward(q, k, v, d ** -0.5, doc, **kw)
+    lib, sizes = abi.lib(), []
+
+    class Lib:
+        split = True
+
+        def __getattr__(self, name):
+            return getattr(lib, name)
+
+        def rmx_attn_bwd_workspace(self, *a):
+            sizes.append(lib.rmx_attn_bwd_workspace(*a) if self.split else 0)
+            return sizes[-1]
+
+    one = Lib()
+    monkeypatch.setattr(abi, "lib", lambda: one)
+    real = torch.empty
+
+    def filled(*a, **kw):  # workspaces hold NaN: nothing unwritten may reach a gradient
+        t = real(*a, **kw)
+        return t.fill_(255) if t.dtype == torch.uint8 else t
+
+    def grads(split):
+        ops._plans.clear()
+        one.split = split
+        r = [g.clone() for g in zigzag.ring_backward(do, q, k, v, o32, lse, d ** -0.5, doc, **kw)]
+        ops._plans.clear()
+        return r
+
+    whole = grads(False)
+    sizes.clear()
+    monkeypatch.setattr(torch, "empty", filled)
+    split = grads(True)
+    assert max(sizes) > 0, "the rule does not split this ring"
+    assert torch.equal(whole[0], split[0])
+    for a, c in zip(whole[1:], split[1:]):
+        assert rel_l2(c.cpu(), a.cpu()) < 1e-6
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_empty_document_blocks_touch_no_memory(d):
+    """A split launch of pairs of different documents, accumulating: neither the accumulators
+    (-0.0 would turn to 0.0) nor the workspace's partial rows are written."""
+    from ringmaster_amd import abi
+    from ringmaster_amd.ring import ops
+
+    print(f"case empty documents d={d}", flush=True)
+    n, hq, hkv = 512, 8, 2
+    q, k, v, do = (bf16_pair((1, n, h, d), s)[1] for h, s in ((hq, 1), (hkv, 2), (hkv, 3), (hq, 4)))
+    stat = torch.zeros((1, hq, n), device="cuda")
+    ar = torch.arange(n, dtype=torch.int32, device="cuda")
+    acc = [torch.full((1, n, hkv, d), -0.0, device="cuda") for _ in range(2)]
+    job = ops.BwdJob(q=q, k=k, v=v, dout=do, lse=stat, delta=stat, nlse=stat, dq_mode=abi.GRAD_NONE,
+                     dkv_mode=abi.GRAD_ACC_F32, dk_acc=acc[0], dv_acc=acc[1], q_gidx=ar + n,
+                     k_gidx=ar, q_doc=ar // 100 + 50, k_doc=ar // 100)
+    lay, arr = ops._pack_bwd([job], d ** -0.5, abi.MASK_DOC, None)
+    lib = abi.lib()
+    need = lib.rmx_attn_bwd_workspace(ctypes.byref(lay), arr, 1)
+    assert need > 0, "the rule does not split this shape"
+    ws = torch.full((need,), 0xFF, dtype=torch.uint8, device="cuda")
+    abi.check(lib.rmx_attn_bwd_ws(ctypes.byref(lay), arr, 1, ws.data_ptr(), need, abi.stream_of(q)))
+    assert all(torch.signbit(a).all() and (a == 0).all() for a in acc)
+    assert (ws[:need - 4 * hkv * (n // 128)] == 0xFF).all()
+
+
 @pytest.mark.parametrize("kind", ["causal", "doc"])
 def test_workspace_contract(kind):
     """A workspace below the queried size is not touched and the call runs unsplit, one of that
