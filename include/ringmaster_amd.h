@@ -227,8 +227,8 @@ int32_t rmx_attn_bwd(const rmx_attn_layout* layout, const rmx_bwd_problem* probl
  * The same with device memory for partial dK/dV sums: a call with few key blocks (or causal
  * ones of very different lengths) then gives each several workgroups, whose fp32 partial
  * gradients are summed in a fixed order before the mode is applied. rmx_attn_bwd_workspace
- * returns the bytes the call can use (0: it runs as rmx_attn_bwd does, also for arguments
- * rmx_attn_bwd refuses); the workspace (nullable, 16-byte aligned) is scratch of this call,
+ * returns the bytes the call can use, which depend on its layout, lengths, windows and modes
+ * and on no address (0: it runs as rmx_attn_bwd does, or those are refused); the workspace (nullable, 16-byte aligned) is scratch of this call,
  * its contents on entry do not matter, and one smaller than that is not used. No counterpart
  * in the reference.
  */

@@ -175,8 +175,9 @@ int32_t rmx_attn_bwd_delta(const rmx_attn_layout* layout, const void* out, int32
                     "rmx_attn_bwd_delta launch");
 }
 
-static int check_attn_bwd(const rmx_attn_layout* layout, const rmx_bwd_problem* problems,
-                          int32_t nproblems) {
+// The part of the backward's checks that reads no address: what its workspace depends on.
+static int check_bwd_shapes(const rmx_attn_layout* layout, const rmx_bwd_problem* problems,
+                            int32_t nproblems) {
   int rc = check_layout(layout);
   if (rc) return rc;
   if (nproblems < 0 || (nproblems > 0 && !problems))
@@ -185,6 +186,16 @@ static int check_attn_bwd(const rmx_attn_layout* layout, const rmx_bwd_problem* 
     const rmx_bwd_problem& p = problems[i];
     if (p.sq < 0 || p.sk < 0) return fail(RMX_EINVAL, "problem %d: negative length", i);
     if ((rc = check_window(layout, p.has_window, p.window_right, i))) return rc;
+  }
+  return RMX_OK;
+}
+
+static int check_attn_bwd(const rmx_attn_layout* layout, const rmx_bwd_problem* problems,
+                          int32_t nproblems) {
+  int rc = check_bwd_shapes(layout, problems, nproblems);
+  if (rc) return rc;
+  for (int i = 0; i < nproblems; ++i) {
+    const rmx_bwd_problem& p = problems[i];
     if (p.sq == 0 || p.sk == 0) continue;
     if ((rc = check_bf16(p.q, "q"))) return rc;
     if ((rc = check_bf16(p.k, "k"))) return rc;
@@ -222,7 +233,7 @@ static int check_attn_bwd(const rmx_attn_layout* layout, const rmx_bwd_problem* 
 
 size_t rmx_attn_bwd_workspace(const rmx_attn_layout* layout, const rmx_bwd_problem* problems,
                               int32_t nproblems) {
-  if (check_attn_bwd(layout, problems, nproblems)) return 0;
+  if (check_bwd_shapes(layout, problems, nproblems)) return 0;
   size_t bytes = 0;
   for (int i = 0; i < nproblems; i += RMX_MAX_BATCHED) {
     const int n = std::min(nproblems - i, RMX_MAX_BATCHED);

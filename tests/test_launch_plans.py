@@ -128,6 +128,21 @@ def test_block_plans_take_scale_and_window_by_value(monkeypatch):
     ops._plans.clear()
 
 
+def test_plans_keep_the_workspace_of_their_shapes():
+    """The first call of a signature may be refused for an address (here tensors two bytes past
+    alignment); the plan that stays is the one an aligned first call leaves."""
+    def step_bytes(off):
+        mk = lambda h: torch.zeros(512 * h * 64 + 8, dtype=torch.bfloat16)[  # noqa: E731
+            off:off + 512 * h * 64].view(1, 512, h, 64)
+        stat = torch.zeros(1, 8, 512)
+        bases = dict(q=mk(8), k=mk(2), v=mk(2), dout=mk(8), lse=stat, delta=stat, nlse=stat,
+                     dq=mk(8), dk=mk(2), dv=mk(2))
+        job = ops.BwdJob(dq_mode=abi.GRAD_WRITE_BF16, dkv_mode=abi.GRAD_WRITE_BF16, **bases)
+        return ops.LaunchPlan([([job], 0.125, abi.MASK_CAUSAL)], bases).steps[0][3]
+
+    assert step_bytes(1) == step_bytes(0) > 0
+
+
 def test_plans_are_bounded():
     ops._plans.clear()
     for i in range(ops.PLANS_MAX + 9):
