@@ -43,6 +43,47 @@ def _recorded(monkeypatch, fn):
     return list(calls)
 
 
+def _bound(monkeypatch, fn):
+    """The calls of ``fn`` as (kind, layout bytes, problem table, bases): ``bases`` are the tensors
+    the call's plan was bound to, which stay alive with the result, so that no later call's
+    tensors can take their addresses."""
+    bound = []
+    bind = ops.LaunchPlan.bind
+
+    def recording(self, bases):
+        bound.extend([{k: t for k, t in bases.items() if t is not None}] * len(self.steps))
+        return bind(self, bases)
+
+    with monkeypatch.context() as m:
+        m.setattr(ops.LaunchPlan, "bind", recording)
+        calls = _recorded(m, fn)
+    assert len(bound) == len(calls)
+    return [(kind, lay, np.frombuffer(rows, dtype=ops._table_dtype(
+        abi.FwdProblem if kind == "fwd" else abi.BwdProblem)), bases)
+        for (kind, lay, rows, _), bases in zip(calls, bound)]
+
+
+def _check_moved(built, kept, first, layouts_equal=True):
+    """Call by call, the kept plan's tables equal the built one's, every pointer at the same
+    offset of its own call's base tensor and inside it; ``first``: the calls the plans were built
+    by, whose addresses must not appear."""
+    assert len(built) == len(kept) == len(first)
+    for (ka, la, ta, ba), (kc, lc, tc, bc), (_, _, _, bf) in zip(built, kept, first):
+        assert ka == kc and (not layouts_equal or la == lc) and len(ta) == len(tc)
+        for f in ta.dtype.names:
+            if ta.dtype[f] == np.int32:
+                assert (ta[f] == tc[f]).all(), f
+            elif f not in ba:
+                assert not ta[f].any() and not tc[f].any(), f
+            else:
+                t = bc[f]
+                span = (1 + sum((n - 1) * st for n, st in zip(t.shape, t.stride()))) * t.element_size()
+                at = tc[f].astype(np.int64) - t.data_ptr()
+                assert (at == ta[f].astype(np.int64) - ba[f].data_ptr()).all(), f
+                assert ((at >= 0) & (at < span)).all(), f
+                assert t.data_ptr() != bf[f].data_ptr(), f"{f}: the check needs another address"
+
+
 @pytest.mark.parametrize("layout,causal,docs,window", [
     ("zigzag", True, False, None), ("contiguous", True, False, None),
     ("contiguous", False, True, None), ("distflash", True, True, None),
@@ -63,6 +104,7 @@ def test_ring_plans_follow_their_base_tensors(monkeypatch, layout, causal, docs,
 
     def passes(t):
         q, k, v, do, doc = t
+        zigzag._ROWS_CACHE.clear()  # (the global indices are kept and would be the same tensor)
         out, lse, o32 = zigzag.ring_forward(q, k, v, 0.125, doc, layout=layout, causal=causal,
                                             window=window)
         zigzag.ring_backward(do, q, k, v, o32, lse, 0.125, doc, layout=layout, causal=causal,
@@ -70,21 +112,99 @@ def test_ring_plans_follow_their_base_tensors(monkeypatch, layout, causal, docs,
 
     first, second = inputs(1), inputs(2)
     ops._plans.clear()
-    built = _recorded(monkeypatch, lambda: passes(second))
+    built = _bound(monkeypatch, lambda: passes(second))
     ops._plans.clear()
-    passes(first)
+    before = _bound(monkeypatch, lambda: passes(first))
     n_plans = len(ops._plans)
-    kept = _recorded(monkeypatch, lambda: passes(second))
+    kept = _bound(monkeypatch, lambda: passes(second))
     assert len(ops._plans) == n_plans, "the second pass built plans of its own"
-    assert [c[:2] + c[3:] for c in built] == [c[:2] + c[3:] for c in kept]
-    for a, c in zip(built, kept):
-        st = abi.FwdProblem if a[0] == "fwd" else abi.BwdProblem
-        ta, tc = (np.frombuffer(x[2], dtype=ops._table_dtype(st)) for x in (a, c))
-        for f in ta.dtype.names:
-            if f in ("q", "k", "v", "dout") or ta.dtype[f] == np.int32:
+    _check_moved(built, kept, before)
+    for (_, _, ta, _), (_, _, tc, _) in zip(built, kept):
+        for f in ("q", "k", "v", "dout"):
+            if f in ta.dtype.names:
                 assert (ta[f] == tc[f]).all(), f
-            else:  # allocated per call: null together
-                assert ((ta[f] == 0) == (tc[f] == 0)).all(), f
+    ops._plans.clear()
+
+
+def test_ring_plans_of_some_ranks(monkeypatch):
+    """``only_ranks`` is part of a plan's key: two subsets keep two plans, each its own blocks."""
+    mk = lambda seed: torch.randn(4, 1, 2, 16, 64, generator=torch.Generator().manual_seed(  # noqa: E731
+        seed)).to(torch.bfloat16)
+    first, second = mk(1), mk(2)
+
+    def passes(q, ranks):
+        out, lse, o32 = zigzag.ring_forward(q, q, q, 0.125, only_ranks=ranks)
+        zigzag.ring_backward(out, q, q, q, o32, lse, 0.125, only_ranks=ranks)
+
+    built = {}
+    for ranks in ({0}, {1, 3}):
+        ops._plans.clear()
+        built[frozenset(ranks)] = _bound(monkeypatch, lambda: passes(second, ranks))
+    ops._plans.clear()
+    before = {frozenset(r): _bound(monkeypatch, lambda: passes(first, r)) for r in ({0}, {1, 3})}
+    n_plans = len(ops._plans)
+    for ranks, ref in built.items():
+        _check_moved(ref, _bound(monkeypatch, lambda: passes(second, set(ranks))), before[ranks])
+    assert len(ops._plans) == n_plans
+    ops._plans.clear()
+
+
+@pytest.mark.parametrize("keep_f32", [False, True])
+def test_block_plans_follow_their_tensors_and_the_seed(monkeypatch, keep_f32):
+    """A block's forward and backward plans: pointers move with their tensors, and the dropout
+    seed, which is no part of the signature, with the call."""
+    from ringmaster_amd.ring.kernels import block_backward, block_forward
+
+    def inputs(seed):
+        g = torch.Generator().manual_seed(seed)
+        mk = lambda h: torch.randn(2, 24, h, 64, generator=g).to(torch.bfloat16)  # noqa: E731
+        return mk(4), mk(2), mk(2), mk(4)
+
+    def passes(t, seed):
+        q, k, v, do = t
+        out, lse, *o32 = block_forward(q, k, v, 0.125, True, keep_f32=keep_f32, dropout=(0.25, seed))
+        block_backward(do, q, k, v, out, lse, 0.125, True, out_f32=o32[0] if o32 else None,
+                       dropout=(0.25, seed))
+
+    first, second = inputs(1), inputs(2)
+    ops._plans.clear()
+    built = _bound(monkeypatch, lambda: passes(second, (7 << 32) + 5))
+    ops._plans.clear()
+    before = _bound(monkeypatch, lambda: passes(first, 3))
+    n_plans = len(ops._plans)
+    kept = _bound(monkeypatch, lambda: passes(second, (7 << 32) + 5))
+    assert len(ops._plans) == n_plans
+    _check_moved(built, kept, before)
+    seeds = lambda calls: {(lay.drop_seed_lo, lay.drop_seed_hi) for lay in (  # noqa: E731
+        abi.AttnLayout.from_buffer_copy(c[1]) for c in calls)}
+    assert seeds(kept) == {(5, 7)} and seeds(before) == {(3, 0)}
+    ops._plans.clear()
+
+
+@pytest.mark.parametrize("f32", [False, True])
+def test_delta_plans_hold_no_address(monkeypatch, f32):
+    """The delta pass keeps a layout only; its addresses are the call's."""
+    seen = []
+
+    class Lib:
+        def rmx_attn_bwd_delta(self, lay, out, is_f32, dout, delta, lse, nlse, sq, stream):
+            seen.append((bytes(lay._obj), out, is_f32, dout, delta, lse, nlse, sq))
+            return 0
+
+    monkeypatch.setattr(abi, "lib", Lib)
+    monkeypatch.setattr(abi, "stream_of", lambda t: None)
+    ops._plans.clear()
+    held = []
+    for _ in range(2):
+        dout = torch.zeros(2, 24, 4, 64, dtype=torch.bfloat16)
+        out = torch.zeros(2, 24, 4, 64, dtype=torch.float32 if f32 else torch.bfloat16)
+        delta, lse, nlse = (torch.zeros(2, 4, 24) for _ in range(3))
+        held.append((out, dout, delta, lse, nlse))
+        ops.attn_bwd_delta(out, dout, delta, 2, lse=lse, nlse=nlse)
+        o, g, d, l, n = (t.data_ptr() for t in held[-1])
+        assert seen[-1][1:] == (o, int(f32), g, d, l, n, 24)
+    assert len(ops._plans) == 1 and seen[0][0] == seen[1][0]
+    ops._plans.clear()
 
 
 def test_ring_plans_take_the_scale_by_value(monkeypatch):
