@@ -319,6 +319,8 @@ def ring_backward(dout, q, k, v, out, lse, scale: float, doc: torch.Tensor | Non
         out = out.contiguous()
     delta = torch.empty((c.P, c.b, c.hq, c.L), dtype=torch.float32, device=dev)
     nlse = torch.empty_like(delta)
+    if lse.shape != delta.shape:
+        raise ValueError(f"lse must be {tuple(delta.shape)} (got {tuple(lse.shape)})")
     if not lse.is_contiguous():
         lse = lse.contiguous()
     flat = (c.P * c.b, c.L, c.hq, c.d)

@@ -134,7 +134,8 @@ def test_packed_ring_split_equals_whole(monkeypatch, d, docs, layout, causal):
     def grads(split):
         ops._plans.clear()
         one.split = split
-        r = [g.clone() for g in zigzag.ring_backward(do, q, k, v, o32, lse, d ** -0.5, doc, **kw)]
+        for _ in range(2):  # the second pass runs from the plans that the first one left
+            r = [g.clone() for g in zigzag.ring_backward(do, q, k, v, o32, lse, d ** -0.5, doc, **kw)]
         ops._plans.clear()
         return r
 

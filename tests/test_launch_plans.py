@@ -126,6 +126,27 @@ def test_ring_plans_follow_their_base_tensors(monkeypatch, layout, causal, docs,
     ops._plans.clear()
 
 
+def test_kept_ring_plans_refuse_what_building_refused(monkeypatch):
+    """The global lse is no part of the backward plan's key: one of another layout is refused
+    with the plan in place as without it."""
+    q = torch.randn(2, 1, 2, 16, 64).to(torch.bfloat16)
+    do = torch.randn(2, 1, 16, 2, 64).to(torch.bfloat16)
+    out, lse = torch.zeros(2, 1, 16, 2, 64), torch.zeros(2, 1, 2, 16)
+
+    def passes(stat):
+        return _recorded(monkeypatch, lambda: zigzag.ring_backward(do, q, q, q, out, stat, 0.125))
+
+    swapped = lse.transpose(2, 3).contiguous()
+    ops._plans.clear()
+    with pytest.raises(ValueError):
+        passes(swapped)
+    ops._plans.clear()
+    assert passes(lse)
+    with pytest.raises(ValueError):
+        passes(swapped)
+    ops._plans.clear()
+
+
 def test_ring_plans_of_some_ranks(monkeypatch):
     """``only_ranks`` is part of a plan's key: two subsets keep two plans, each its own blocks."""
     mk = lambda seed: torch.randn(4, 1, 2, 16, 64, generator=torch.Generator().manual_seed(  # noqa: E731
