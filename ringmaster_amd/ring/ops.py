@@ -15,7 +15,6 @@ import ctypes
 import dataclasses
 import threading
 
-import numpy as np
 import torch
 
 from ringmaster_amd import abi
@@ -320,8 +319,8 @@ def cast_half(tensors, dtype):
 # than a small ring step's kernels. A plan keeps what those jobs come to for one signature of
 # shapes, strides, types and options: the layouts, and the problem tables with every pointer as
 # an offset from its base tensor. A later call of the same signature adds its own base
-# addresses to a copy of the table. Plans hold no addresses and no tensors, are immutable and
-# at most PLANS_MAX of them are kept.
+# addresses to a copy of the table. Plans hold no address and no tensor of a call, are immutable
+# and at most PLANS_MAX of them are kept.
 PLANS_MAX = 256
 _plans: collections.OrderedDict = collections.OrderedDict()
 _plans_lock = threading.Lock()
@@ -330,14 +329,6 @@ _plans_lock = threading.Lock()
 def signature(*tensors):
     """What a plan depends on of its base tensors."""
     return tuple(None if t is None else (t.shape, t.stride(), t.dtype, t.device) for t in tensors)
-
-
-def _table_dtype(struct):
-    kinds = {ctypes.c_void_p: "u8", ctypes.c_int32: "i4"}
-    return np.dtype({"names": [n for n, _ in struct._fields_],
-                     "formats": [kinds[t] for _, t in struct._fields_],
-                     "offsets": [getattr(struct, n).offset for n, _ in struct._fields_],
-                     "itemsize": ctypes.sizeof(struct)})
 
 
 class _NoSpan:
@@ -374,26 +365,29 @@ class LaunchPlan:
             self.steps.append((lay, lo, len(jobs), nbytes))
             parts.append(bytes(arr))
             lo += len(jobs)
-        self.table = (np.frombuffer(bytearray(b"".join(parts)), dtype=_table_dtype(self.struct))
-                      if parts else None)
-        self.fields = []
+        # [problem, 8-byte word of the struct], on the host
+        self.words = ctypes.sizeof(self.struct) // 8
+        self.table = (torch.frombuffer(bytearray(b"".join(parts)), dtype=torch.int64)
+                      .view(lo, self.words) if parts else None)
+        self.fields = []  # (word, name)
         for name, base in bases.items():
             if self.table is None or base is None:
                 continue
-            col = self.table[name]
+            word = getattr(self.struct, name).offset // 8
+            col = self.table[:, word]
             if not col.any():
                 continue
             if not col.all():
                 raise AssertionError(f"{name} is set in some problems only")
-            col -= np.uint64(base.data_ptr())
-            self.fields.append(name)
+            col -= base.data_ptr()
+            self.fields.append((word, name))
 
     def bind(self, bases):
         """The problem tables at the addresses of ``bases``."""
-        t = self.table.copy()
-        for name in self.fields:
-            t[name] += np.uint64(bases[name].data_ptr())
-        return t
+        at = [0] * self.words
+        for word, name in self.fields:
+            at[word] = bases[name].data_ptr()
+        return self.table + torch.tensor(at, dtype=torch.int64, device="cpu")
 
     def _layout(self, lay, seed):
         if not self.drop:
@@ -403,7 +397,14 @@ class LaunchPlan:
         return lay
 
     def problems(self, table, lo):
-        return ctypes.byref(self.struct.from_buffer(table.view(np.uint8), lo * table.itemsize))
+        """The rows of a bound table from ``lo`` on (which the caller keeps alive)."""
+        return ctypes.byref(self.struct.from_address(table.data_ptr() + 8 * self.words * lo))
+
+    def _set(self, table, field, value):
+        """A copy of a bound table with an int32 field of every problem set."""
+        table = table.clone()
+        table.view(torch.int32)[:, getattr(self.struct, field).offset // 4] = value
+        return table
 
     def run_fwd(self, bases, seed, like, span):
         """Launch the forward steps; ``span()`` brackets each (timing)."""
@@ -425,8 +426,7 @@ class LaunchPlan:
             for lay, lo, n, nbytes in self.steps:
                 _launch_bwd(lib, self._layout(lay, seed), self.problems(t, lo), n, nbytes, like)
             return
-        tk, tq = t.copy(), t
-        tk["dq_mode"] = tq["dkv_mode"] = abi.GRAD_NONE
+        tk, tq = (self._set(t, f, abi.GRAD_NONE) for f in ("dq_mode", "dkv_mode"))
         for lay, lo, n, nbytes in self.steps:
             lay = self._layout(lay, seed)
             with span("attn_bwd_dkdv"):

@@ -15,6 +15,14 @@ def _host(monkeypatch):
     monkeypatch.setattr(abi, "require_device", lambda *t: None)
 
 
+def _table_dtype(struct):
+    kinds = {ctypes.c_void_p: "u8", ctypes.c_int32: "i4"}
+    return np.dtype({"names": [n for n, _ in struct._fields_],
+                     "formats": [kinds[t] for _, t in struct._fields_],
+                     "offsets": [getattr(struct, n).offset for n, _ in struct._fields_],
+                     "itemsize": ctypes.sizeof(struct)})
+
+
 def _recorded(monkeypatch, fn):
     """The (layout bytes, problem bytes) of every call ``fn`` makes, with no library."""
     calls = []
@@ -58,7 +66,7 @@ def _bound(monkeypatch, fn):
         m.setattr(ops.LaunchPlan, "bind", recording)
         calls = _recorded(m, fn)
     assert len(bound) == len(calls)
-    return [(kind, lay, np.frombuffer(rows, dtype=ops._table_dtype(
+    return [(kind, lay, np.frombuffer(rows, dtype=_table_dtype(
         abi.FwdProblem if kind == "fwd" else abi.BwdProblem)), bases)
         for (kind, lay, rows, _), bases in zip(calls, bound)]
 
@@ -282,6 +290,41 @@ def test_plans_keep_the_workspace_of_their_shapes():
         return ops.LaunchPlan([([job], 0.125, abi.MASK_CAUSAL)], bases).steps[0][3]
 
     assert step_bytes(1) == step_bytes(0) > 0
+
+
+@pytest.mark.parametrize("timed", [False, True])
+def test_one_call_or_one_per_gradient(monkeypatch, timed):
+    """Without a timer a step's dK/dV and dQ are one call, with one two calls of a gradient each,
+    which differ from it in the other gradient's mode alone."""
+    q = torch.randn(2, 1, 2, 16, 64).to(torch.bfloat16)
+    do, out = torch.randn(2, 1, 16, 2, 64).to(torch.bfloat16), torch.zeros(2, 1, 16, 2, 64)
+    lse = torch.zeros(2, 1, 2, 16)
+    spans = []
+
+    class Span:
+        def __call__(self, name):
+            spans.append(name)
+            return self
+
+        def __enter__(self):
+            pass
+
+        def __exit__(self, *exc):
+            return False
+
+    ops._plans.clear()
+    calls = _recorded(monkeypatch, lambda: zigzag.ring_backward(
+        do, q, q, q, out, lse, 0.125, timer=Span() if timed else None))
+    tables = [np.frombuffer(rows, dtype=_table_dtype(abi.BwdProblem)) for _, _, rows, _ in calls]
+    modes = [(set(t["dq_mode"].tolist()), set(t["dkv_mode"].tolist())) for t in tables]
+    w, a, n = {abi.GRAD_WRITE_F32}, {abi.GRAD_ACC_F32}, {abi.GRAD_NONE}
+    if timed:
+        assert modes == [(n, w), (w, n), (n, a), (a, n)]
+        assert spans == ["attn_bwd_delta"] + ["attn_bwd_dkdv", "attn_bwd_dq"] * 2
+        assert all(t["dk_acc"].all() and t["dq_acc"].all() for t in tables)
+    else:
+        assert modes == [(w, w), (a, a)]
+    ops._plans.clear()
 
 
 def test_plans_are_bounded():
