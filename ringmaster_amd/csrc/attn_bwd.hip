@@ -128,9 +128,9 @@ hipError_t launch_attn_bwd_delta(const rmx_attn_layout& L, const void* out, int 
 // workgroup cost what the kernels measure on a lone CU,
 // workgroups run in rounds over the CUs, and a split launch adds the fold kernel and the
 // partial gradients' traffic. Launches of many rounds stay whole. Whole -> split, us a launch:
-// 4096^2 causal 32/8 heads of 128 403 -> 314 (2), 2048^2 189 -> 101 (3), 512^2 58 -> 34 (4);
-// 4096^2 causal 16/4 heads of 256 821 -> 343 (4), of 64 253 -> 102 (4); the same 4096^2 with
-// 32 KV heads fills the chip and would go from 321 to 419 in two.
+// 4096^2 causal 32/8 heads of 128 365 -> 266 (2), 2048^2 182 -> 91 (3), 512^2 56 -> 33 (4);
+// 4096^2 causal 16/4 heads of 256 803 -> 296 (4), of 64 236 -> 92 (4); the same 4096^2 with
+// 32 KV heads of 128 fills the chip and stays whole (267; an earlier build 321, in two 419).
 // A packed ring's backward (every kernel of it), whole -> split: 4 ranks x 1024 tokens, 8/2 heads of
 // 128, documents of 64 tokens 269 -> 214, of 2048 504 -> 321; 8 x 766, 4/2 heads of 64, of 364 217 -> 209;
 // over 22 rings of the range at most 1.02 of the whole one's time.
@@ -194,7 +194,7 @@ struct FoldParams {
   rmx_attn_layout L;
   rmx_bwd_problem P[RMX_MAX_BATCHED];
   SplitParts parts;
-  int n, nsplit;
+  int nsplit;
 };
 
 // Sum of the splits' partial dV (blockIdx.y 0) and dK (1) rows, stored in their problem's mode.
@@ -206,20 +206,22 @@ __global__ __launch_bounds__(256) void dkdv_fold_kernel(const FoldParams prm) {
   const rmx_attn_layout& L = prm.L;
   const int g = blockIdx.y, D = L.head_dim, per = L.batch * L.hkv;
   const int col = 4 * (threadIdx.x % CPR);
-  const int64_t row = (int64_t)blockIdx.x * RPB + threadIdx.x / CPR;
-  int64_t local = row;  // (key, batch, kv head) of problem p
-  int p = 0, block = 0;
-  for (; p < prm.n && local >= (int64_t)per * prm.P[p].sk; ++p) {
-    local -= (int64_t)per * prm.P[p].sk;
+  // problem p of this workgroup, its first row and key block (a split launch has under 1024 key
+  // blocks: rows fit 32 bits); one problem per workgroup keeps p and its fields in scalars
+  int p = 0, wg = blockIdx.x, row0 = 0, block = 0;
+  for (int n; wg >= (n = (per * prm.P[p].sk + RPB - 1) / RPB); ++p) {
+    wg -= n;
+    row0 += per * prm.P[p].sk;
     block += per * split_key_blocks(prm.P[p].sk);
   }
-  if (col >= D || p == prm.n) return;
   const rmx_bwd_problem& P = prm.P[p];
-  const int key = (int)(local / per), bh = (int)(local - (int64_t)key * per);
+  const int local = wg * RPB + threadIdx.x / CPR;  // (batch, kv head, key)
+  if (col >= D || local >= per * P.sk) return;
+  const int bh = local / P.sk, key = local - bh * P.sk;
   const int bb = bh / L.hkv, h = bh % L.hkv;
   // (an empty block is its first workgroup's, which has stored it if the mode writes)
   if (L.mask == RMX_MASK_DOC && prm.parts.empty[block + bh * split_key_blocks(P.sk) + key / 128]) return;
-  const float* src = prm.parts.base + g * prm.parts.grad + row * D + col;
+  const float* src = prm.parts.base + g * prm.parts.grad + (int64_t)(row0 + local) * D + col;
   f32x4 v = *reinterpret_cast<const f32x4*>(src);
 #pragma unroll 4
   for (int s = 1; s < prm.nsplit; ++s)
@@ -252,9 +254,12 @@ __global__ __launch_bounds__(256) void dkdv_fold_kernel(const FoldParams prm) {
 }
 
 template <int HD>
-static void launch_fold_t(const FoldParams& prm, int64_t rows, bool f16, hipStream_t stream) {
+static void launch_fold_t(const FoldParams& prm, int n, bool f16, hipStream_t stream) {
   constexpr int RPB = 256 / (HD / 4);
-  const dim3 grid((unsigned)((rows + RPB - 1) / RPB), 2);
+  int wgs = 0;
+  for (int i = 0; i < n; ++i)
+    wgs += (prm.L.batch * prm.L.hkv * prm.P[i].sk + RPB - 1) / RPB;
+  const dim3 grid(wgs, 2);
   if (f16)
     hipLaunchKernelGGL((dkdv_fold_kernel<HD, RMX_DTYPE_F16>), grid, dim3(256), 0, stream, prm);
   else
@@ -267,16 +272,14 @@ hipError_t launch_dkdv_fold(const rmx_attn_layout& L, const rmx_bwd_problem* pro
   prm.L = L;
   for (int i = 0; i < n; ++i) prm.P[i] = probs[i];
   prm.parts = split.at(ws);
-  prm.n = n;
   prm.nsplit = split.n;
-  const int64_t rows = split.grad / L.head_dim;
   const bool f16 = L.dtype == RMX_DTYPE_F16;
   if (L.head_dim > 128)
-    launch_fold_t<256>(prm, rows, f16, stream);
+    launch_fold_t<256>(prm, n, f16, stream);
   else if (L.head_dim > 64)
-    launch_fold_t<128>(prm, rows, f16, stream);
+    launch_fold_t<128>(prm, n, f16, stream);
   else
-    launch_fold_t<64>(prm, rows, f16, stream);
+    launch_fold_t<64>(prm, n, f16, stream);
   return hipGetLastError();
 }
 

@@ -43,28 +43,12 @@ struct BwdParams {
 };
 
 // ---------------------------------------------------------------- shared helpers
-// Write a 4-float run of a gradient row according to the output mode.
-template <int DT>
-__device__ __forceinline__ void grad_store4(int mode, float* acc, uint16_t* bf, f32x4 v) {
-  if (mode == RMX_GRAD_WRITE_F32) {
-    *reinterpret_cast<f32x4*>(acc) = v;
-  } else if (mode == RMX_GRAD_ACC_F32) {
-    *reinterpret_cast<f32x4*>(acc) = *reinterpret_cast<const f32x4*>(acc) + v;
-  } else {
-    if (mode == RMX_GRAD_ACC_FINAL) v += *reinterpret_cast<const f32x4*>(acc);
-    u32x2 w;
-    w[0] = cvt_pk<DT>(v[0], v[1]);
-    w[1] = cvt_pk<DT>(v[2], v[3]);
-    *reinterpret_cast<u32x2*>(bf) = w;
-  }
-}
-
 // first of n items of share i of s
 __device__ __forceinline__ int split_lo(int n, int i, int s) { return (int)((int64_t)n * i / s); }
 
 // ---------------------------------------------------------------- dK/dV splits
-// Partial gradients are rows [problem][key][batch, kv head] of head_dim: a problem's rows follow
-// those of the problems before it, and the strides are the same for all of them.
+// Partial gradients are rows [problem][batch, kv head][key] of head_dim, a problem's rows behind
+// those of the problems before it.
 // rows of the workspace before problem p
 __device__ __forceinline__ int64_t split_row0(const BwdParams& prm, int p) {
   int64_t keys = 0;
@@ -83,7 +67,7 @@ __device__ __forceinline__ GradOut grad_out(const BwdParams& prm, const rmx_bwd_
   if (share < 0) return {P.dv_acc, P.dk_acc, L.ka_sb, L.ka_ss, L.ka_sh};
   const int64_t D = L.head_dim, grad = prm.parts.grad;
   float* const dv = prm.parts.base + 2 * grad * share + split_row0(prm, p) * D;
-  return {dv, dv + grad, L.hkv * D, (int64_t)L.batch * L.hkv * D, D};
+  return {dv, dv + grad, (int64_t)L.hkv * P.sk * D, D, P.sk * D};
 }
 
 // index of key block kb of (problem p, group = batch * hkv + kv head)
@@ -1234,8 +1218,8 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_kernel(const BwdParams p
   // 64-column groups swapped in every second group of four rows so that the two lane halves
   // write different banks) and come back as 16-byte chunks of whole rows, one mode test per
   // chunk; the accumulating modes read all of a lane's prior chunks before its first store
-  // (one wait, not one memory round trip per row). A launch of one tile: 28.4 -> 12.8 us at
-  // head dim 128, 19.4 -> 8.7 at 64.
+  // (one wait, not one memory round trip per row). A launch of one tile: 28.4 -> 11.7 us at
+  // head dim 128, 19.4 -> 8.1 at 64.
   // Caller pointers below vector alignment take the element-wise form, straight from the
   // accumulators; the dropout kernels a compact loop over the staged rows. The choice is the
   // register allocator's: with the compact loop the FULL and causal main loops move 47 values
@@ -1900,11 +1884,19 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_d256_kernel(const BwdPar
 
   // ---- epilogue: lane (hl, l32) holds column d = 32 db + l32 of keys kw0 + c_row(hl, r).
   // Each gradient is staged through LDS as [key][d] fp32 rows (the tiles are dead) and
-  // stored as 4-column runs of whole rows: one mode test per run, not per element.
-  const int mode = share >= 0 ? RMX_GRAD_WRITE_F32 : P.dkv_mode;
-  const GradOut O = grad_out(prm, P, wc.p, share);
+  // stored as 4-column runs of whole rows: one mode test per run, not per element. The rows of
+  // the writing modes go in a short loop: unrolled, with an address and a test per row, the
+  // epilogue was 60 KB of code, and a launch of one tile took 29.8 us instead of 16.0.
+  int pe = wc.p;  // (as in the kernel above)
+  asm volatile("" : "+s"(pe));
+  const rmx_bwd_problem& E = prm.P[pe];
+  const int mode = share >= 0 ? RMX_GRAD_WRITE_F32 : E.dkv_mode;
+  const GradOut O = grad_out(prm, E, pe, share);
   float* const stg = reinterpret_cast<float*>(smem);
-  const int col = 4 * (tid & 63), rw = tid >> 6;  // columns col .. col + 3 of rows rw + 4 i
+  const int col = 4 * (tid & 63);  // columns col .. col + 3 of rows wave + 4 i
+  const bool rd = mode == RMX_GRAD_ACC_F32 || mode == RMX_GRAD_ACC_FINAL;
+  const bool w32 = mode == RMX_GRAD_WRITE_F32 || mode == RMX_GRAD_ACC_F32;
+  const int rows = sk - k0 - wave;  // (rows wave + r, r < rows)
   auto store = [&](const f32x16* acc, float sc, float* gacc, uint16_t* gbf) {
     __syncthreads();  // every wave is past its last tile reads (or the previous gradient)
 #pragma unroll
@@ -1914,60 +1906,65 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv_d256_kernel(const BwdPar
         stg[(32 * wave + c_row(hl, r)) * HD + 32 * db + l32] = acc[db][r] * sc;
     __syncthreads();
     if (col >= D) return;  // columns past the head dim are not stored
-    const bool vf = ((uintptr_t)gacc & 15) == 0, vb = share >= 0 || ((uintptr_t)gbf & 7) == 0;
-    auto gptr = [&](int kk) {
-      return gacc ? gacc + bb * O.sb + (int64_t)kk * O.ss + kvh * O.sh + col : nullptr;
+    const bool vec = (!(rd || w32) || ((uintptr_t)gacc & 15) == 0) &&
+                     (w32 || ((uintptr_t)gbf & 7) == 0);
+    const float* src = stg + wave * HD + col;
+    float* ga = gacc + bb * O.sb + kvh * O.sh + (int64_t)(k0 + wave) * O.ss + col;
+    uint16_t* gb = gbf + bb * L.dk_sb + kvh * L.dk_sh + (int64_t)(k0 + wave) * L.dk_ss + col;
+    const int64_t sa = 4 * O.ss, sb = 4 * L.dk_ss;
+    auto put = [&](const f32x4& v) __attribute__((always_inline)) {
+      if (w32) {
+        *reinterpret_cast<f32x4*>(ga) = v;
+      } else {
+        u32x2 w;
+        w[0] = cvt_pk<DT>(v[0], v[1]);
+        w[1] = cvt_pk<DT>(v[2], v[3]);
+        *reinterpret_cast<u32x2*>(gb) = w;
+      }
+      ga += sa;
+      gb += sb;
     };
-    auto bptr = [&](int kk) {
-      return gbf ? gbf + bb * L.dk_sb + (int64_t)kk * L.dk_ss + kvh * L.dk_sh + col : nullptr;
-    };
-    if (vf && vb) {
+    if (vec && !rd) {
+#pragma unroll 4
+      for (int r = 0; r < BKV; r += 4, src += 4 * HD) {
+        if (r >= rows) break;
+        put(*reinterpret_cast<const f32x4*>(src));
+      }
+      return;
+    }
+    if (vec) {
       // the accumulating modes read the prior values of 16 of the thread's rows before
       // their first store (one wait per 16 rows, not one memory round trip per row)
-      const bool rd = mode == RMX_GRAD_ACC_F32 || mode == RMX_GRAD_ACC_FINAL;
-      const int wmode = mode == RMX_GRAD_ACC_F32 ? RMX_GRAD_WRITE_F32
-                        : mode == RMX_GRAD_ACC_FINAL ? RMX_GRAD_WRITE_BF16 : mode;
       constexpr int RUN = 16;
-#pragma unroll
-      for (int i0 = 0; i0 < BKV / 4; i0 += RUN) {
+#pragma unroll 1
+      for (int r0 = 0; r0 < BKV && r0 < rows; r0 += 4 * RUN) {
         f32x4 prev[RUN];
 #pragma unroll
-        for (int i = 0; i < RUN; ++i) {
-          const int kk = k0 + rw + 4 * (i0 + i);
-          prev[i] = rd && kk < sk ? *reinterpret_cast<const f32x4*>(gptr(kk)) : f32x4{};
-        }
+        for (int i = 0; i < RUN; ++i)
+          prev[i] = r0 + 4 * i < rows ? *reinterpret_cast<const f32x4*>(ga + i * sa) : f32x4{};
 #pragma unroll
-        for (int i = 0; i < RUN; ++i) {
-          const int row = rw + 4 * (i0 + i), kk = k0 + row;
-          if (kk >= sk) return;
-          f32x4 v = *reinterpret_cast<const f32x4*>(stg + row * HD + col);
-          if (rd) v += prev[i];
-          grad_store4<DT>(wmode, gptr(kk), bptr(kk), v);
+        for (int i = 0; i < RUN; ++i, src += 4 * HD) {
+          if (r0 + 4 * i >= rows) break;
+          f32x4 v = *reinterpret_cast<const f32x4*>(src);
+          v += prev[i];
+          put(v);
         }
       }
       return;
     }
-    for (int row = rw; row < BKV && k0 + row < sk; row += 4) {
-      const int kk = k0 + row;
-      const f32x4 v = *reinterpret_cast<const f32x4*>(stg + row * HD + col);
-      float* ga = gptr(kk);
-      uint16_t* gb = bptr(kk);
-#pragma unroll
+#pragma unroll 1
+    for (int r = 0; r < BKV && r < rows; r += 4, src += 4 * HD, ga += sa, gb += sb)
+#pragma unroll 1
       for (int e = 0; e < 4; ++e) {  // a caller pointer below vector alignment
-        if (mode == RMX_GRAD_WRITE_F32) {
-          ga[e] = v[e];
-        } else if (mode == RMX_GRAD_ACC_F32) {
-          ga[e] += v[e];
-        } else if (mode == RMX_GRAD_ACC_FINAL) {
-          gb[e] = f2e<DT>(ga[e] + v[e]);
-        } else {
-          gb[e] = f2e<DT>(v[e]);
-        }
+        const float x = rd ? ga[e] + src[e] : src[e];
+        if (w32)
+          ga[e] = x;
+        else
+          gb[e] = f2e<DT>(x);
       }
-    }
   };
-  store(dv, 1.f, O.dv, P.dv);
-  store(dk, -L.scale, O.dk, P.dk);
+  store(dv, 1.f, O.dv, E.dv);
+  store(dk, -L.scale, O.dk, E.dk);
 }
 
 // dQ of the n problems in prm.P (in launch order)

@@ -15,7 +15,7 @@ hipError_t launch_attn_bwd_delta(const rmx_attn_layout& L, const void* out, int 
                                  const uint16_t* dout, float* delta, const float* lse, float* nlse,
                                  int sq, hipStream_t stream);
 // A split dK/dV launch's workspace: `base` holds n splits x (dV, dK) of `grad` elements each, a
-// gradient being rows [problem][key][batch, kv head] of head_dim; `empty` one word per key block
+// gradient being rows [problem][batch, kv head][key] of head_dim; `empty` one word per key block
 // ([problem][batch, kv head][block], RMX_MASK_DOC only): 1 where no query attends it.
 struct SplitParts {
   float* base;
