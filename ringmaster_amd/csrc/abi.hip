@@ -301,11 +301,13 @@ int32_t rmx_cast_half(const float* const* src, uint16_t* const* dst, const int64
     return fail(RMX_EINVAL, "unknown element type %d", dtype);
   if (count == 0) return RMX_OK;
   if (!src || !dst || !n) return fail(RMX_EINVAL, "NULL array list");
+  int64_t wgs = 0;  // 2048 elements each
   for (int i = 0; i < count; ++i) {
     if (n[i] < 0 || n[i] % 8)
       return fail(RMX_EINVAL, "array %d: %lld elements (a multiple of 8)", i, (long long)n[i]);
-    if (n[i] / 2048 >= 2147483647LL)
-      return fail(RMX_EUNSUPPORTED, "array %d: more than 2^31 workgroups", i);
+    wgs += n[i] / 2048 + 1;
+    if (wgs >= 2147483647LL)
+      return fail(RMX_EUNSUPPORTED, "arrays up to %d: more than 2^31 workgroups", i);
     if (n[i] && (!src[i] || !dst[i])) return fail(RMX_EINVAL, "array %d is NULL", i);
     if (!aligned(src[i], 16) || !aligned(dst[i], 16))
       return fail(RMX_EINVAL, "array %d must be 16-byte aligned", i);
