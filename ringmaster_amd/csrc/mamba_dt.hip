@@ -74,6 +74,16 @@ __device__ __forceinline__ float add_log1p(float x, float z) {  // x + log1p(z),
   const float t = x + h, b = t - x;  // and that of x + h (Knuth's two-sum)
   return t + (low + ((x - (t - b)) + (h - b)));
 }
+// d softplus / dx = 1 / (1 + z) for x >= 0, z / (1 + z) below: the quotient by the reciprocal and one
+// residual step against the unrounded 1 + z. Its rms error for x in [-4, -2), [0.5, 1) and [2, 4) is
+// 3.50, 2.69 and 1.83e-8; of expf(x) / (expf(x) + 1) 4.78, 3.27 and 2.18e-8; of z times a refined
+// reciprocal of the rounded 1 + z 5.13, 3.76 and 3.74e-8, 0.4 us sooner.
+__device__ __forceinline__ float softplus_grad(float x, float z) {
+#pragma clang fp contract(off)
+  const float d = 1.f + z, dl = z - (d - 1.f), r = __builtin_amdgcn_rcpf(d);
+  const float m = x >= 0.f ? 1.f : z, q = m * r;
+  return fmaf(fmaf(-dl, q, fmaf(-d, q, m)), r, q);
+}
 __device__ __forceinline__ float softplus_t(float x) {
   return x > 20.f ? x : add_log1p(fmaxf(x, 0.f), expf(-fabsf(x)));
 }
@@ -275,11 +285,9 @@ __device__ __forceinline__ void dt_bwd_chunk(const DtArgs& a, const DtPos<HT>& p
     const float ge = Ah * R + d[i];
     float e = x[i], gdt = ge;
     if (a.softplus) {
-      const float z = expf(-fabsf(y)), d = 1.f + z;
+      const float z = expf(-fabsf(y));
       e = y > 20.f ? y : add_log1p(fmaxf(y, 0.f), z);
-      float r = __builtin_amdgcn_rcpf(d);
-      r = fmaf(fmaf(-d, r, 1.f), r, r);
-      gdt = y > 20.f ? ge : ge * (y >= 0.f ? r : z * r);
+      gdt = y > 20.f ? ge : ge * softplus_grad(y, z);
     }
     if (i < p.n) {
       pa += R * e;

@@ -164,3 +164,23 @@ def test_softplus_is_as_exact_as_the_library(lo, hi, bar):
     rms = ((e - ref) / ref).pow(2).mean().sqrt().item()
     print(f"case softplus [{lo}, {hi}): rms {rms:.3e}", flush=True)
     assert rms < bar
+
+
+@pytest.mark.parametrize("lo,hi,bar", [(-8, -4, 5.0e-8), (-2, -1, 4.45e-8), (-0.5, 0, 3.4e-8),
+                                       (0.5, 1, 3.3e-8), (2, 4, 2.2e-8), (4, 10, 1.8e-8)])
+def test_softplus_gradient_is_as_exact_as_the_library(lo, hi, bar):
+    """The step's derivative (dL/de = 1, no other gradient) stays within the rms error of
+    expf(x) / (expf(x) + 1) over the same range: 4.99, 4.45, 3.38, 3.27, 2.18 and 1.75e-8."""
+    from ringmaster_amd import abi
+
+    rows, T, H = 16, 1024, 64
+    dt = (torch.rand((rows, T, H), generator=torch.Generator().manual_seed(5)) * (hi - lo) + lo).cuda()
+    A, bias, g_A, g_b = (torch.zeros(H, device="cuda") for _ in range(4))
+    g_e, g_dt = torch.ones_like(dt), torch.empty_like(dt)
+    abi.check(abi.lib().rmx_mamba2_dt_cumsum_bwd(
+        dt.data_ptr(), 1, bias.data_ptr(), A.data_ptr(), 1, None, g_e.data_ptr(), None, None,
+        g_dt.data_ptr(), g_A.data_ptr(), g_b.data_ptr(), rows, T, H, abi.stream_of(dt)))
+    ref = torch.sigmoid(dt.double())
+    rms = ((g_dt - ref) / ref).pow(2).mean().sqrt().item()
+    print(f"case softplus gradient [{lo}, {hi}): rms {rms:.3e}", flush=True)
+    assert rms < bar
